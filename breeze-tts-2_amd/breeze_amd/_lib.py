@@ -35,6 +35,8 @@ EXPORTS = (
     "bz_gemv_workspace",
     "bz_gemv",
     "bz_gemv_noalloc",
+    "bz_gemm_workspace",
+    "bz_gemm_tiled",
     "bz_rmsnorm",
     "bz_silu_mul",
     "bz_quantize_int4",
@@ -113,6 +115,10 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.bz_gemv.argtypes = [ctypes.POINTER(GemvDesc), vp]
     lib.bz_gemv_noalloc.restype = ctypes.c_int
     lib.bz_gemv_noalloc.argtypes = [ctypes.POINTER(GemvDesc), vp]
+    lib.bz_gemm_workspace.restype = ctypes.c_size_t
+    lib.bz_gemm_workspace.argtypes = [i32, i32, i32, i32, i32]
+    lib.bz_gemm_tiled.restype = ctypes.c_int
+    lib.bz_gemm_tiled.argtypes = [i32, vp, i64, i32, vp, i32, i32, vp, i64, i32, vp, ctypes.c_size_t, i32, vp]
     lib.bz_rmsnorm.restype = ctypes.c_int
     lib.bz_rmsnorm.argtypes = [vp, i64, vp, f32, vp, i64, i32, i32, vp]
     lib.bz_silu_mul.restype = ctypes.c_int

@@ -491,21 +491,46 @@ def dequant(wfmt: int, w: torch.Tensor, n: int, k: int, *, sc0=None, sc1=None, g
 def dequant_matmul(x: torch.Tensor, w: torch.Tensor, wfmt: int, n: int, k: int,
                    chunk_bytes: int = 16 << 20) -> torch.Tensor:
     """x [M, k] @ w_eff^T -> bf16 [M, n] for prefill-sized M, over an unpaired
-    tiled weight (BZ_W_INT4_TILED, group 128, or BZ_W_FP8_TILED).  The weight
-    is decoded by the GPU path's own unpacking (bz_dequant) one run of whole
-    16-row blocks at a time, at most ``chunk_bytes`` of fp32 per run, each
-    run cast to bf16 and multiplied by torch's GEMM into its output columns:
-    the transient memory stays bounded whatever the weight's size (a whole
-    fp32 copy of a 10240 x 2560 weight would be 105 MB)."""
+    tiled weight (BZ_W_INT4_TILED, group 128, or BZ_W_FP8_TILED): one GEMM
+    (bz_gemm_tiled) that decodes the weight in registers, so no decoded copy
+    exists; where it slices K, the slices' fp32 sums are held for the call.
+    An x that autograd follows goes through torch's linear over the decoded
+    weight instead (at most ``chunk_bytes`` of fp32 weight at a time)."""
     if wfmt not in (W_INT4_TILED, W_FP8_TILED):
         raise ValueError(f"dequant_matmul reads the unpaired tiled formats, not format {wfmt}")
     _require_gpu("x", x, x.device)
+    _require_gpu("w", w, x.device)
+    w = w.contiguous()
     _check_weight(w, wfmt, n, k, 128, None, None)
     if x.dim() != 2 or x.shape[1] != k:
         raise ValueError(f"x must be [M, {k}], got {tuple(x.shape)}")
+    if (x.requires_grad and torch.is_grad_enabled()) or torch.autograd.forward_ad._current_level >= 0:
+        return _dequant_linear(x, w, wfmt, n, k, chunk_bytes)
+    x = _rows_aligned(x)
+    if not k <= x.stride(0) <= _GEMM_MAX_LDX:  # rows that overlap (an expanded row) or lie far apart
+        x = x.contiguous()
+    M = x.shape[0]
+    out = torch.empty(M, n, device=x.device, dtype=torch.bfloat16)
+    if M == 0:
+        return out
+    lib = _lib.lib()
+    need = lib.bz_gemm_workspace(wfmt, M, n, k, 0)
+    # from the caching allocator: its memory is reused in stream order
+    sums = torch.empty(need, device=x.device, dtype=torch.uint8) if need else None
+    _lib.check(lib.bz_gemm_tiled(wfmt, x.data_ptr(), x.stride(0), M, w.data_ptr(), n, k, out.data_ptr(), n, DT_BF16,
+                                 _ptr(sums), need, 0, _lib.stream_of(x)), "bz_gemm_tiled")
+    return out
+
+
+_GEMM_MAX_LDX = 1 << 22  # widest row stride bz_gemm_tiled takes (32-bit offsets within a row tile)
+
+
+def _dequant_linear(x: torch.Tensor, w: torch.Tensor, wfmt: int, n: int, k: int, chunk_bytes: int) -> torch.Tensor:
+    """dequant_matmul as torch ops on x, one run of whole 16-row blocks of the
+    decoded weight at a time: what autograd can follow."""
     x = x.to(torch.bfloat16)
     block = tiled_bytes(wfmt, 16, k)
-    wb = w.contiguous().view(torch.uint8).reshape(-1)
+    wb = w.view(torch.uint8).reshape(-1)
     rows = max(16, chunk_bytes // (4 * k) // 16 * 16)
     out = torch.empty(x.shape[0], n, device=x.device, dtype=torch.bfloat16)
     for r0 in range(0, n, rows):

@@ -224,6 +224,21 @@ size_t bz_gemv_workspace(const bz_gemv_desc* d);
  * models/fused/kernels.py:336). */
 int bz_gemv(const bz_gemv_desc* d, void* stream);
 
+/* Prefill GEMM: out[M][N] = x[M][K] @ w_eff^T for prompt-sized M over an
+ * unpaired tiled weight (BZ_W_INT4_TILED, group 128, or BZ_W_FP8_TILED); x
+ * bf16 with 16-byte aligned rows (ldx >= K), out bf16 or fp32 (ldo >= N),
+ * fp32 accumulation.  Replaces torch._weight_int4pack_mm and
+ * torch._scaled_mm (weight-only form) for the rows of a prompt
+ * (models/int4_linear.py:103-108, models/fp8_linear.py:76-82).
+ * bz_gemm_workspace gives the bytes it needs (16-byte aligned; fp32 sums of
+ * its K slices, contents irrelevant before and after; 0 when it runs as one
+ * slice): without them the call is refused.  cfg = 0 takes the built-in
+ * launch shape, else row groups | row blocks per wave << 8 | K slices << 16
+ * (a part left 0 keeps the rule's choice). */
+size_t bz_gemm_workspace(int32_t wfmt, int32_t M, int32_t N, int32_t K, int32_t cfg);
+int bz_gemm_tiled(int32_t wfmt, const void* x, int64_t ldx, int32_t M, const void* w, int32_t N, int32_t K, void* out,
+                  int64_t ldo, int32_t out_dtype, void* workspace, size_t workspace_bytes, int32_t cfg, void* stream);
+
 /* Measurement aid, no counterpart in the reference: reads `bytes` (a
  * multiple of `chunk`, which is a multiple of 16 and at most 256 KiB;
  * 16-byte aligned) from device memory `p` once, one workgroup per
