@@ -8,6 +8,7 @@
 #include <algorithm>
 
 #include "bz_gemv_panel.h"
+#include "bz_gemv_rows.h"
 #include "bz_gemv_tile.h"
 #include "bz_gemv_wide.h"
 
@@ -615,6 +616,35 @@ static int gemv_panel_rows(const bz_gemv_desc* d, hipStream_t st) {
     return BZ_OK;
 }
 
+// Launch shape of the bf16 row kernel (bz_gemv_rows.h) for `rows` <= 4 rows of
+// x, or false where it does not apply (a forced launch shape, K past its
+// spans).  Four weight rows per wave, or two where four give less than one
+// workgroup per CU or a second, mostly empty round (257..383 workgroups).
+// Measured on MI355X at M = 2, four against two rows: N4096 K2048 4.96 / 5.27
+// us, N2048 K2048 4.12 / 3.80, N2560 K4096 (320 workgroups) 6.65 / 6.07,
+// N6144 K2560 (384) 7.95 / 8.12, N1024 K8192 (4 waves per row) 5.39 / 5.40.
+// The kernel was the faster one at every shape and M = 1..4 timed, against
+// the better of the dot2 and matrix-core kernels: N4096 K2048 M = 2 6.94 ->
+// 4.96, N2048 K2048 5.36 -> 3.80, N12288 K2048 SiLU-gate 13.1 -> 10.8, N1024
+// K8192 8.36 -> 5.39, N8192 K2560 M = 3 11.5 -> 10.5.
+static bool rows_plan(const bz_gemv_desc* d, const DescInfo& di, int rows, RowsLaunch& l) {
+    if (d->wfmt != BZ_W_BF16 || d->cfg_path || d->cfg_waves || d->cfg_tiles || d->cfg_depth) return false;
+    if (d->K > kRowsMaxK || (int64_t)rows * d->ldx * 2 >= (int64_t(1) << 31)) return false;
+    l.pair = d->epilogue == BZ_EPI_SILU_GATE;
+    const int spans = (d->K + 512 * kRowsMaxKc - 1) / (512 * kRowsMaxKc);
+    l.ks = spans <= 1 ? 1 : spans <= 2 ? 2 : 4;
+    l.kc = (d->K + 512 * l.ks - 1) / (512 * l.ks);
+    l.m = rows <= 2 ? rows : 4;
+    auto grid = [&](int r) {
+        const int64_t cols = (int64_t)(kRowsWaves / l.ks) * (l.pair ? r / 2 : r);
+        return (unsigned)((di.n_out + cols - 1) / cols);
+    };
+    const unsigned g4 = grid(4);
+    l.r = g4 < 256 || (g4 > 256 && g4 < 384) ? 2 : 4;
+    l.grid = grid(l.r);
+    return true;
+}
+
 }  // namespace bz
 
 using namespace bz;
@@ -792,6 +822,15 @@ extern "C" int bz_gemv(const bz_gemv_desc* d, void* stream) {
     if (rows < 1) return BZ_ERR_UNSUPPORTED;
     for (int m0 = 0; m0 < M; m0 += rows) {
         l.M = (M - m0) < rows ? (M - m0) : rows;
+        RowsLaunch rl;
+        if (rows_plan(d, di, l.M, rl)) {
+            p.x = static_cast<const uint16_t*>(d->x) + (int64_t)m0 * d->ldx;
+            p.out = static_cast<uint8_t*>(d->out) + (int64_t)m0 * d->ldo * osz;
+            p.res = d->residual ? static_cast<const uint8_t*>(d->residual) + (int64_t)m0 * d->ldr * rsz : nullptr;
+            const int rrc = launch_rows(p, rl, l.M, st);
+            if (rrc != BZ_OK) return rrc;
+            continue;
+        }
         const int lds = path == PATH_I8 ? i8_lds_layout(l.M, T, l.nw, K, tpw).total
                         : mfma          ? mfma_lds_layout(l.M, T, l.nw, K, wf, tpw).total
                                         : lds_layout(l.M, T, l.nw, K, wf, tpw).total;

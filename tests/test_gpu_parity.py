@@ -469,3 +469,23 @@ def test_rowmajor_full_size(name, fmt, n, k, norm, epi, m):
     xn = O.rmsnorm_f32(xf, O.bf16_bits_to_f32(gamma)) if norm else xf
     ref = O.gemv_ref(xn, w_eff, epi, O.bf16_bits_to_f32(res_bits) if epi == 2 else None)
     assert O.rel_err(f32(out), ref) <= TOL
+
+
+@pytest.mark.parametrize("N,K,epi", [(2, 8, 1), (34, 520, 1), (37, 1032, 0), (1030, 2560, 2), (1028, 2568, 2), (40, 5120, 0),
+                                     (36, 5128, 1), (26, 10240, 2), (1056, 520, 0), (9, 10248, 0)])
+@pytest.mark.parametrize("M", [1, 2, 3, 4, 6])
+def test_bf16_gemv_rule(N, K, epi, M):
+    """The bf16 GEMV's own launch shape: the edges of its 512-k pieces, of one,
+    two and four waves per row (2560, 5120, 10240) and past them, of its
+    columns per wave, with and without the norm and padded rows of x."""
+    w, gamma, x = O.synth(N, K, M, seed=N + M)
+    wb = O.f32_to_bf16_bits(w)
+    n_out = N // 2 if epi == 1 else N
+    res_bits = O.f32_to_bf16_bits(np.random.default_rng(8).standard_normal((M, n_out)).astype(np.float32))
+    wide = torch.full((M, K + 8), float("nan"), device="cuda", dtype=torch.bfloat16)
+    wide[:, :K] = bf16_tensor(x)
+    for norm in (False, True):
+        got = G.gemv(wide[:, :K], bf16_tensor(wb), G.W_BF16, N, gamma=bf16_tensor(gamma) if norm else None,
+                     epilogue=epi, residual=bf16_tensor(res_bits) if epi == 2 else None)
+        a, b = _xn(x, gamma, norm)
+        _check(got, a, b, O.bf16_bits_to_f32(wb), epi, O.bf16_bits_to_f32(res_bits) if epi == 2 else None)
