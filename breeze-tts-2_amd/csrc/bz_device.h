@@ -184,6 +184,20 @@ __device__ __forceinline__ uint32_t buffer_ld4(__amdgpu_buffer_rsrc_t r, uint32_
     return __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0);
 }
 
+// Element i of an array of 1 << log2 bytes each (log2 <= 2, chosen at run time)
+// as the aligned dword that holds it and the element's shift in it, without a
+// branch on the type: loads in the arms of a type branch made the compiler
+// wait for every load in flight where the arms meet.
+struct RawWord {
+    uint32_t w, shift;
+};
+__device__ __forceinline__ RawWord ld_elem(const void* p, int log2, int64_t i) {
+    const uint32_t low = (uint32_t)(reinterpret_cast<uintptr_t>(p) & 3u);
+    const int64_t at = (i << log2) + low;  // from the aligned dword that holds p
+    return {*reinterpret_cast<const uint32_t*>(static_cast<const char*>(p) - low + (at & ~(int64_t)3)),
+            (uint32_t)(at & 3) * 8u};
+}
+
 __device__ __forceinline__ float silu(float g) { return g / (1.0f + __expf(-g)); }
 
 // Lane placement of 16-byte pieces.  A wave instruction whose lane 4 a + b

@@ -16,8 +16,8 @@
 //     workgroup, whose sums meet in LDS (the only barrier).
 //   * The wave's R M sums are reduced over its lanes by DPP, in a fixed order.
 //   * Bound by HBM: 1.67 us of launch plus the bytes at the 7.39 TB/s of a plain
-//     read is 3.94 us for N4096 K2048 and 2.81 for N2048 K2048; it takes 4.66
-//     and 3.62 at M = 1, 4.96 and 3.80 at M = 2 (graph replays over 1 GiB of
+//     read is 3.94 us for N4096 K2048 and 2.81 for N2048 K2048; it takes 4.65
+//     and 3.48 at M = 1, 5.01 and 3.65 at M = 2 (graph replays over 1 GiB of
 //     weight copies on MI355X).  The kernel that staged x in LDS behind a
 //     barrier and walked its tiles through a rolling pipeline took 6.01, 4.94,
 //     6.94 and 5.36.
@@ -80,11 +80,8 @@ __global__ void __launch_bounds__(kRowsWaves * 64) gemv_rows(const uint16_t* hx,
     // output i = (row i / OC, column c0 + i % OC) belongs to lane i
     const int om = lane / OC, oc = c0 + lane % OC;
     const bool mine = lane < OC * M && om < hM && oc < hn_out;
-    float resv = 0.0f;
-    if (p.epi == BZ_EPI_RESIDUAL && mine) {
-        const int64_t ri = (int64_t)om * p.ldr + oc;
-        resv = p.res_f32 ? static_cast<const float*>(p.res)[ri] : bf16_to_f32(static_cast<const uint16_t*>(p.res)[ri]);
-    }
+    RawWord resv = {0u, 0u};
+    if (p.epi == BZ_EPI_RESIDUAL && mine) resv = ld_elem(p.res, p.res_f32 ? 2 : 1, (int64_t)om * p.ldr + oc);
     __builtin_amdgcn_sched_barrier(0);
 
     float ss[M];
@@ -168,7 +165,7 @@ __global__ void __launch_bounds__(kRowsWaves * 64) gemv_rows(const uint16_t* hx,
     const float inv = hnorm ? rsqrtf(s2 / (float)hK + p.eps) : 1.0f;
     a *= inv;
     if (PAIR) a = silu(a) * (b * inv);
-    a += resv;
+    if (p.epi == BZ_EPI_RESIDUAL) a += p.res_f32 ? __uint_as_float(resv.w) : bf16_lo(resv.w >> resv.shift);
     const int64_t oi = (int64_t)om * p.ldo + oc;
     if (p.out_f32)
         static_cast<float*>(p.out)[oi] = a;
