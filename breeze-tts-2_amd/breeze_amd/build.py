@@ -50,7 +50,7 @@ HIP_FLAGS = [
 NO_SCRATCH = (r"gemv_persist", r"gemv_mfma", r"gemv_i8mma", r"gemv_tile", r"gemv_stream", r"gemv_wide", r"gemv_panel",
               r"gemm_tiled", r"gemv_rows",
               r"head_f32", r"qkv_rope_cache",
-              r"attn_kernelILi[124]ELi\d+ELb0E")
+              r"attn_kernelILi[124]ELi\d+ELb0E", r"attn_bf16")
 
 
 def kernel_resources(remarks: str) -> list[tuple[str, int, int]]:

@@ -15,21 +15,20 @@
 // q_out fp32 [B][HQ][D]; out bf16 [B][ld_out] with q head h at columns
 // h*D..h*D+D-1.  Partials (split > 1) fp32 [B][HQ][split][D + 4] = (acc, m, l).
 //
-// attn_decode runs one workgroup per (batch row, kv head, split), so the G =
+// Attention runs one workgroup per (batch row, kv head, split), so the G =
 // HQ/HKV query heads sharing a kv head read its keys and values once.  Its
-// four waves take 16-position blocks of the split in turn:
-//   scores   v_mfma_f32_16x16x32_bf16 with A = the G query rows (padded to
-//            16) and B = 16 key rows; q is carried as bf16 hi + lo parts
-//            (two MFMAs, ~16 significant bits; an fp32 cache also splits k)
+// waves take 16-position blocks in turn:
+//   scores   v_mfma_f32_16x16x32_bf16 over key rows and query rows; q is
+//            carried as bf16 hi + lo parts (two MFMAs, ~16 significant bits;
+//            an fp32 cache also splits k)
 //   softmax  online (running max m, sum l) per head, exp2-based
-//   p v      bf16 cache, D <= 256: v_mfma_f32_16x16x16_bf16 per 16-column
-//            tile, A = p (through LDS, as bf16 hi + lo), B = 4 value rows
-//            of one column, which lane (col, grp) loads directly (4 rows x
-//            D/16 contiguous columns) so no cross-lane transpose is needed;
-//            fp32 cache or D = 512: VALU, lane l owns D/64 consecutive
-//            columns of every head and reads each value row with one
-//            coalesced load
+//   p v      bf16 cache, D <= 256 (attn_bf16): v_mfma_f32_16x16x16_bf16 per
+//            16 columns, p as bf16 hi + lo; fp32 cache or D = 512
+//            (attn_kernel): VALU, lane l owns D/64 consecutive columns of
+//            every head and reads each value row with one coalesced load
 // The waves' (m, l, acc) are merged through LDS in a fixed order.
+#include <algorithm>
+
 #include "bz_attn.h"
 #include "bz_device.h"
 
@@ -68,6 +67,18 @@ __device__ __forceinline__ uint32_t ld_raw(const void* p, int kind, int64_t i) {
     if (kind == BZ_DT_F32) return reinterpret_cast<const uint32_t*>(p)[i];
     if (kind == BZ_MASK_BOOL) return reinterpret_cast<const uint8_t*>(p)[i];
     return reinterpret_cast<const uint16_t*>(p)[i];
+}
+
+// Element i of such an array without a branch on the type (ld_elem), and its
+// value once the dword is there.
+__device__ __forceinline__ RawWord ld_word(const void* p, int kind, int64_t i) {
+    return ld_elem(p, kind == BZ_DT_F32 ? 2 : (kind == BZ_MASK_BOOL ? 0 : 1), i);
+}
+__device__ __forceinline__ float word_f32(RawWord r, int kind) {
+    const uint32_t raw = r.w >> r.shift;
+    const float num = __uint_as_float(kind == BZ_DT_F32 ? raw : raw << 16);
+    const float allow = raw & 0xFFu ? 0.0f : -1e30f;
+    return kind == BZ_MASK_BOOL ? allow : num;
 }
 
 // bf16 / fp32 as a value; a bool mask entry as additive (nonzero = attend
@@ -126,25 +137,17 @@ __global__ void __launch_bounds__(kRopeThreads) qkv_rope_cache_kernel(
     const void* cosp, const void* sinp, bool cs_f32, int64_t ld_cs, const int64_t* pos_p, float* q_out, void* kc,
     void* vc, int S, bool cache_f32, int64_t* seq_len) {
     __shared__ float vals[kMaxRopeDim];
-    __shared__ float part[kRopeThreads / 64];
     const int b = blockIdx.x, h = blockIdx.y;
     const bool is_q = h < HQ;
     const uint16_t* src = qkv + (int64_t)b * ld_qkv + (int64_t)h * D;
     const uint16_t* nw = is_q ? qn : kn;
-    float ss = 0.0f;
-    for (int d = threadIdx.x; d < D; d += kRopeThreads) {
-        const float v = bf16_to_f32(src[d]);
-        vals[d] = v;
-        ss += v * v;
-    }
-    ss = wave_sum64(ss);
-    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = ss;
+    for (int d = threadIdx.x; d < D; d += kRopeThreads) vals[d] = bf16_to_f32(src[d]);
     __syncthreads();
     float inv = 1.0f;
-    if (nw) {
-        float t = 0.0f;
-        for (int w = 0; w < kRopeThreads / 64; ++w) t += part[w];
-        inv = 1.0f / sqrtf(t / (float)D + eps);
+    if (nw) {  // every wave, in the order of attn_bf16: columns l + 64 e of a lane, then the lanes
+        float ss = 0.0f;
+        for (int d = threadIdx.x & 63; d < D; d += 64) ss = fmaf(vals[d], vals[d], ss);
+        inv = 1.0f / sqrtf(wave_sum64(ss) / (float)D + eps);
     }
     const int half = D >> 1;
     const int64_t cs = (int64_t)b * ld_cs;
@@ -176,7 +179,7 @@ __global__ void __launch_bounds__(kRopeThreads) qkv_rope_cache_kernel(
 // Decode attention: one workgroup per (batch row b, kv head j, split sp).
 // ---------------------------------------------------------------------------
 constexpr int kBlk = 16;           // positions per block (the MFMA's 16 columns)
-constexpr int kUnsplitMax = 160;   // attended positions up to which a call runs unsplit
+constexpr int kUnsplitMax = 160;   // attended positions up to which attn_kernel runs unsplit
 constexpr float kNegBig = -1e30f;  // initial running max, as the reference
 constexpr float kLog2e = 1.4426950408889634f;
 
@@ -206,26 +209,21 @@ struct AttnParams {
     const int64_t* pos;
     float scale;
     int HQ, HKV, G, S, split;
+    int split_cap;       // splits attn_bf16 uses at most: split, or one workgroup per CU
     float* part;         // [B][HQ][split][D + 4] (acc, m, l, 2 pad)
     unsigned* counters;  // [B][HKV] arrivals, zero between calls
     uint16_t* out;
     int64_t ld_out;
 };
 
-// The registers of one 16-position block: key operands and raw value words.
-// MV (bf16 cache, D <= 256): p v on the matrix cores, and lane (col, grp)
-// holds value rows 4 grp .. 4 grp + 3 of the block at columns D/16 col ..
-// D/16 col + D/16 - 1 -- column D/16 col + c of those 4 rows is exactly the
-// B operand of the 16x16x16 MFMA of column tile c.  Otherwise (VALU p v)
-// lane l holds columns DL l .. DL l + DL - 1 of all 16 rows.
+// attn_kernel's registers of one 16-position block: key operands and raw
+// value words (lane l holds columns DL l .. DL l + DL - 1 of all 16 rows).
 template <int DL, bool F32C>
 struct KvBlock {
-    static constexpr int T = 2 * DL;  // MFMA k-steps per key row
-    static constexpr bool MV = !F32C && DL <= 4;
-    static constexpr int VW = MV ? 2 * DL : (F32C ? DL : (DL >= 2 ? DL / 2 : 1));  // value words per row
-    static constexpr int VR = MV ? 4 : kBlk;                                     // value rows per lane
+    static constexpr int T = 2 * DL;                                    // MFMA k-steps per key row
+    static constexpr int VW = F32C ? DL : (DL >= 2 ? DL / 2 : 1);  // value words per row
     u32x4 kh[T], kl[T];
-    uint32_t v[VR][VW];
+    uint32_t v[kBlk][VW];
     uint32_t mraw;  // raw mask entry at this lane's key position
 };
 
@@ -285,68 +283,26 @@ __device__ __forceinline__ float vword(const uint32_t (&w)[KvBlock<DL, F32C>::VW
     return (e & 1) ? bf16_hi(w[e >> 1]) : bf16_lo(w[e >> 1]);
 }
 
-// bf16 caches with D = 128 or 256 (the matrix-core p v path) load a block
-// through range-checked buffer loads over the (row, kv head)'s cache, so a
-// wave can issue a block's loads that send no request (an empty range).
-__host__ __device__ constexpr bool kv_buffered(int DL, bool F32C) { return !F32C && DL >= 2 && DL <= 4; }
-
 // One block's loads: key rows s0 + col (lane col), value rows s0 .. s0 + 15
 // and the mask entries, rows past the split's last one clamped to it.  s0
 // and s_hi are wave-uniform, so the value rows' addresses are scalar and
-// each load carries only the lane's column offset.  On the buffered path a
-// block that is not `live` reads zeros without memory requests (its mask
-// entry still loads, at a clamped position); the other paths always load.
+// each load carries only the lane's column offset.
 template <int DL, bool F32C>
 __device__ __forceinline__ void load_block(const AttnParams& a, int64_t kv_base, int s0, int s_hi, int64_t mrow,
-                                           int lane, KvBlock<DL, F32C>& blk, bool live = true) {
+                                           int lane, KvBlock<DL, F32C>& blk) {
     constexpr int D = 64 * DL;
     constexpr int ES = F32C ? 4 : 2;  // element bytes
     const int last = max(s_hi - 1, 0);  // an empty range reads row 0 (every cache has one), unused
     const int col = lane & 15, grp = lane >> 4;
     const int kpos = min(s0 + col, last);
     blk.mraw = ld_raw(a.mask, a.mask_dtype, mrow + kpos);  // first: its load depends on the dtype
-    if constexpr (kv_buffered(DL, F32C)) {
-        const uint32_t bytes = live ? (uint32_t)a.S * (D * 2) : 0u;  // S D 2 < 2^32 (checked at set-up)
-        const __amdgpu_buffer_rsrc_t kr = buffer_rsrc(static_cast<const char*>(a.kc) + kv_base * 2, bytes);
-        const __amdgpu_buffer_rsrc_t vr = buffer_rsrc(static_cast<const char*>(a.vc) + kv_base * 2, bytes);
-        const uint32_t ko = (uint32_t)kpos * (D * 2) + 16 * grp;
-        for (int t = 0; t < KvBlock<DL, F32C>::T; ++t) {
-            blk.kh[t] = buffer_ld16(kr, ko + 64 * t);
-            blk.kl[t] = u32x4{0u, 0u, 0u, 0u};
-        }
-        for (int r = 0; r < 4; ++r) {
-            const uint32_t vo = (uint32_t)min(s0 + 4 * grp + r, last) * (D * 2) + 8 * DL * col;
-            for (int i = 0; i < DL / 2; ++i) {
-                const u32x4 t = buffer_ld16(vr, vo + 16 * i);
-                for (int e = 0; e < 4; ++e) blk.v[r][4 * i + e] = t[e];
-            }
-        }
-        return;
-    }
     const char* kc = static_cast<const char*>(a.kc) + kv_base * ES;
     const char* krow = kc + (int64_t)kpos * (D * ES) + 8 * grp * ES;
     for (int t = 0; t < KvBlock<DL, F32C>::T; ++t) load_k8<F32C>(krow, 32 * t, blk.kh[t], blk.kl[t]);
     const char* vc = static_cast<const char*>(a.vc) + kv_base * ES;
-    if constexpr (KvBlock<DL, F32C>::MV) {
-        for (int r = 0; r < 4; ++r) {
-            const int row = min(s0 + 4 * grp + r, last);
-            const uint16_t* vp = reinterpret_cast<const uint16_t*>(vc + (int64_t)row * (D * ES)) + 4 * DL * col;
-            if constexpr (DL == 1) {
-                const u32x2 t = *reinterpret_cast<const u32x2*>(vp);
-                blk.v[r][0] = t[0];
-                blk.v[r][1] = t[1];
-            } else {
-                for (int i = 0; i < DL / 2; ++i) {
-                    const u32x4 t = ldg16(vp + 8 * i);
-                    for (int e = 0; e < 4; ++e) blk.v[r][4 * i + e] = t[e];
-                }
-            }
-        }
-    } else {
-        for (int p = 0; p < kBlk; ++p) {
-            const int row = min(s0 + p, last);
-            load_vraw<DL, F32C>(vc + (int64_t)row * (D * ES), DL * lane, blk.v[p]);
-        }
+    for (int p = 0; p < kBlk; ++p) {
+        const int row = min(s0 + p, last);
+        load_vraw<DL, F32C>(vc + (int64_t)row * (D * ES), DL * lane, blk.v[p]);
     }
 }
 
@@ -370,6 +326,456 @@ __device__ __forceinline__ float sum16(float v) {
 
 __device__ __forceinline__ float bcast(float v, int lane) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
+}
+
+// The waves' state in LDS ([wave][GM heads], accumulator rows of ROW floats),
+// behind a barrier, into the output or, over nsp > 1 splits, the workspace,
+// whose last arrival combines them.  The first nact waves have state.
+template <int D, int GM, int NWV, int ROW>
+__device__ __forceinline__ void merge_and_combine(const AttnParams& a, int b, int j, int sp, int nsp, int nact, int tid,
+                                                  const float* st_m, const float* st_l, const float* st_acc, int* last) {
+    // Merge the waves in a fixed order; write the output or the partial.
+    // Each thread forms its head's wave weights itself (8 values from LDS):
+    // no serial step and no barrier between the state and the merge.
+    constexpr int kThreads = 64 * NWV;
+    const int G = a.G;
+    const int64_t hq0 = (int64_t)b * a.HQ + (int64_t)j * G;
+    for (int i = tid; i < G * D; i += kThreads) {
+        const int h = i / D, d = i - h * D;
+        float mt = kNegBig;
+        for (int w = 0; w < nact; ++w) mt = fmaxf(mt, st_m[w * GM + h]);
+        float lt = 0.0f, at = 0.0f;
+        for (int w = 0; w < nact; ++w) {
+            const float f = fexp2((st_m[w * GM + h] - mt) * kLog2e);
+            lt += st_l[w * GM + h] * f;
+            at += st_acc[(w * GM + h) * ROW + d] * f;
+        }
+        if (nsp == 1) {
+            a.out[(int64_t)b * a.ld_out + (int64_t)(j * G + h) * D + d] = f32_to_bf16(lt > 0.0f ? at / lt : 0.0f);
+        } else {  // agent-scope stores: coherent across XCDs without an L2 write-back
+            float* pp = a.part + ((hq0 + h) * a.split + sp) * (D + 4);
+            __hip_atomic_store(&pp[d], at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (d == 0) {
+                __hip_atomic_store(&pp[D], mt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                __hip_atomic_store(&pp[D + 1], lt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+        }
+    }
+    if (nsp == 1) return;
+
+    // The last workgroup of (b, j) to finish combines the splits.  Every
+    // thread waits until its partial stores have completed (agent-scope
+    // stores complete at the point of coherence) before the workgroup counts
+    // its arrival; the last one reads the partials with agent-scope loads.
+    // No L2 write-back or invalidate is needed for that.
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (tid == 0) {
+        const unsigned prev =
+            __hip_atomic_fetch_add(&a.counters[b * a.HKV + j], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        *last = prev == (unsigned)nsp - 1u;
+    }
+    __syncthreads();
+    if (!*last) return;
+    // Element i = (h, d): each thread loads, for its NE elements, every
+    // split's partial and its head's (m, l) in batches of SB splits (all in
+    // flight at once; SB NE <= 16 keeps them in registers), and merges them
+    // in split order, online: with M the running max, acc and L are rescaled
+    // by exp(M_old - M) and gain w_s acc_s and w_s l_s, w_s = exp(m_s - M).
+    // One memory round trip per batch and no barrier (the weights were first
+    // formed per head in LDS: a second round trip and a barrier).
+    constexpr int NE = (GM * D + kThreads - 1) / kThreads;
+    constexpr int SB = NE <= 2 ? 8 : (NE <= 4 ? 4 : (NE <= 8 ? 2 : 1));
+    float acc0[NE], lsum[NE], mrun[NE];
+    for (int q = 0; q < NE; ++q) {
+        acc0[q] = 0.0f;
+        lsum[q] = 0.0f;
+        mrun[q] = kNegBig;
+    }
+    for (int s0 = 0; s0 < nsp; s0 += SB) {
+        float v[NE][SB], ms[NE][SB], ls[NE][SB];
+        for (int q = 0; q < NE; ++q) {
+            const int i = min(tid + q * kThreads, G * D - 1);
+            const int h = i / D, d = i - h * D;
+            const float* ph = a.part + (hq0 + h) * a.split * (D + 4);
+            for (int u = 0; u < SB; ++u) {
+                const float* pp = ph + min(s0 + u, nsp - 1) * (D + 4);
+                v[q][u] = __hip_atomic_load(pp + d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                ms[q][u] = __hip_atomic_load(pp + D, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                ls[q][u] = __hip_atomic_load(pp + D + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+        }
+        for (int q = 0; q < NE; ++q) {
+            float mb = mrun[q];
+            for (int u = 0; u < SB; ++u)
+                if (s0 + u < nsp) mb = fmaxf(mb, ms[q][u]);
+            const float rs = fexp2((mrun[q] - mb) * kLog2e);
+            acc0[q] *= rs;
+            lsum[q] *= rs;
+            mrun[q] = mb;
+            for (int u = 0; u < SB; ++u)
+                if (s0 + u < nsp) {
+                    const float w = fexp2((ms[q][u] - mb) * kLog2e);
+                    acc0[q] += v[q][u] * w;
+                    lsum[q] += ls[q][u] * w;
+                }
+        }
+    }
+    for (int q = 0; q < NE; ++q) {
+        const int i = tid + q * kThreads;
+        if (i < G * D) {
+            const int h = i / D, d = i - h * D;
+            const float lt = lsum[q];
+            a.out[(int64_t)b * a.ld_out + (int64_t)(j * G + h) * D + d] =
+                f32_to_bf16(lt > 0.0f ? acc0[q] / lt : 0.0f);
+        }
+    }
+    if (tid == 0) __hip_atomic_store(&a.counters[b * a.HKV + j], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// ---------------------------------------------------------------------------
+// Decode attention over a bf16 cache, D = 64, 128 or 256: one workgroup per
+// (batch row b, kv head j, split sp), its waves taking 16-position blocks.
+//
+// Bound by latency: a step attends a few hundred positions, so each wave has
+// one or two blocks and the chain launch, loads, q, scores, softmax, p v,
+// merge is what it takes.  Hence
+//   * one barrier before the blocks: a wave norms and rotates a whole q or k
+//     head by itself (its sum of squares by DPP, the rotary partner column in
+//     the same lane) and writes it to LDS as the MFMA operand's hi and lo
+//     bf16 parts; the new key and value reach the block that holds them
+//     through LDS too, not through the cache;
+//   * the scores transposed, A = 16 key rows, B = the G <= 16 query heads:
+//     lane (head, grp) gets positions 4 grp .. 4 grp + 3, which is exactly the B
+//     operand of p v on v_mfma_f32_16x16x16_bf16 (A = the transposed value
+//     rows), so p never leaves its lane; a head's max and sum over the
+//     positions are two lane-row swaps (v_permlane32_swap, v_permlane16_swap);
+//   * the first workgroup of a (row, kv head) issues its first blocks' loads
+//     before it knows the position: block wave + NW sp is its first whatever
+//     the number of splits in use.
+//   * loads whose element type is a run-time argument (mask, cos, sin) take the
+//     aligned dword: a branch on the type put a wait for everything in flight
+//     at its end.
+// Measured on MI355X (cold caches, graph replays, default split) against the
+// kernel with four prologue barriers, scores not transposed and p through
+// LDS: 8 / 2 heads of 128, B = 2, 17 positions 5.25 -> 4.11 us; 16 / 8 heads of
+// 128, B = 2, 612 of 1024 positions 8.61 -> 7.59; 16 / 4 heads of 256, B = 2,
+// 128 positions 8.87 -> 7.82, 1902 of 2048 13.9 -> 12.8.
+// ---------------------------------------------------------------------------
+template <int DL>
+struct KvRows {
+    u32x4 k[2 * DL];         // key row `col`, elements 32 t + 8 grp + 0..7
+    uint32_t v[4][2 * DL];   // value rows 4 grp + r, columns v_col(c, col) of attn_bf16, c = 0..4 DL - 1
+    RawWord mraw[4];         // mask entries of positions 4 grp + r
+};
+
+// Reduce over the four 16-lane rows of a wave; every lane gets the result of
+// its column.
+template <typename F>
+__device__ __forceinline__ float across_rows(float v, F f) {
+    const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    const float t = f(__uint_as_float(a[0]), __uint_as_float(a[1]));
+    const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(t), __float_as_uint(t), false, false);
+    return f(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+
+template <int DL, int GM, bool FUSED, int NWV>
+__global__ void __launch_bounds__(64 * NWV) attn_bf16(const void* hrows, const void* hcos, const void* hsin,
+                                                      const int64_t* hpos, void* hkc, void* hvc, int hld_qkv,
+                                                      uint32_t hshape, AttnParams a) {
+    constexpr int D = 64 * DL, T = 2 * DL, NT = 4 * DL;
+    // column of operand row i of p v's tile c: lanes read value rows in runs
+    // of 16 bytes side by side (with each lane's columns contiguous, a 256-wide
+    // row took two half-used passes over its lines)
+    auto v_col = [](int c, int i) { return DL == 1 ? 4 * i + c : 128 * (c >> 3) + 8 * i + (c & 7); };
+    constexpr int kAccRow = D + 4;  // floats of one head's partial (16-byte rows, off the bank period)
+    __shared__ u32x4 qop[T][2][64];             // B operands of the query heads: hi, lo
+    __shared__ __attribute__((aligned(16))) uint16_t knew[D], vnew[D];  // the new token's key and value
+    __shared__ float st_m[NWV][GM], st_l[NWV][GM];
+    __shared__ __attribute__((aligned(16))) float st_acc[NWV][GM][kAccRow];
+    __shared__ int last;
+    const int b = blockIdx.x, j = blockIdx.y, sp = blockIdx.z;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int col = lane & 15, grp = lane >> 4;
+    const int G = hshape & 31u, HKV = (hshape >> 5) & 0xFFFFu, HQ = G * HKV;
+
+    const int64_t pos = *hpos;
+
+    // 1. raw rows of the prologue: row r = wave + NWV i is query head j G + r
+    //    (r < G), the key head (r = G) or the value head (G + 1); lane l holds
+    //    columns l + 64 e.  Rows past the last read as zeros without requests.
+    constexpr int NR = FUSED ? GM + 2 : GM, NI = (NR + NWV - 1) / NWV;
+    const int nrows = FUSED ? G + 2 : G;
+    uint32_t raw[NI][DL], nw[NI][DL];
+    RawWord cs[DL], sn[DL];
+    const int cs_kind = hshape >> 21 & 1u ? BZ_DT_F32 : BZ_DT_BF16;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+        const int r = wave + NWV * i;
+        if constexpr (FUSED) {
+            const int head = r < G ? j * G + r : (r == G ? HQ + j : HQ + HKV + j);
+            const __amdgpu_buffer_rsrc_t rs = buffer_rsrc(
+                static_cast<const uint16_t*>(hrows) + (int64_t)b * hld_qkv + (int64_t)(r < nrows ? head : 0) * D,
+                r < nrows ? (uint32_t)D * 2u : 0u);
+#pragma unroll
+            for (int e = 0; e < DL; ++e) raw[i][e] = __builtin_amdgcn_raw_buffer_load_b16(rs, (lane + 64 * e) * 2, 0, 0);
+        } else {
+            const __amdgpu_buffer_rsrc_t rs =
+                buffer_rsrc(static_cast<const float*>(hrows) + ((int64_t)b * HQ + (int64_t)j * G + (r < nrows ? r : 0)) * D,
+                            r < nrows ? (uint32_t)D * 4u : 0u);
+#pragma unroll
+            for (int e = 0; e < DL; ++e) raw[i][e] = buffer_ld4(rs, (lane + 64 * e) * 4);
+        }
+    }
+    if constexpr (FUSED) {
+        const int64_t c0 = hshape >> 22 & 1u ? 0 : (int64_t)b * a.ld_cs;
+#pragma unroll
+        for (int e = 0; e < DL; ++e) {
+            cs[e] = ld_word(hcos, cs_kind, c0 + lane + 64 * e);
+            sn[e] = ld_word(hsin, cs_kind, c0 + lane + 64 * e);
+        }
+        // (everything so far needs preloaded arguments only)
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            const int r = wave + NWV * i;
+            const uint16_t* w = r < G ? a.qn : a.kn;  // without norm weights or past the normed rows: an empty range
+            const __amdgpu_buffer_rsrc_t ws = buffer_rsrc(w, w && r <= G ? (uint32_t)D * 2u : 0u);
+#pragma unroll
+            for (int e = 0; e < DL; ++e) nw[i][e] = __builtin_amdgcn_raw_buffer_load_b16(ws, (lane + 64 * e) * 2, 0, 0);
+        }
+    }
+
+    // 2. the wave's first block.  Rows past the cache read as zeros; rows past
+    //    the attended range are loaded as they are and dropped below.
+    const int64_t kv_base = ((int64_t)b * HKV + j) * a.S * D;
+    const uint32_t kv_bytes = (uint32_t)a.S * (D * 2);  // S D 4 < 2^32 (checked at set-up)
+    const int64_t mrow = (int64_t)b * a.ld_mask;
+    auto load_rows = [&](KvRows<DL>& blk, int s0, uint32_t bytes) {
+        const __amdgpu_buffer_rsrc_t kr = buffer_rsrc(static_cast<const uint16_t*>(hkc) + kv_base, bytes);
+        const __amdgpu_buffer_rsrc_t vr = buffer_rsrc(static_cast<const uint16_t*>(hvc) + kv_base, bytes);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) blk.mraw[r] = ld_word(a.mask, a.mask_dtype, mrow + min(s0 + 4 * grp + r, a.S - 1));
+        const uint32_t ko = (uint32_t)(s0 + col) * (D * 2) + 16 * grp;
+#pragma unroll
+        for (int t = 0; t < T; ++t) blk.k[t] = buffer_ld16(kr, ko + 64 * t);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const uint32_t vo = (uint32_t)(s0 + 4 * grp + r) * (D * 2) + (DL == 1 ? 8 : 16) * col;
+            if constexpr (DL == 1) {
+                const u32x2 t = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(vr, vo, 0, 0));
+                blk.v[r][0] = t[0];
+                blk.v[r][1] = t[1];
+            } else {
+#pragma unroll
+                for (int i = 0; i < DL / 2; ++i) {
+                    const u32x4 t = buffer_ld16(vr, vo + 256 * i);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) blk.v[r][4 * i + e] = t[e];
+                }
+            }
+        }
+    };
+    // cache positions [0, min(pos, S - 1)]; none for pos < 0 (output 0)
+    const int kv_len = pos < 0 ? 0 : (pos >= a.S ? a.S : (int)pos + 1);
+    const int nblk = (kv_len + kBlk - 1) / kBlk;
+    // Splits in use (decided from the device position, so a captured graph
+    // follows it): none while two blocks per wave cover the positions, else
+    // as many as have a block for every wave, and no more workgroups than
+    // CUs; the others leave before any barrier.  Measured on MI355X, unsplit
+    // against 8 splits: D = 128 (16 / 8 heads, B = 2) 6.56 / 7.02 us at 256
+    // positions, 7.59 / 7.03 at 331; D = 256 (16 / 4 heads, B = 1) 8.69 / 8.78
+    // at 160, 10.35 / 10.01 at 256.  64 (row, kv head) pairs at 2001 positions:
+    // 4 splits 16.6 us, 5 21.8, 8 19.5, 16 25.8.
+    constexpr int kUnsplit = DL == 4 ? 224 : 256;
+    const int nsp =
+        kv_len <= kUnsplit ? 1 : min(a.split_cap, (nblk + NWV - 1) / NWV);
+    KvRows<DL> cur;
+    int s0 = (sp * NWV + wave) * kBlk;
+    uint32_t live = kv_bytes;
+    if (sp != 0) {  // split 0 does not wait for the position here
+        if (sp >= nsp) return;
+        if (s0 >= kv_len) live = 0u;
+    }
+    load_rows(cur, s0, live);
+
+    const int new_blk = FUSED && pos >= 0 && pos < a.S ? (int)pos / kBlk : -1;  // holds the new token
+    const bool has_new = new_blk >= 0 && (new_blk / NWV) % nsp == sp;
+
+    // 3. each wave's rows: norm, rotate, to LDS
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+        const int r = wave + NWV * i;
+        if (r >= nrows) continue;
+        float v[DL];
+        if constexpr (FUSED) {
+            if (r == G + 1) {
+                if (has_new) {
+#pragma unroll
+                    for (int e = 0; e < DL; ++e) {
+                        const int d = lane + 64 * e;
+                        vnew[d] = (uint16_t)raw[i][e];
+                        static_cast<uint16_t*>(hvc)[kv_base + pos * D + d] = (uint16_t)raw[i][e];
+                    }
+                }
+                continue;
+            }
+            float ss = 0.0f;
+#pragma unroll
+            for (int e = 0; e < DL; ++e) {
+                v[e] = __uint_as_float(raw[i][e] << 16);
+                ss = fmaf(v[e], v[e], ss);
+            }
+            if (a.qn) {
+                const float inv = 1.0f / sqrtf(wave_sum64(ss) / (float)D + a.eps);
+#pragma unroll
+                for (int e = 0; e < DL; ++e) v[e] = v[e] * inv * __uint_as_float(nw[i][e] << 16);
+            }
+            // rotate_half(v) = [-v2, v1]; the partner column d +- D/2 is in
+            // this lane (D >= 128) or 32 lanes away (D = 64)
+            float o[DL];
+#pragma unroll
+            for (int e = 0; e < DL; ++e) {
+                float rr;
+                if constexpr (DL == 1) {
+                    rr = __shfl_xor(v[0], 32, 64);
+                    if (lane < 32) rr = -rr;
+                } else {
+                    rr = e < DL / 2 ? -v[e + DL / 2] : v[e - DL / 2];
+                }
+                o[e] = v[e] * word_f32(cs[e], cs_kind) + rr * word_f32(sn[e], cs_kind);
+            }
+            if (r == G) {
+                if (has_new) {
+#pragma unroll
+                    for (int e = 0; e < DL; ++e) {
+                        const int d = lane + 64 * e;
+                        const uint16_t h = f32_to_bf16(o[e]);
+                        knew[d] = h;
+                        static_cast<uint16_t*>(hkc)[kv_base + pos * D + d] = h;
+                    }
+                }
+                continue;
+            }
+#pragma unroll
+            for (int e = 0; e < DL; ++e) v[e] = o[e];
+        } else {
+#pragma unroll
+            for (int e = 0; e < DL; ++e) v[e] = __uint_as_float(raw[i][e]);
+        }
+        // element d of head r: step d / 32, lane r + 16 ((d / 8) % 4), element d % 8
+        uint16_t* q16 = reinterpret_cast<uint16_t*>(&qop[0][0][0]);
+#pragma unroll
+        for (int e = 0; e < DL; ++e) {
+            const int d = lane + 64 * e;
+            const int at = ((d >> 5) * 2 * 64 + r + 16 * ((d >> 3) & 3)) * 8 + (d & 7);
+            const float x = v[e] * a.scale;
+            const uint16_t h = f32_to_bf16(x);
+            q16[at] = h;
+            q16[at + 64 * 8] = f32_to_bf16(x - bf16_to_f32(h));
+        }
+    }
+    if (FUSED && a.seq_len && b == 0 && j == 0 && sp == 0 && tid == 0) *a.seq_len = pos + 1;
+    __syncthreads();
+
+    // 4. the wave's blocks: lane (col, grp) holds head col's scores at
+    //    positions 4 grp + r; m is the head's running max (the same in its
+    //    four lanes), l this lane's share of the sum, acc[c][r] the head's
+    //    output at column v_col(c, 4 grp + r)
+    float m = kNegBig, l = 0.0f;
+    f32x4_t acc[NT];
+#pragma unroll
+    for (int c = 0; c < NT; ++c) acc[c] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    const bool any = s0 < kv_len;
+    auto process = [&](KvRows<DL>& cur, int s0) __attribute__((always_inline)) {
+        if (has_new && s0 == new_blk * kBlk) {  // uniform: the new token's rows from LDS
+            const int at = (int)pos - s0;
+            u32x4 kn[T];
+            uint32_t vn[2 * DL];
+#pragma unroll
+            for (int t = 0; t < T; ++t) kn[t] = *reinterpret_cast<const u32x4*>(&knew[32 * t + 8 * grp]);
+#pragma unroll
+            for (int i = 0; i < 2 * DL; ++i) vn[i] = *reinterpret_cast<const uint32_t*>(&vnew[v_col(2 * i, col)]);
+#pragma unroll
+            for (int t = 0; t < T; ++t)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) cur.k[t][q] = col == at ? kn[t][q] : cur.k[t][q];
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int i = 0; i < 2 * DL; ++i) cur.v[r][i] = 4 * grp + r == at ? vn[i] : cur.v[r][i];
+        }
+        f32x4_t sc = {0.0f, 0.0f, 0.0f, 0.0f}, sl = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int t = 0; t < T; ++t) {
+            sc = mfma16(cur.k[t], qop[t][0][lane], sc);
+            sl = mfma16(cur.k[t], qop[t][1][lane], sl);
+        }
+        float s[4], bm = kNegBig;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const bool valid = s0 + 4 * grp + r < kv_len;
+            s[r] = valid ? sc[r] + sl[r] + word_f32(cur.mraw[r], a.mask_dtype) : kNegBig;
+            bm = fmaxf(bm, s[r]);
+            // (a value row past the range may hold anything)
+#pragma unroll
+            for (int i = 0; i < 2 * DL; ++i) cur.v[r][i] = valid ? cur.v[r][i] : 0u;
+        }
+        const float mn = fmaxf(m, across_rows(bm, [](float x, float y) { return fmaxf(x, y); }));
+        const float alpha = fexp2((m - mn) * kLog2e);
+        m = mn;
+        float p[4], ps = 0.0f;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            p[r] = s0 + 4 * grp + r < kv_len ? fexp2((s[r] - mn) * kLog2e) : 0.0f;
+            ps += p[r];
+        }
+        l = l * alpha + ps;
+        const uint32_t h01 = pack_bf16x2(p[0], p[1]), h23 = pack_bf16x2(p[2], p[3]);
+        const u32x2 ph = {h01, h23};
+        const u32x2 pl = {pack_bf16x2(p[0] - bf16_lo(h01), p[1] - bf16_hi(h01)),
+                          pack_bf16x2(p[2] - bf16_lo(h23), p[3] - bf16_hi(h23))};
+#pragma unroll
+        for (int c = 0; c < NT; ++c) {
+            // A: column v_col(c, col) of value rows 4 grp .. 4 grp + 3
+            const uint32_t w0 = cur.v[0][c >> 1], w1 = cur.v[1][c >> 1], w2 = cur.v[2][c >> 1], w3 = cur.v[3][c >> 1];
+            const uint32_t sel = c & 1 ? 0x07060302u : 0x05040100u;  // high or low halves of a pair of rows
+            const u32x2 av = {__builtin_amdgcn_perm(w1, w0, sel), __builtin_amdgcn_perm(w3, w2, sel)};
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[c][r] *= alpha;
+            acc[c] = mfma16k16(av, ph, acc[c]);
+            acc[c] = mfma16k16(av, pl, acc[c]);
+        }
+    };
+    // (the first block by itself: behind a loop the waits for its key rows
+    // would also wait for its value rows)
+    if (any) process(cur, s0);
+    for (s0 += nsp * NWV * kBlk; s0 < kv_len; s0 += nsp * NWV * kBlk) {
+        load_rows(cur, s0, kv_bytes);
+        process(cur, s0);
+    }
+
+    // 5. the waves' state to LDS, merged in wave order; a wave past the
+    //    positions has none
+    const int nact = min(NWV, nblk - sp * NWV);  // <= 0 only without any position
+    if (any) {
+        l = across_rows(l, [](float x, float y) { return x + y; });
+        if (col < G) {
+            if (grp == 0) {
+                st_m[wave][col] = m;
+                st_l[wave][col] = l;
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int c = 0; c < NT; c += 4)
+                    *reinterpret_cast<float4*>(&st_acc[wave][col][v_col(c, 4 * grp + r)]) =
+                        make_float4(acc[c][r], acc[c + 1][r], acc[c + 2][r], acc[c + 3][r]);
+        }
+    }
+    __syncthreads();
+    merge_and_combine<D, GM, NWV, kAccRow>(a, b, j, sp, nsp, nact, tid, &st_m[0][0], &st_l[0][0], &st_acc[0][0][0], &last);
 }
 
 // DL = D / 64 columns per lane; GM = 4 or 16 heads of register state (G <=
@@ -396,15 +802,12 @@ __global__ void __launch_bounds__(64 * NWV) attn_kernel(const void* hrows, const
     constexpr int kAttnThreads = 64 * NWV;
     constexpr int D = 64 * DL;
     constexpr int T = D / 32;
-    constexpr bool PF = !F32C && DL <= 4 && NWV == 4;  // prefetch the next block (registers allow it)
     using Blk = KvBlock<DL, F32C>;
-    constexpr bool MV = Blk::MV;          // p v on the matrix cores
-    constexpr int NT = D / 16;            // its column tiles
     __shared__ float qf[GM][D];
     __shared__ float css[(GM + 2) * DL];
     __shared__ float rinv[GM + 1];
     __shared__ u32x4 qop[T][2][64];  // the A operand (q hi, lo) of every lane
-    __shared__ float p_lds[kAttnWaves][kBlk * GM];  // MV: [head][position], else [position][head]
+    __shared__ float p_lds[kAttnWaves][kBlk * GM];  // [position][head]
     __shared__ float st_m[kAttnWaves][GM], st_l[kAttnWaves][GM];
     __shared__ float st_acc[kAttnWaves][GM][D];  // also the raw qkv rows of the prologue
     __shared__ int last;
@@ -464,9 +867,9 @@ __global__ void __launch_bounds__(64 * NWV) attn_kernel(const void* hrows, const
     // Short contexts run unsplit: the workgroup of split 0 takes every
     // position and writes the output itself; the others leave before any
     // barrier.  Up to about 160 positions that beats a split plus the
-    // cross-workgroup combine (measured on MI355X, 16 q / 4 kv heads of 256:
-    // unsplit 8.5 against 9.7 us at 128 positions, even at 160, split 9.9
-    // against 10.2 us at 192).  The choice follows the device position, so a
+    // cross-workgroup combine (measured on MI355X over bf16 caches, 16 q / 4 kv
+    // heads of 256: unsplit 8.5 against 9.7 us at 128 positions, even at 160,
+    // split 9.9 against 10.2 us at 192).  The choice follows the device position, so a
     // captured graph adapts to it.
     const int nsp = kv_len <= kUnsplitMax ? 1 : a.split;
     if (sp >= nsp) return;
@@ -480,19 +883,11 @@ __global__ void __launch_bounds__(64 * NWV) attn_kernel(const void* hrows, const
     // except the block that holds the new token, which its wave loads after
     // the workgroup has written that token's key and value (the barrier at
     // the end of the prologue orders the workgroup's own stores before its
-    // loads).  Later blocks load after that barrier anyway.  On the buffered
-    // path every wave issues the block's loads, empty (no requests) where the
-    // wave has no block or holds the new token: with the same loads on every
-    // path, the waits for the query rows below count exactly instead of also
-    // waiting for the cache rows behind a branch.  Measured on MI355X (16 q /
-    // 4 kv heads of 256, bf16 cache of 1024, one row): 9.5 -> 8.6 us at 128
-    // positions, 13.6 -> 12.7 us at 1024 over 8 splits; 0.2-0.3 us slower at
-    // 256-512 positions over 8 splits, where most waves issue empty loads.
+    // loads).
     Blk cur;
     int s0 = s_lo + wave * kBlk;
     const bool first_new = has_new && pos >= s0 && pos < s0 + kBlk;
-    const bool first_live = !first_new && s0 < s_hi;
-    if (kv_buffered(DL, F32C) || first_live) load_block<DL, F32C>(a, kv_base, s0, s_hi, mrow, lane, cur, first_live);
+    if (!first_new && s0 < s_hi) load_block<DL, F32C>(a, kv_base, s0, s_hi, mrow, lane, cur);
 
     if constexpr (FUSED) {
         // raw rows: [0, G) query heads, G: key head j, G + 1: value head j;
@@ -579,11 +974,8 @@ __global__ void __launch_bounds__(64 * NWV) attn_kernel(const void* hrows, const
     float acc[GM][DL];  // VALU p v: head h, this lane's DL columns
     for (int h = 0; h < GM; ++h)
         for (int e = 0; e < DL; ++e) acc[h][e] = 0.0f;
-    f32x4_t accm[MV ? NT : 1];  // MV: tile c, lane (col, grp): heads 4 grp + r at column NT col + c
-    for (int c = 0; c < (MV ? NT : 1); ++c) accm[c] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
 
-    // One block: scores on the matrix cores, online softmax, p v on the
-    // matrix cores (MV) or the VALU.
+    // One block: scores on the matrix cores, online softmax, p v on the VALU.
     auto process = [&](Blk& blk, const int s0) __attribute__((always_inline)) {
         const int kpos = s0 + col;
         const bool valid = kpos < s_hi;
@@ -605,44 +997,11 @@ __global__ void __launch_bounds__(64 * NWV) attn_kernel(const void* hrows, const
             m[r] = mn;
             // every head slot of the block is written (rows past G hold
             // finite values of zero query rows and are never output)
-            if (4 * grp + r < GM) {
-                if constexpr (MV)
-                    p_lds[wave][(4 * grp + r) * kBlk + col] = pr;
-                else
-                    p_lds[wave][col * GM + 4 * grp + r] = pr;
-            }
+            if (4 * grp + r < GM) p_lds[wave][col * GM + 4 * grp + r] = pr;
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        if constexpr (MV) {
-            // A: head col's p at positions 4 grp .. 4 grp + 3 (rows from G
-            // on repeat head GM - 1 and are never output), as bf16 hi + lo
-            const float4 pq = *reinterpret_cast<const float4*>(&p_lds[wave][min(col, GM - 1) * kBlk + 4 * grp]);
-            const uint16_t h0 = f32_to_bf16(pq.x), h1 = f32_to_bf16(pq.y), h2 = f32_to_bf16(pq.z),
-                           h3 = f32_to_bf16(pq.w);
-            const u32x2 ah = {(uint32_t)h0 | ((uint32_t)h1 << 16), (uint32_t)h2 | ((uint32_t)h3 << 16)};
-            const u32x2 al = {pack_bf16x2(pq.x - bf16_to_f32(h0), pq.y - bf16_to_f32(h1)),
-                              pack_bf16x2(pq.z - bf16_to_f32(h2), pq.w - bf16_to_f32(h3))};
-            // the accumulator lane (col, grp) holds heads 4 grp + r: its own alphas
-            for (int c = 0; c < NT; ++c)
-                for (int r = 0; r < 4; ++r) accm[c][r] *= alpha[r];
-            for (int c = 0; c < NT; ++c) {
-                // B: column NT col + c of value rows 4 grp .. 4 grp + 3
-                const uint32_t w0 = blk.v[0][c >> 1], w1 = blk.v[1][c >> 1], w2 = blk.v[2][c >> 1],
-                               w3 = blk.v[3][c >> 1];
-                u32x2 bv;
-                if (c & 1) {
-                    bv[0] = (w0 >> 16) | (w1 & 0xFFFF0000u);
-                    bv[1] = (w2 >> 16) | (w3 & 0xFFFF0000u);
-                } else {
-                    bv[0] = (w0 & 0xFFFFu) | (w1 << 16);
-                    bv[1] = (w2 & 0xFFFFu) | (w3 << 16);
-                }
-                accm[c] = mfma16k16(ah, bv, accm[c]);
-                accm[c] = mfma16k16(al, bv, accm[c]);
-            }
-        } else {
         // rescale by head h's alpha (lane 16 (h / 4), element h % 4)
         for (int h = 0; h < GM; ++h) {
             const float al = bcast(alpha[h & 3], 16 * (h >> 2));
@@ -662,28 +1021,14 @@ __global__ void __launch_bounds__(64 * NWV) attn_kernel(const void* hrows, const
             for (int h = 0; h < GM; ++h)
                 for (int e = 0; e < DL; ++e) acc[h][e] += pw[h] * vv[e];
         }
-        }
         // p_lds is rewritten by this wave's next block
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
     };
     constexpr int kStride = kAttnWaves * kBlk;
-    if constexpr (PF) {
-        // two register blocks in turn: the next one loads while this one computes
-        Blk other;
-        for (; s0 < s_hi; s0 += 2 * kStride) {
-            const int s1 = s0 + kStride;
-            if (s1 < s_hi) load_block<DL, F32C>(a, kv_base, s1, s_hi, mrow, lane, other);
-            process(cur, s0);
-            if (s1 >= s_hi) break;
-            if (s1 + kStride < s_hi) load_block<DL, F32C>(a, kv_base, s1 + kStride, s_hi, mrow, lane, cur);
-            process(other, s1);
-        }
-    } else {
-        for (; s0 < s_hi; s0 += kStride) {
-            process(cur, s0);
-            if (s0 + kStride < s_hi) load_block<DL, F32C>(a, kv_base, s0 + kStride, s_hi, mrow, lane, cur);
-        }
+    for (; s0 < s_hi; s0 += kStride) {
+        process(cur, s0);
+        if (s0 + kStride < s_hi) load_block<DL, F32C>(a, kv_base, s0 + kStride, s_hi, mrow, lane, cur);
     }
 
     // Per-wave state to LDS: head 4 grp + r's m and l (l summed over the
@@ -697,135 +1042,36 @@ __global__ void __launch_bounds__(64 * NWV) attn_kernel(const void* hrows, const
             st_l[wave][h] = ls;
         }
     }
-    if constexpr (MV) {
-        for (int r = 0; r < 4; ++r) {
-            const int h = 4 * grp + r;
-            if (h < G)
-                for (int c = 0; c < NT; c += 4)
-                    *reinterpret_cast<float4*>(&st_acc[wave][h][NT * col + c]) =
-                        make_float4(accm[c][r], accm[c + 1][r], accm[c + 2][r], accm[c + 3][r]);
-        }
-    } else {
-        for (int h = 0; h < GM; ++h)
-            if (h < G)
-                for (int e = 0; e < DL; ++e) st_acc[wave][h][DL * lane + e] = acc[h][e];
-    }
+    for (int h = 0; h < GM; ++h)
+        if (h < G)
+            for (int e = 0; e < DL; ++e) st_acc[wave][h][DL * lane + e] = acc[h][e];
     __syncthreads();
 
-    // Merge the waves in a fixed order; write the output or the partial.
-    // Each thread forms its head's wave weights itself (8 values from LDS):
-    // no serial step and no barrier between the state and the merge.
-    const int64_t hq0 = (int64_t)b * a.HQ + (int64_t)j * G;
-    for (int i = tid; i < G * D; i += kAttnThreads) {
-        const int h = i / D, d = i - h * D;
-        float mt = kNegBig;
-        for (int w = 0; w < kAttnWaves; ++w) mt = fmaxf(mt, st_m[w][h]);
-        float lt = 0.0f, at = 0.0f;
-        for (int w = 0; w < kAttnWaves; ++w) {
-            const float f = fexp2((st_m[w][h] - mt) * kLog2e);
-            lt += st_l[w][h] * f;
-            at += st_acc[w][h][d] * f;
-        }
-        if (nsp == 1) {
-            a.out[(int64_t)b * a.ld_out + (int64_t)(j * G + h) * D + d] = f32_to_bf16(lt > 0.0f ? at / lt : 0.0f);
-        } else {  // agent-scope stores: coherent across XCDs without an L2 write-back
-            float* pp = a.part + ((hq0 + h) * a.split + sp) * (D + 4);
-            __hip_atomic_store(&pp[d], at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (d == 0) {
-                __hip_atomic_store(&pp[D], mt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                __hip_atomic_store(&pp[D + 1], lt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
-        }
-    }
-    if (nsp == 1) return;
-
-    // The last workgroup of (b, j) to finish combines the splits.  Every
-    // thread waits until its partial stores have completed (agent-scope
-    // stores complete at the point of coherence) before the workgroup counts
-    // its arrival; the last one reads the partials with agent-scope loads.
-    // No L2 write-back or invalidate is needed for that.
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    if (tid == 0) {
-        const unsigned prev =
-            __hip_atomic_fetch_add(&a.counters[b * a.HKV + j], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        last = prev == (unsigned)a.split - 1u;
-    }
-    __syncthreads();
-    if (!last) return;
-    // Element i = (h, d): each thread loads, for its NE elements, every
-    // split's partial and its head's (m, l) in batches of SB splits (all in
-    // flight at once; SB NE <= 16 keeps them in registers), and merges them
-    // in split order, online: with M the running max, acc and L are rescaled
-    // by exp(M_old - M) and gain w_s acc_s and w_s l_s, w_s = exp(m_s - M).
-    // One memory round trip per batch and no barrier (the weights were first
-    // formed per head in LDS: a second round trip and a barrier).
-    constexpr int NE = (GM * D + kAttnThreads - 1) / kAttnThreads;
-    constexpr int SB = NE <= 2 ? 8 : (NE <= 4 ? 4 : (NE <= 8 ? 2 : 1));
-    float acc0[NE], lsum[NE], mrun[NE];
-    for (int q = 0; q < NE; ++q) {
-        acc0[q] = 0.0f;
-        lsum[q] = 0.0f;
-        mrun[q] = kNegBig;
-    }
-    for (int s0 = 0; s0 < a.split; s0 += SB) {
-        float v[NE][SB], ms[NE][SB], ls[NE][SB];
-        for (int q = 0; q < NE; ++q) {
-            const int i = min(tid + q * kAttnThreads, G * D - 1);
-            const int h = i / D, d = i - h * D;
-            const float* ph = a.part + (hq0 + h) * a.split * (D + 4);
-            for (int u = 0; u < SB; ++u) {
-                const float* pp = ph + min(s0 + u, a.split - 1) * (D + 4);
-                v[q][u] = __hip_atomic_load(pp + d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                ms[q][u] = __hip_atomic_load(pp + D, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                ls[q][u] = __hip_atomic_load(pp + D + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
-        }
-        for (int q = 0; q < NE; ++q) {
-            float mb = mrun[q];
-            for (int u = 0; u < SB; ++u)
-                if (s0 + u < a.split) mb = fmaxf(mb, ms[q][u]);
-            const float rs = fexp2((mrun[q] - mb) * kLog2e);
-            acc0[q] *= rs;
-            lsum[q] *= rs;
-            mrun[q] = mb;
-            for (int u = 0; u < SB; ++u)
-                if (s0 + u < a.split) {
-                    const float w = fexp2((ms[q][u] - mb) * kLog2e);
-                    acc0[q] += v[q][u] * w;
-                    lsum[q] += ls[q][u] * w;
-                }
-        }
-    }
-    for (int q = 0; q < NE; ++q) {
-        const int i = tid + q * kAttnThreads;
-        if (i < G * D) {
-            const int h = i / D, d = i - h * D;
-            const float lt = lsum[q];
-            a.out[(int64_t)b * a.ld_out + (int64_t)(j * G + h) * D + d] =
-                f32_to_bf16(lt > 0.0f ? acc0[q] / lt : 0.0f);
-        }
-    }
-    if (tid == 0) __hip_atomic_store(&a.counters[b * a.HKV + j], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    merge_and_combine<D, GM, kAttnWaves, D>(a, b, j, sp, nsp, kAttnWaves, tid, &st_m[0][0], &st_l[0][0],
+                                            &st_acc[0][0][0], &last);
 }
 
-// Waves per workgroup: 8 for a bf16 cache with D <= 256 and up to 4 query
-// heads per kv head (one 16-position block per wave at a time, no double
-// buffer, so the blocks of a short context run side by side), else 4 (two
-// blocks in turn per wave on the double-buffered path, or the VALU path).
+// Waves per workgroup: attn_bf16 eight (four where 16 heads of 256 columns
+// fill the LDS), attn_kernel four.
 template <int DL, int GM, bool FUSED>
 static void launch_attn(const AttnParams& a, bool f32c, dim3 grid, hipStream_t st) {
     const void* rows = FUSED ? static_cast<const void*>(a.qkv) : static_cast<const void*>(a.q);
     const int ld = (int)a.ld_qkv;  // bz_attn_step: checked to fit 32 bits
-    if (f32c)
+    if (f32c) {
         hipLaunchKernelGGL((attn_kernel<DL, GM, true, FUSED, 4>), grid, dim3(64 * 4), 0, st, rows, a.cosp, a.sinp, a.pos,
                            a.kc, a.vc, ld, a.G, a);
-    else if constexpr (DL <= 4 && GM == 4)
-        hipLaunchKernelGGL((attn_kernel<DL, GM, false, FUSED, 8>), grid, dim3(64 * 8), 0, st, rows, a.cosp, a.sinp, a.pos,
-                           a.kc, a.vc, ld, a.G, a);
-    else
+    } else if constexpr (DL <= 4) {
+        constexpr int NWV = GM == 16 && DL == 4 ? 4 : 8;
+        // G, HKV, whether cos / sin are fp32 and whether one row serves all:
+        // what the first loads need in one preloaded word (grid.y <= 65535)
+        const uint32_t shape =
+            (uint32_t)a.G | (uint32_t)a.HKV << 5 | (a.cs_f32 ? 1u << 21 : 0u) | (a.ld_cs == 0 ? 1u << 22 : 0u);
+        hipLaunchKernelGGL((attn_bf16<DL, GM, FUSED, NWV>), grid, dim3(64 * NWV), 0, st, rows, a.cosp, a.sinp, a.pos,
+                           a.kc, a.vc, ld, shape, a);
+    } else {
         hipLaunchKernelGGL((attn_kernel<DL, GM, false, FUSED, 4>), grid, dim3(64 * 4), 0, st, rows, a.cosp, a.sinp, a.pos,
                            a.kc, a.vc, ld, a.G, a);
+    }
 }
 
 template <bool FUSED>
@@ -873,6 +1119,7 @@ static int attn_setup(AttnParams& a, const void* k_cache, const void* v_cache, i
     a.G = G;
     a.S = S;
     a.split = split;
+    a.split_cap = std::max(1, std::min<int>(split, (int)(256 / ((int64_t)B * HKV))));
     a.part = static_cast<float*>(workspace);
     a.counters = split > 1 ? reinterpret_cast<unsigned*>(a.part + partial_floats(B, HQ, D, split)) : nullptr;
     a.out = static_cast<uint16_t*>(out);

@@ -65,11 +65,13 @@ int bz_qkv_rope_cache(const void* qkv, int64_t ld_qkv, int32_t B, int32_t HQ,
  * ranges; for split > 1 the last workgroup of each (row, kv head) to finish
  * combines the ranges, through `workspace` (bz_attn_workspace bytes, zeroed
  * once before its first use: the kernel leaves its arrival counters at zero
- * again).  While at most 160 positions are attended (decided on the device
- * from *pos) the call runs unsplit whatever `split` says: the workgroup of
- * split 0 covers every position and writes the output, the others return at
- * once and the workspace is not touched.  Calls that share a workspace must
- * not overlap.  Replaces
+ * again).  While few positions are attended (decided on the device from
+ * *pos: up to 256, for D = 256 up to 224, and 160 over an fp32 cache or D =
+ * 512) the call runs unsplit whatever `split` says: the workgroup of split 0
+ * covers every position and writes the output, the others return at once and
+ * the workspace is not touched.  Over a bf16 cache with D <= 256 a longer call
+ * uses no more splits than have 128 positions or than fill the CUs.  Calls
+ * that share a workspace must not overlap.  Replaces
  * attn_decode_kernel + attn_combine_kernel, models/fused/kernels.py:404-475
  * (attention_step :528-536 picks split 1 for S <= 256, else 8;
  * bz_attn_default_split is this build's choice).

@@ -287,3 +287,33 @@ def test_attention_step_graph_replays_track_device_position():
         torch.cuda.synchronize()
         np.testing.assert_array_equal(f32(out), f32(ref))
         np.testing.assert_array_equal(f32(kc), f32(kc2))
+
+
+@pytest.mark.parametrize("HQ,HKV,D", [(16, 4, 256), (16, 8, 128), (16, 1, 64), (48, 3, 256)])
+@pytest.mark.parametrize("B,pos", [(1, 223), (1, 224), (1, 255), (1, 256), (2, 300), (24, 500)])
+def test_attention_step_split_rule(HQ, HKV, D, B, pos):
+    """The bf16 kernel around the positions where it starts to split (224 for D
+    = 256, else 256), over rows and kv heads that leave it few splits, with a
+    cache that holds NaN past the position: equal to one split, and to the
+    oracle; the mask in each element type, at an odd offset in its buffer."""
+    S, split = 512, 4
+    qkv, keys, values = _case(B, HQ, HKV, D, S, 40 + pos, fill=pos)
+    cos, sin = (O.round_bf16(t) for t in _rope_tables(B, D, 41))
+    allow = np.random.default_rng(42).random((B, S)) > 0.1
+    allow[:, pos] = True
+    madd = np.where(allow, 0.0, float(torch.finfo(torch.bfloat16).min)).astype(np.float32)
+    outs = []
+    for kind, sp in (("bf16", split), ("f32", split), ("bool", split), ("bf16", 1)):
+        flat = torch.from_numpy(allow if kind == "bool" else madd)
+        wide = torch.zeros(B, S + 3, dtype={"bf16": torch.bfloat16, "f32": torch.float32, "bool": torch.bool}[kind])
+        wide[:, 3:] = flat
+        kc, vc = _bf16(keys), _bf16(values)
+        kc[:, :, pos + 1:], vc[:, :, pos + 1:] = float("nan"), float("nan")
+        out = T.attention_step(_bf16(qkv), _bf16(cos), _bf16(sin), torch.tensor([pos], device=DEV), kc, vc,
+                               wide.to(DEV)[:, 3:].view(B, 1, 1, S), None, None, 1e-6, split=sp)
+        assert torch.isfinite(out).all()
+        outs.append(f32(out))
+    assert np.array_equal(outs[0], outs[1])
+    assert O.rel_err(outs[0], outs[3]) <= TIGHT and O.rel_err(outs[2], outs[3]) <= TIGHT
+    q_ref = A.qkv_rope_cache(qkv, HQ, HKV, D, cos, sin, pos, keys, values)
+    assert O.rel_err(outs[0], A.attn_decode(q_ref, keys, values, madd, pos)) <= TIGHT
