@@ -48,7 +48,7 @@ HIP_FLAGS = [
 # instances with D <= 256 (attn_kernel<DL = 1, 2, 4, GM, F32C = false, ...>)
 # are covered, its fp32-cache and D = 512 instances are allowed scratch.
 NO_SCRATCH = (r"gemv_persist", r"gemv_mfma", r"gemv_i8mma", r"gemv_tile", r"gemv_stream", r"gemv_wide", r"gemv_panel",
-              r"gemm_tiled", r"gemv_rows",
+              r"gemm_tiled", r"gemv_rows", r"gemv_slab",
               r"head_f32", r"qkv_rope_cache",
               r"attn_kernelILi[124]ELi\d+ELb0E", r"attn_bf16")
 

@@ -9,6 +9,7 @@
 
 #include "bz_gemv_panel.h"
 #include "bz_gemv_rows.h"
+#include "bz_gemv_slab.h"
 #include "bz_gemv_tile.h"
 #include "bz_gemv_wide.h"
 
@@ -357,13 +358,39 @@ static int wide_rule(const bz_gemv_desc* d, int rows) {
 // kernel and cfg_tiles >= 1 the several-block kernel with that many blocks
 // per workgroup (cfg_waves waves, 0 = the kernel's own rule, either way).
 struct TiledPlan {
-    bool wide;
+    bool wide, slab;
     StreamLaunch s;
     WideLaunch w;
+    SlabLaunch b;
 };
+
+// Launch shape of the few-row-block fp8 kernel (bz_gemv_slab.h) for `rows`
+// rows of x, or false where another kernel is the better one: about one
+// workgroup per CU, 4, 8 or 16 rows of a block each.  A lane's x is loaded
+// again by every workgroup and row group, so it loses with more rows of x or
+// more blocks (measured on MI355X, the other kernels' time first, us): M = 2
+// N2560 K4096 4.20 / 4.48, N2560 K10240 6.89 / 7.94; M = 4 N1024 K8192 5.43 /
+// 5.39, N2048 K2048 3.67 / 3.58, N2048 K6144 5.06 / 5.50, but N1024 K1024 3.50
+// / 2.84 and N1024 K2048 3.56 / 3.15; M = 1 N4096 K2560 4.03 / 3.81.
+static bool slab_plan(const bz_gemv_desc* d, int rows, SlabLaunch& l) {
+    if (d->cfg_path || d->wfmt != BZ_W_FP8_TILED || d->gamma || d->n_out2) return false;
+    const int NU = tiled_units(d->wfmt, d->K), nblk = d->N / 16;
+    if (nblk > (rows == 1 ? 256 : rows == 2 ? 128 : rows <= 4 && d->K <= 2048 ? 64 : 0)) return false;
+    // (one short row of x: N1024 K1024 8 rows 2.38 us, 4 rows 2.52)
+    l.rl = nblk <= 64 && (rows > 1 || d->K > 2048) ? 1 : nblk <= 128 ? 2 : 4;
+    const int groups = (NU + 3) / 4;
+    l.ni = (groups + kStreamMaxWaves - 1) / kStreamMaxWaves;
+    if (l.ni > kSlabMaxNi || NU > kStreamMaxWaves * 10) return false;  // the longest rows of the streaming kernels
+    l.m = rows <= 2 ? rows : 4;
+    l.nw = std::max((groups + l.ni - 1) / l.ni, l.rl * l.m);  // a group of 16 lanes per output
+    l.grid = (unsigned)(nblk * (4 / l.rl));
+    return true;
+}
 
 static int tiled_plan(const bz_gemv_desc* d, int rows, TiledPlan& pl) {
     int T;
+    pl.slab = slab_plan(d, rows, pl.b);
+    if (pl.slab) return BZ_OK;
     if (d->cfg_path == PATH_STREAM) {
         if (d->cfg_tiles < 0 || d->cfg_tiles > kWideMaxBlocks) return BZ_ERR_INVALID_ARG;
         T = d->cfg_tiles;
@@ -415,7 +442,7 @@ static int gemv_tiled(const bz_gemv_desc* d, const DescInfo& di, hipStream_t st)
         p.out = static_cast<uint8_t*>(d->out) + (int64_t)m0 * d->ldo * osz;
         p.out2 = d->n_out2 ? static_cast<uint8_t*>(d->out2) + (int64_t)m0 * d->ldo2 * osz : nullptr;
         p.res = d->residual ? static_cast<const uint8_t*>(d->residual) + (int64_t)m0 * d->ldr * rsz : nullptr;
-        const int lrc = q.wide ? launch_wide(d->wfmt, p, q.w, d->N / 16, st) : launch_stream(d->wfmt, p, q.s, st);
+        const int lrc = q.slab ? launch_slab(p, q.b, st) : q.wide ? launch_wide(d->wfmt, p, q.w, d->N / 16, st) : launch_stream(d->wfmt, p, q.s, st);
         if (lrc != BZ_OK) return lrc;
     }
     return BZ_OK;

@@ -659,3 +659,28 @@ def test_gemv_wide_rejects_bad_block_counts():
     x = bf16_tensor(_x(1, k, 741))
     with pytest.raises(RuntimeError, match="status 1"):
         G.gemv(x, buf, tf, n, cfg=(0, 0, 9, 5))
+
+
+@pytest.mark.parametrize("n,k", [(16, 64), (1024, 192), (1024, 2048), (1024, 2112), (1040, 1024), (2048, 4160), (2064, 576),
+                                 (4096, 128), (96, 10240)])
+@pytest.mark.parametrize("m", [1, 2, 3, 4])
+def test_few_block_fp8_rule(n, k, m):
+    """The rule's launch around the edges of the few-row-block kernel (64, 128
+    and 256 blocks; odd units; one and several unit groups per wave; K where 3
+    and 4 rows leave it): fp32 outputs, whose only error is the order of the
+    fp32 sums (K 2^-23 of the sum of magnitudes), with no residual and with one
+    of either type, x inside a wider buffer of NaN."""
+    c = _fp8_case(n, k, n + k)
+    buf, fmt = _tiled_f8(c, False)
+    xb = O.f32_to_bf16_bits(_rng(m).standard_normal((m, k)).astype(np.float32))
+    wide = torch.full((m, k + 64), float("nan"), device="cuda", dtype=torch.bfloat16)
+    wide[:, :k] = bf16_tensor(xb)
+    x = O.bf16_bits_to_f32(xb).astype(np.float64)
+    w = c.w_eff.astype(np.float64)
+    ref, mag = x @ w.T, np.abs(x) @ np.abs(w).T
+    for res_dt in (None, torch.bfloat16, torch.float32):
+        res = None if res_dt is None else torch.randn(m, n + 3, device="cuda").to(res_dt)[:, 3:]
+        got = f32(G.gemv(wide[:, :k], buf, fmt, n, epilogue=G.EPI_NONE if res is None else G.EPI_RESIDUAL, residual=res,
+                         out_dtype=torch.float32))
+        want = ref if res is None else ref + f32(res)
+        assert np.all(np.abs(got - want) <= k * 2.0 ** -23 * mag + 2.0 ** -22 * np.abs(want) + 1e-30), (res_dt,)
