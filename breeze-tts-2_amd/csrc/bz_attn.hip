@@ -137,17 +137,25 @@ __global__ void __launch_bounds__(kRopeThreads) qkv_rope_cache_kernel(
     const void* cosp, const void* sinp, bool cs_f32, int64_t ld_cs, const int64_t* pos_p, float* q_out, void* kc,
     void* vc, int S, bool cache_f32, int64_t* seq_len) {
     __shared__ float vals[kMaxRopeDim];
+    __shared__ float part[kRopeThreads / 64];
     const int b = blockIdx.x, h = blockIdx.y;
     const bool is_q = h < HQ;
     const uint16_t* src = qkv + (int64_t)b * ld_qkv + (int64_t)h * D;
     const uint16_t* nw = is_q ? qn : kn;
-    for (int d = threadIdx.x; d < D; d += kRopeThreads) vals[d] = bf16_to_f32(src[d]);
+    float ss = 0.0f;
+    for (int d = threadIdx.x; d < D; d += kRopeThreads) {
+        const float v = bf16_to_f32(src[d]);
+        vals[d] = v;
+        ss += v * v;
+    }
+    ss = wave_sum64(ss);
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = ss;
     __syncthreads();
     float inv = 1.0f;
-    if (nw) {  // every wave, in the order of attn_bf16: columns l + 64 e of a lane, then the lanes
-        float ss = 0.0f;
-        for (int d = threadIdx.x & 63; d < D; d += 64) ss = fmaf(vals[d], vals[d], ss);
-        inv = 1.0f / sqrtf(wave_sum64(ss) / (float)D + eps);
+    if (nw) {
+        float t = 0.0f;
+        for (int w = 0; w < kRopeThreads / 64; ++w) t += part[w];
+        inv = 1.0f / sqrtf(t / (float)D + eps);
     }
     const int half = D >> 1;
     const int64_t cs = (int64_t)b * ld_cs;
@@ -458,9 +466,12 @@ __device__ __forceinline__ void merge_and_combine(const AttnParams& a, int b, in
 //     at its end.
 // Measured on MI355X (cold caches, graph replays, default split) against the
 // kernel with four prologue barriers, scores not transposed and p through
-// LDS: 8 / 2 heads of 128, B = 2, 17 positions 5.25 -> 4.11 us; 16 / 8 heads of
-// 128, B = 2, 612 of 1024 positions 8.61 -> 7.59; 16 / 4 heads of 256, B = 2,
-// 128 positions 8.87 -> 7.82, 1902 of 2048 13.9 -> 12.8.
+// LDS: 8 / 2 heads of 128, B = 2, 17 positions 5.25 -> 4.25 us; 16 / 8 heads of
+// 128, B = 2, 612 of 1024 positions 8.55 -> 7.68; 16 / 4 heads of 256, B = 2,
+// 128 positions 8.71 -> 7.77, 1902 of 2048 13.96 -> 12.94.  Every sum keeps that
+// kernel's order (norm: 64 columns over the lanes, then in column order; scores:
+// hi and lo in one chain; l: 16 positions as sum16 adds them), so an unsplit
+// step gives the same bits: tokens are picked from what it feeds.
 // ---------------------------------------------------------------------------
 template <int DL>
 struct KvRows {
@@ -477,6 +488,17 @@ __device__ __forceinline__ float across_rows(float v, F f) {
     const float t = f(__uint_as_float(a[0]), __uint_as_float(a[1]));
     const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(t), __float_as_uint(t), false, false);
     return f(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+
+// The four rows' values of a column, in every lane of it.
+__device__ __forceinline__ void all_rows(float v, float (&o)[4]) {
+    const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    const auto lo = __builtin_amdgcn_permlane16_swap(a[0], a[0], false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap(a[1], a[1], false, false);
+    o[0] = __uint_as_float(lo[0]);
+    o[1] = __uint_as_float(lo[1]);
+    o[2] = __uint_as_float(hi[0]);
+    o[3] = __uint_as_float(hi[1]);
 }
 
 template <int DL, int GM, bool FUSED, int NWV>
@@ -584,10 +606,10 @@ __global__ void __launch_bounds__(64 * NWV) attn_bf16(const void* hrows, const v
     // follows it): none while two blocks per wave cover the positions, else
     // as many as have a block for every wave, and no more workgroups than
     // CUs; the others leave before any barrier.  Measured on MI355X, unsplit
-    // against 8 splits: D = 128 (16 / 8 heads, B = 2) 6.56 / 7.02 us at 256
-    // positions, 7.59 / 7.03 at 331; D = 256 (16 / 4 heads, B = 1) 8.69 / 8.78
-    // at 160, 10.35 / 10.01 at 256.  64 (row, kv head) pairs at 2001 positions:
-    // 4 splits 16.6 us, 5 21.8, 8 19.5, 16 25.8.
+    // against 8 splits: D = 128 (16 / 8 heads, B = 2) 7.54 / 7.09 us at 331
+    // positions (6.56 / 7.02 at 256 when both could be forced); D = 256 (16 / 4
+    // heads, B = 1) 8.69 / 8.78 at 160, 10.63 / 10.22 at 256.  64 (row, kv head)
+    // pairs at 2001 positions: 4 splits 16.5 us, 5 21.8, 8 19.5, 16 25.8.
     constexpr int kUnsplit = DL == 4 ? 224 : 256;
     const int nsp =
         kv_len <= kUnsplit ? 1 : min(a.split_cap, (nblk + NWV - 1) / NWV);
@@ -621,14 +643,14 @@ __global__ void __launch_bounds__(64 * NWV) attn_bf16(const void* hrows, const v
                 }
                 continue;
             }
-            float ss = 0.0f;
+            float ss = 0.0f;  // each 64 columns over the lanes, then in column order
 #pragma unroll
             for (int e = 0; e < DL; ++e) {
                 v[e] = __uint_as_float(raw[i][e] << 16);
-                ss = fmaf(v[e], v[e], ss);
+                ss += wave_sum64(v[e] * v[e]);
             }
             if (a.qn) {
-                const float inv = 1.0f / sqrtf(wave_sum64(ss) / (float)D + a.eps);
+                const float inv = 1.0f / sqrtf(ss / (float)D + a.eps);
 #pragma unroll
                 for (int e = 0; e < DL; ++e) v[e] = v[e] * inv * __uint_as_float(nw[i][e] << 16);
             }
@@ -681,9 +703,9 @@ __global__ void __launch_bounds__(64 * NWV) attn_bf16(const void* hrows, const v
 
     // 4. the wave's blocks: lane (col, grp) holds head col's scores at
     //    positions 4 grp + r; m is the head's running max (the same in its
-    //    four lanes), l this lane's share of the sum, acc[c][r] the head's
+    //    four lanes), l[r] the sum of its position's weights, acc[c][r] the head's
     //    output at column v_col(c, 4 grp + r)
-    float m = kNegBig, l = 0.0f;
+    float m = kNegBig, l[4] = {0.0f, 0.0f, 0.0f, 0.0f};
     f32x4_t acc[NT];
 #pragma unroll
     for (int c = 0; c < NT; ++c) acc[c] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
@@ -696,27 +718,28 @@ __global__ void __launch_bounds__(64 * NWV) attn_bf16(const void* hrows, const v
 #pragma unroll
             for (int t = 0; t < T; ++t) kn[t] = *reinterpret_cast<const u32x4*>(&knew[32 * t + 8 * grp]);
 #pragma unroll
-            for (int i = 0; i < 2 * DL; ++i) vn[i] = *reinterpret_cast<const uint32_t*>(&vnew[v_col(2 * i, col)]);
-#pragma unroll
             for (int t = 0; t < T; ++t)
 #pragma unroll
                 for (int q = 0; q < 4; ++q) cur.k[t][q] = col == at ? kn[t][q] : cur.k[t][q];
+            if constexpr (DL == 4) __builtin_amdgcn_sched_barrier(0);  // the registers of both do not fit at once
+#pragma unroll
+            for (int i = 0; i < 2 * DL; ++i) vn[i] = *reinterpret_cast<const uint32_t*>(&vnew[v_col(2 * i, col)]);
 #pragma unroll
             for (int r = 0; r < 4; ++r)
 #pragma unroll
                 for (int i = 0; i < 2 * DL; ++i) cur.v[r][i] = 4 * grp + r == at ? vn[i] : cur.v[r][i];
         }
-        f32x4_t sc = {0.0f, 0.0f, 0.0f, 0.0f}, sl = {0.0f, 0.0f, 0.0f, 0.0f};
+        f32x4_t sc = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int t = 0; t < T; ++t) {
             sc = mfma16(cur.k[t], qop[t][0][lane], sc);
-            sl = mfma16(cur.k[t], qop[t][1][lane], sl);
+            sc = mfma16(cur.k[t], qop[t][1][lane], sc);
         }
         float s[4], bm = kNegBig;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const bool valid = s0 + 4 * grp + r < kv_len;
-            s[r] = valid ? sc[r] + sl[r] + word_f32(cur.mraw[r], a.mask_dtype) : kNegBig;
+            s[r] = valid ? sc[r] + word_f32(cur.mraw[r], a.mask_dtype) : kNegBig;
             bm = fmaxf(bm, s[r]);
             // (a value row past the range may hold anything)
 #pragma unroll
@@ -725,13 +748,12 @@ __global__ void __launch_bounds__(64 * NWV) attn_bf16(const void* hrows, const v
         const float mn = fmaxf(m, across_rows(bm, [](float x, float y) { return fmaxf(x, y); }));
         const float alpha = fexp2((m - mn) * kLog2e);
         m = mn;
-        float p[4], ps = 0.0f;
+        float p[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             p[r] = s0 + 4 * grp + r < kv_len ? fexp2((s[r] - mn) * kLog2e) : 0.0f;
-            ps += p[r];
+            l[r] = l[r] * alpha + p[r];
         }
-        l = l * alpha + ps;
         const uint32_t h01 = pack_bf16x2(p[0], p[1]), h23 = pack_bf16x2(p[2], p[3]);
         const u32x2 ph = {h01, h23};
         const u32x2 pl = {pack_bf16x2(p[0] - bf16_lo(h01), p[1] - bf16_hi(h01)),
@@ -760,11 +782,12 @@ __global__ void __launch_bounds__(64 * NWV) attn_bf16(const void* hrows, const v
     //    positions has none
     const int nact = min(NWV, nblk - sp * NWV);  // <= 0 only without any position
     if (any) {
-        l = across_rows(l, [](float x, float y) { return x + y; });
+        float ql[4];
+        all_rows((l[0] + l[1]) + (l[2] + l[3]), ql);
         if (col < G) {
             if (grp == 0) {
                 st_m[wave][col] = m;
-                st_l[wave][col] = l;
+                st_l[wave][col] = (ql[0] + ql[3]) + (ql[2] + ql[1]);  // the order of sum16
             }
 #pragma unroll
             for (int r = 0; r < 4; ++r)
