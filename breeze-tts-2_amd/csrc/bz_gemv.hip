@@ -364,33 +364,28 @@ struct TiledPlan {
     SlabLaunch b;
 };
 
-// Launch shape of the few-row-block fp8 kernel (bz_gemv_slab.h) for `rows`
-// rows of x, or false where another kernel is the better one: about one
-// workgroup per CU, 4, 8 or 16 rows of a block each.  A lane's x is loaded
-// again by every workgroup and row group, so it loses with more rows of x or
-// more blocks (measured on MI355X, the other kernels' time first, us): M = 2
-// N2560 K4096 4.20 / 4.48, N2560 K10240 6.89 / 7.94; M = 4 N1024 K8192 5.43 /
-// 5.39, N2048 K2048 3.67 / 3.58, N2048 K6144 5.06 / 5.50, but N1024 K1024 3.50
-// / 2.84 and N1024 K2048 3.56 / 3.15; M = 1 N4096 K2560 4.03 / 3.81.
-static bool slab_plan(const bz_gemv_desc* d, int rows, SlabLaunch& l) {
+// Whether the few-row-block fp8 kernel (bz_gemv_slab.h) takes the place of a
+// streaming plan of one block per workgroup, and its launch shape: 4 workgroups
+// per block, so while the blocks alone do not occupy the CUs.  Every workgroup
+// loads x again, so 3 and 4 rows of it over more than 64 blocks lose: N2048
+// K6144 5.00 us on the kernel below, 5.92 on this one; N1536 K1024 3.53 / 4.02;
+// N1024 K8192 5.40 / 4.42.
+static bool slab_plan(const bz_gemv_desc* d, int rows, TiledPlan& pl) {
     if (d->cfg_path || d->wfmt != BZ_W_FP8_TILED || d->gamma || d->n_out2) return false;
-    const int NU = tiled_units(d->wfmt, d->K), nblk = d->N / 16;
-    if (nblk > (rows == 1 ? 256 : rows == 2 ? 128 : rows <= 4 && d->K <= 2048 ? 64 : 0)) return false;
-    // (one short row of x: N1024 K1024 8 rows 2.38 us, 4 rows 2.52)
-    l.rl = nblk <= 64 && (rows > 1 || d->K > 2048) ? 1 : nblk <= 128 ? 2 : 4;
-    const int groups = (NU + 3) / 4;
-    l.ni = (groups + kStreamMaxWaves - 1) / kStreamMaxWaves;
-    if (l.ni > kSlabMaxNi || NU > kStreamMaxWaves * 10) return false;  // the longest rows of the streaming kernels
-    l.m = rows <= 2 ? rows : 4;
-    l.nw = std::max((groups + l.ni - 1) / l.ni, l.rl * l.m);  // a group of 16 lanes per output
-    l.grid = (unsigned)(nblk * (4 / l.rl));
+    const int nblk = d->N / 16;
+    if (nblk > (rows <= 2 ? kSlabMaxBlocks : rows <= kSlabMaxM ? 64 : 0)) return false;
+    pl.b.chain = pl.wide;
+    pl.b.nv = pl.wide ? pl.w.nw : pl.s.nw;
+    pl.b.upw = pl.wide ? pl.w.upw : pl.s.upw;
+    // 4 parts per wave; a group of 16 lanes per output
+    pl.b.threads = 64u * (unsigned)std::max((pl.b.nv + 3) / 4, rows);
+    pl.b.grid = (unsigned)(nblk * (16 / kSlabRows));
     return true;
 }
 
 static int tiled_plan(const bz_gemv_desc* d, int rows, TiledPlan& pl) {
     int T;
-    pl.slab = slab_plan(d, rows, pl.b);
-    if (pl.slab) return BZ_OK;
+    pl.slab = false;
     if (d->cfg_path == PATH_STREAM) {
         if (d->cfg_tiles < 0 || d->cfg_tiles > kWideMaxBlocks) return BZ_ERR_INVALID_ARG;
         T = d->cfg_tiles;
@@ -401,7 +396,9 @@ static int tiled_plan(const bz_gemv_desc* d, int rows, TiledPlan& pl) {
         if (T && wide_plan(d, rows, T, pl.w) == BZ_ERR_UNSUPPORTED && pl.w.upw == 0) T = 0;
     }
     pl.wide = T > 0;
-    return pl.wide ? wide_plan(d, rows, T, pl.w) : stream_plan(d, rows, pl.s);
+    const int rc = pl.wide ? wide_plan(d, rows, T, pl.w) : stream_plan(d, rows, pl.s);
+    if (rc == BZ_OK) pl.slab = slab_plan(d, rows, pl);
+    return rc;
 }
 
 // The tiled formats: up to kStreamMaxRows rows per launch (fewer when their

@@ -1,120 +1,116 @@
 // Decode GEMV over an unpaired fp8 tiled weight with few row blocks: a
-// workgroup takes only 4, 8 or 16 rows of a 16-row block, so that a projection
-// to a narrow hidden size (N = 1024: 64 blocks) still occupies every CU.
+// workgroup takes only 4 rows of a 16-row block, so that a projection to a
+// narrow hidden size (N = 1024: 64 blocks) still occupies every CU.
 //
 // Replaces rms_gemv_kernel + gemv_epilogue_kernel without the norm prologue
 // (models/fused/kernels.py:41-138): the down and output projections.
 //
 // Work decomposition
-//   * One wave instruction reads 4 rows x 64 bytes of 4 consecutive tiles: lane
-//     l holds 16 codes of row (l / 4) % 4 of its group, unit l / 16, piece l % 4
-//     (16 lanes read 256 contiguous bytes).  RL of them, 4 rows apart, share
-//     the lane's x.
-//   * The x a lane needs (16 values per unit and row of x) goes from L2 into
-//     its registers; there is no LDS staging.  x first, then the weights, all
-//     loads of a wave in flight at once.
-//   * gfx950's exact e4m3 -> bf16 conversion, then v_dot2_f32_bf16; the lanes of
-//     a row meet by DPP and lane-row swaps, the waves (split over K) in LDS
-//     behind the only barrier.
+//   * The K split is that of the one- or several-block kernel it stands in for
+//     (NV waves of UPW consecutive units, one accumulator chain each, their
+//     sums met in the same order), and so are the MFMAs a chain consists of:
+//     the result is the same, bit for bit.  A token picked from it does not
+//     depend on which kernel ran.
+//   * v_mfma_f32_16x16x32_bf16 has room for 16 columns and 16 rows of x, the 4
+//     weight rows and up to 4 rows of x need a quarter of each.  So one wave
+//     runs the chains of 4 split-K parts side by side: column 4 c + row holds
+//     the weight rows' codes of part c, row 4 m + c of A the x row m over part
+//     c's units, and the products of unlike parts are dropped.  Each lane then
+//     loads 16 bytes of weights per unit, 256 contiguous bytes per part.
+//   * x goes from L2 into the registers of the A operand: no LDS staging.  x
+//     first, then the weights, all loads of a wave in flight at once; the one
+//     barrier is before the epilogue.
 //   * Bound by HBM latency at these sizes.  Measured on MI355X with a residual
-//     (graph replays over >= 1 GiB of weight copies; floor = 1.67 us + bytes at
-//     7.39 TB/s), the one- or several-block kernel -> this one: N1024 K8192
-//     (floor 2.81) M = 1 4.98 -> 3.62 us, M = 2 5.13 -> 4.26; N1024 K1024
-//     (1.81) 2.67 -> 2.38, 2.75 -> 2.61; N2048 K6144 (3.37) 5.10 -> 4.25, 4.75
-//     -> 4.52; N2560 K10240 (5.22) M = 1 7.14 -> 6.73.
+//     (graph replays over 1 GiB of weight copies; floor = 1.67 us + bytes at
+//     7.39 TB/s), the kernel it stands in for -> this one, M = 1, 2, 4: N1024
+//     K8192 (floor 2.81) 4.99 -> 3.92, 5.10 -> 4.01, 5.40 -> 4.42; N1024 K1024
+//     (1.81) 2.66 -> 2.44, 2.75 -> 2.46, 3.00 -> 3.00; N2048 K2048 (2.24) 3.29 ->
+//     3.06, 3.44 -> 3.13; N2048 K6144 (3.37) 5.05 -> 4.76, 4.73 -> 4.63.
 #pragma once
 
 #include "bz_gemv_stream.h"
 
 namespace bz {
 
-constexpr int kSlabMaxNi = 3;  // groups of 4 units per wave (16 waves: K <= 12288)
+constexpr int kSlabRows = 4;      // weight rows per workgroup = split-K parts per wave
+constexpr int kSlabMaxM = 4;      // rows of x
+constexpr int kSlabMaxBlocks = 128;
 
 struct SlabLaunch {
-    int m, rl, ni, nw;
-    unsigned grid;
+    int nv, upw;  // split-K parts and units per part, of the plan it stands in for
+    int chain;    // 1: that plan adds its parts one after the other, 0: by a tree
+    unsigned threads, grid;
 };
 
-// Sum over the four 16-lane rows of a wave, in every lane.
-__device__ __forceinline__ float rows4_sum(float v) {
-    const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    const float t = __uint_as_float(a[0]) + __uint_as_float(a[1]);
-    const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(t), __float_as_uint(t), false, false);
-    return __uint_as_float(b[0]) + __uint_as_float(b[1]);
-}
-
-template <int M, int RL, int NI>
-__global__ void __launch_bounds__(1024) gemv_slab(const uint8_t* hw, const uint16_t* hx, int hchunk, int hldx, int hK,
-                                                  int hNU, int hM, StreamParams p) {
-    __shared__ float red[4 * RL * M][16];  // [row][x row] by wave
-    constexpr int RQ = 4 * RL, PB = 16 / RQ;  // rows per workgroup, workgroups per block
-    const int tid = threadIdx.x, lane = tid & 63, NW = blockDim.x >> 6;
+template <int UPW>
+__global__ void __launch_bounds__(256) gemv_slab(const uint8_t* hw, const uint16_t* hx, int hchunk, int hldx, int hNU,
+                                                 int hM, int hnv, int hchain, StreamParams p) {
+    __shared__ __attribute__((aligned(16))) float red[kSlabMaxM * kSlabRows][16];  // [x row, weight row][part]
+    const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int blk = (int)blockIdx.x / PB, r0 = ((int)blockIdx.x % PB) * RQ;
-    const int u0 = wave * NI * 4 + (lane >> 4), rr = (lane >> 2) & 3, piece = lane & 3;
+    const int blk = (int)blockIdx.x >> 2, r0 = ((int)blockIdx.x & 3) * kSlabRows;
+    const int j = lane & 15, kq = lane >> 4;
     const uint8_t* chunk = hw + (int64_t)blk * hchunk;
+    // column j of B: weight row j % 4 over the units of part j / 4; row j of
+    // A: x row j / 4 over the units of part j % 4
+    const int ub = (wave * 4 + (j >> 2)) * UPW, ua = (wave * 4 + (j & 3)) * UPW, xm = j >> 2;
 
-    const __amdgpu_buffer_rsrc_t xrs = buffer_rsrc(hx, (uint32_t)(((int64_t)(hM - 1) * hldx + hK) * 2));
+    const __amdgpu_buffer_rsrc_t xrs =
+        buffer_rsrc(hx, (uint32_t)(((int64_t)(hM - 1) * hldx + (int64_t)hNU * 64) * 2));
     const __amdgpu_buffer_rsrc_t wrs = buffer_rsrc(chunk, (uint32_t)hNU * 1024u);
-    u32x4 xv[NI][M][2], wv[NI][RL];
+    // a unit past the row and a row of x past the call's read as zeros without
+    // a request, and add 0
+    u32x4 xv[UPW][2], wv[UPW];
 #pragma unroll
-    for (int i = 0; i < NI; ++i)
-#pragma unroll
-        for (int m = 0; m < M; ++m) {
-            const int u = u0 + 4 * i;
-            const uint32_t o =
-                u < hNU && m < hM ? (uint32_t)(((int64_t)m * hldx + u * 64 + piece * 16) * 2) : kBufferOob;
-            xv[i][m][0] = buffer_ld16(xrs, o);
-            xv[i][m][1] = buffer_ld16(xrs, o == kBufferOob ? o : o + 16);
-        }
+    for (int q = 0; q < UPW; ++q) {
+        const uint32_t o = xm < hM && ua + q < hNU
+                               ? (uint32_t)(((int64_t)xm * hldx + (ua + q) * 64 + kq * 16) * 2)
+                               : kBufferOob;
+        xv[q][0] = buffer_ld16(xrs, o);
+        xv[q][1] = buffer_ld16(xrs, o == kBufferOob ? o : o + 16);
+    }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int i = 0; i < NI; ++i)
-#pragma unroll
-        for (int t = 0; t < RL; ++t)
-            wv[i][t] = buffer_ld16_nt(wrs, (uint32_t)(u0 + 4 * i) * 1024u + (r0 + 4 * t + rr) * 64 + piece * 16);
+    for (int q = 0; q < UPW; ++q)
+        wv[q] = buffer_ld16_nt(wrs, (uint32_t)(ub + q) * 1024u + (r0 + (j & 3)) * 64 + kq * 16);
     __builtin_amdgcn_sched_barrier(0);
-    // output g = (row, x row) belongs to the 16 lanes of group g: its row
-    // scale and residual
-    constexpr int kOut = RQ * M;
-    const int g = min(tid >> 4, kOut - 1), gw = tid & 15;
-    const int orow = r0 + g / M, om = g % M;
+    // output g = (x row, weight row) belongs to the 16 lanes of group g: its
+    // row scale and residual
+    const int g = min(tid >> 4, hM * kSlabRows - 1), gw = tid & 15;
+    const int om = g / kSlabRows, orow = r0 + g % kSlabRows;
     const float rs = reinterpret_cast<const float*>(chunk + (int64_t)hNU * 1024)[orow];
-    const int log2 = p.res_f32 ? 2 : 1;
-    const int64_t ri = (int64_t)min(om, hM - 1) * p.ldr + blk * 16 + orow;
     RawWord resv = {0u, 0u};
-    if (p.epi == BZ_EPI_RESIDUAL) resv = ld_elem(p.res, log2, ri);
+    if (p.epi == BZ_EPI_RESIDUAL) resv = ld_elem(p.res, p.res_f32 ? 2 : 1, (int64_t)om * p.ldr + blk * 16 + orow);
     __builtin_amdgcn_sched_barrier(0);
 
-    float acc[RL][M];
+    f32x4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int t = 0; t < RL; ++t)
-#pragma unroll
-        for (int m = 0; m < M; ++m) acc[t][m] = 0.0f;
-#pragma unroll
-    for (int i = 0; i < NI; ++i)
-#pragma unroll
-        for (int t = 0; t < RL; ++t)
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const uint32_t lo = fp8x2_bf16<false>(wv[i][t][q]), hi = fp8x2_bf16<true>(wv[i][t][q]);
-#pragma unroll
-                for (int m = 0; m < M; ++m) {
-                    acc[t][m] = dot2(lo, xv[i][m][q >> 1][2 * (q & 1)], acc[t][m]);
-                    acc[t][m] = dot2(hi, xv[i][m][q >> 1][2 * (q & 1) + 1], acc[t][m]);
-                }
-            }
-#pragma unroll
-    for (int t = 0; t < RL; ++t)
-#pragma unroll
-        for (int m = 0; m < M; ++m) {
-            const float v = rows4_sum(sum4(acc[t][m]));
-            if (lane < 16 && piece == 0) red[(4 * t + rr) * M + m][wave] = v;
-        }
+    for (int q = 0; q < UPW; ++q) {
+        const u32x4 b0 = {fp8x2_bf16<false>(wv[q][0]), fp8x2_bf16<true>(wv[q][0]), fp8x2_bf16<false>(wv[q][1]),
+                          fp8x2_bf16<true>(wv[q][1])};
+        const u32x4 b1 = {fp8x2_bf16<false>(wv[q][2]), fp8x2_bf16<true>(wv[q][2]), fp8x2_bf16<false>(wv[q][3]),
+                          fp8x2_bf16<true>(wv[q][3])};
+        acc = mfma_bf16(xv[q][0], b0, acc);
+        acc = mfma_bf16(xv[q][1], b1, acc);
+    }
+    // lane (j, kq) holds rows 4 kq + e of column j: x row kq, its own part at e = j / 4
+    const int part = j >> 2;
+    const float y = part == 0 ? acc[0] : part == 1 ? acc[1] : part == 2 ? acc[2] : acc[3];
+    red[kq * kSlabRows + (j & 3)][(wave * 4 + part) & 15] = y;
     __syncthreads();
-    if ((tid >> 4) >= kOut) return;
-    const float a = sum16_dpp(gw < NW ? red[g][gw] : 0.0f);
-    if (gw != 0 || om >= hM) return;
+    if ((tid >> 4) >= hM * kSlabRows) return;
+    float a = 0.0f;
+    if (hchain) {  // in order, as the several-block kernel adds its waves
+#pragma unroll
+        for (int w = 0; w < 16; w += 4) {
+            const float4 v = *reinterpret_cast<const float4*>(&red[g][w]);
+            a = (((a + (w < hnv ? v.x : 0.0f)) + (w + 1 < hnv ? v.y : 0.0f)) + (w + 2 < hnv ? v.z : 0.0f)) +
+                (w + 3 < hnv ? v.w : 0.0f);
+        }
+    } else {
+        a = sum16_dpp(gw < hnv ? red[g][gw] : 0.0f);
+    }
+    if (gw != 0) return;
     float o = a * rs;
     if (p.epi == BZ_EPI_RESIDUAL) o += p.res_f32 ? __uint_as_float(resv.w) : bf16_lo(resv.w >> resv.shift);
     const int64_t oi = (int64_t)om * p.ldo + blk * 16 + orow;
@@ -126,37 +122,12 @@ __global__ void __launch_bounds__(1024) gemv_slab(const uint8_t* hw, const uint1
 
 // ---- host side -----------------------------------------------------------------
 
-template <int M, int RL, int NI>
+template <int UPW>
 int launch_slab_kernel(const StreamParams& p, const SlabLaunch& l, hipStream_t st) {
     if (!stream_hot_ok(p)) return BZ_ERR_UNSUPPORTED;
-    hipLaunchKernelGGL((gemv_slab<M, RL, NI>), dim3(l.grid), dim3(l.nw * 64), 0, st, p.w, p.x, (int)p.chunk, (int)p.ldx,
-                       p.K, p.NU, p.M, p);
+    hipLaunchKernelGGL((gemv_slab<UPW>), dim3(l.grid), dim3(l.threads), 0, st, p.w, p.x, (int)p.chunk, (int)p.ldx, p.NU,
+                       p.M, l.nv, l.chain, p);
     return hipGetLastError() == hipSuccess ? BZ_OK : BZ_ERR_LAUNCH;
-}
-
-// (the shapes the rule takes: 16 rows per workgroup for one row of x only;
-// 3 and 4 rows of x over 4 rows and one group per wave)
-template <int M, int RL>
-int launch_slab_ni(const StreamParams& p, const SlabLaunch& l, hipStream_t st) {
-    if (l.ni == 1) return launch_slab_kernel<M, RL, 1>(p, l, st);
-    if constexpr (M <= 2) {
-        switch (l.ni) {
-            case 2: return launch_slab_kernel<M, RL, 2>(p, l, st);
-            case 3: return launch_slab_kernel<M, RL, 3>(p, l, st);
-            default: break;
-        }
-    }
-    return BZ_ERR_INVALID_ARG;
-}
-
-template <int M>
-int launch_slab_rl(const StreamParams& p, const SlabLaunch& l, hipStream_t st) {
-    if (l.rl == 1) return launch_slab_ni<M, 1>(p, l, st);
-    if constexpr (M <= 2)
-        if (l.rl == 2) return launch_slab_ni<M, 2>(p, l, st);
-    if constexpr (M == 1)
-        if (l.rl == 4) return launch_slab_ni<M, 4>(p, l, st);
-    return BZ_ERR_INVALID_ARG;
 }
 
 // bz_gemv_slab.hip

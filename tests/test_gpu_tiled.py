@@ -684,3 +684,9 @@ def test_few_block_fp8_rule(n, k, m):
                          out_dtype=torch.float32))
         want = ref if res is None else ref + f32(res)
         assert np.all(np.abs(got - want) <= k * 2.0 ** -23 * mag + 2.0 ** -22 * np.abs(want) + 1e-30), (res_dt,)
+        # bit for bit the kernel it stands in for (forced: the one-block
+        # kernel, or the several-block kernel with one block)
+        other = 1 if k >= 4096 or (m >= 3 and k <= 8192) else 0
+        assert np.array_equal(got, f32(G.gemv(wide[:, :k], buf, fmt, n, residual=res, out_dtype=torch.float32,
+                                              epilogue=G.EPI_NONE if res is None else G.EPI_RESIDUAL,
+                                              cfg=(0, 0, other, 5)))), (res_dt,)
