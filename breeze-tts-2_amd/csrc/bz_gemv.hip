@@ -650,9 +650,14 @@ static int gemv_panel_rows(const bz_gemv_desc* d, hipStream_t st) {
 // The kernel was the faster one at every shape and M = 1..4 timed, against
 // the better of the dot2 and matrix-core kernels: N4096 K2048 M = 2 6.94 ->
 // 4.96, N2048 K2048 5.36 -> 3.80, N12288 K2048 SiLU-gate 13.1 -> 10.8, N1024
-// K8192 8.36 -> 5.39, N8192 K2560 M = 3 11.5 -> 10.5.
+// K8192 8.36 -> 5.39, N8192 K2560 M = 3 11.5 -> 10.5.  Plain products (no norm,
+// no epilogue) stay on those kernels all the same, for their order of sums: the
+// depth decoder's embedding projector is one, and a last-bit difference there
+// changes the tokens of a frame whose logits nearly tie; it runs once a
+// codebook (N1024 K2048 M = 2 3.9 us, 2.9 here).
 static bool rows_plan(const bz_gemv_desc* d, const DescInfo& di, int rows, RowsLaunch& l) {
     if (d->wfmt != BZ_W_BF16 || d->cfg_path || d->cfg_waves || d->cfg_tiles || d->cfg_depth) return false;
+    if (!d->gamma && d->epilogue == BZ_EPI_NONE) return false;
     if (d->K > kRowsMaxK || (int64_t)rows * d->ldx * 2 >= (int64_t(1) << 31)) return false;
     l.pair = d->epilogue == BZ_EPI_SILU_GATE;
     const int spans = (d->K + 512 * kRowsMaxKc - 1) / (512 * kRowsMaxKc);

@@ -1,6 +1,5 @@
 // Decode GEMV over plain bf16 weights [N][K]: the unquantized projections of
-// a fused layer, the embedding projector and the bf16 head, for up to 4 rows
-// of x per launch.
+// a fused layer, for up to 4 rows of x per launch.
 //
 // Replaces rms_gemv_kernel + gemv_epilogue_kernel for bf16 weights
 // (models/fused/kernels.py:41-138).
