@@ -9,16 +9,16 @@
 //
 //   1. combined logits of the row (and its greedy argmax, first index of the
 //      maximum, as torch.argmax) into LDS, divided by the temperature;
-//   2. the k-th largest entry (k = top_k, or the whole workspace) by a radix
-//      select over unique 64-bit keys (scaled value, then ascending index),
-//      and a bitonic sort of just those k entries (padded to a power of two
-//      >= 64; partners under 64 apart trade through wave shuffles): rank r of
-//      the sorted set is rank r of top-k;
-//   3. the top-k ranks (k = top_k, or the whole workspace for top_k <= 0)
-//      and their softmax (one rank per thread, the workspace is <= 1024
-//      wide), an inclusive block scan of it, and the top-p prefix: rank r
-//      stays when r == 0 or the cumulative probability before it is <= top_p
-//      (the reference's shifted mask), so the kept set is a prefix of ranks;
+//   2. the first k ranks of the row in order (k = top_k, or the whole
+//      workspace for top_k <= 0; the workspace is <= 1024 wide), by unique
+//      64-bit keys (scaled value, then ascending index): a histogram of the
+//      values picks the buckets that hold them and each one's rank comes
+//      from its own bucket; rows that do not suit it take a radix select and
+//      a bitonic sort;
+//   3. their softmax (one rank per thread), an inclusive scan of it, and the
+//      top-p prefix: rank r stays when r == 0 or the cumulative probability
+//      before it is <= top_p (the reference's shifted mask), so the kept set
+//      is a prefix of ranks;
 //   4. one uniform draw u in [0, 1) (Philox4x32-10, Salmon, Moraes, Dror and
 //      Shaw, "Parallel random numbers: as easy as 1, 2, 3", SC 2011; key =
 //      the 64-bit seed, read from device memory so a captured graph picks up
@@ -35,6 +35,7 @@
 #include <math.h>
 #include <stdint.h>
 
+#include "bz_device.h"
 #include "bz_gemv.h"
 #include "bz_sample.h"
 
@@ -109,101 +110,96 @@ __device__ __forceinline__ float wave_scan_incl(float v, int lane) {
 }
 
 constexpr int kPerThread = kSampleWidth / kSampleThreads;  // row entries a thread holds
+constexpr int NW = kSampleThreads / 64;
+constexpr int kBuckets = kSampleThreads;  // value buckets of the fast order, one per thread
+constexpr int kBucketCap = 64;            // fullest bucket the fast order ranks by comparing
+constexpr float kExpSpan = 110.0f;        // expf(-kExpSpan) is 0 in fp32
+static_assert(NW == 16, "one 16-lane row holds a value of each wave");
+constexpr int kCand = kSampleMaxK + kBucketCap;
 
-__global__ void __launch_bounds__(kSampleThreads) sample_cfg_kernel(SampleParams p) {
-    __shared__ uint64_t cand[kSampleMaxK];  // the selected keys, then sorted
-    __shared__ unsigned hist[256];
-    __shared__ float wsum[kSampleThreads / 64];
-    __shared__ float wbest_v[kSampleThreads / 64];
-    __shared__ int wbest_i[kSampleThreads / 64];
-    __shared__ int greedy_s, ncand, sel_digit, sel_need, sel_count, pick, last_kept;
-    const int r = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    constexpr int NW = kSampleThreads / 64;
-    const float* cond = p.logits + (int64_t)r * p.ld;
-    const float* uncond = p.logits + (int64_t)(p.B >= 2 ? p.half + r : r) * p.ld;
-    const float g = p.B >= 2 ? p.guidance[r] : 0.0f;
-    const float temp = p.temperature[r];
+// Bucket of a scaled value, 0 for the row's maximum: subtraction, product
+// with scale >= 0 and truncation each keep the order, so a smaller bucket
+// never holds a smaller value.
+__device__ __forceinline__ int value_bucket(float s, float top, float scale) {
+    return min((int)((top - s) * scale), kBuckets - 1);
+}
 
-    // 1. combined logits, greedy argmax, the scaled entries' keys (registers)
-    float best_v = -INFINITY;
-    int best_i = 0x7FFFFFFF;
-    uint64_t key[kPerThread];
-#pragma unroll
-    for (int q = 0; q < kPerThread; ++q) {
-        const int v = tid + q * kSampleThreads;
-        key[q] = 0;  // absent (below every entry's key)
-        if (v < p.V) {
-            float c = cond[v];
-            if (p.B >= 2) {
-                const float u = uncond[v];
-                c = u + g * (c - u);
-            }
-            if (v >= p.codec) c = -INFINITY;
-            if (p.cfg_out) p.cfg_out[(int64_t)r * p.V + v] = c;
-            if (c > best_v || best_i == 0x7FFFFFFF) {  // ascending v: the first maximum wins
-                best_v = c;
-                best_i = v;
-            }
-            key[q] = entry_key(c / temp, v);
-        }
-    }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        const float ov = __shfl_xor(best_v, o, 64);
-        const int oi = __shfl_xor(best_i, o, 64);
-        if (ov > best_v || (ov == best_v && oi < best_i)) {
-            best_v = ov;
-            best_i = oi;
-        }
-    }
-    if (lane == 0) {
-        wbest_v[wave] = best_v;
-        wbest_i[wave] = best_i;
-    }
-    if (tid == 0) ncand = 0;
+// The row's token, in one wave: to the row and its twin; the row's call
+// count advances.
+__device__ __forceinline__ void put_token(const SampleParams& p, int r, int tok, uint64_t cnt) {
+    tok = tok < 0 ? 0 : (tok >= p.V ? p.V - 1 : tok);
+    p.tokens[r] = tok;
+    if (p.B >= 2) p.tokens[p.half + r] = tok;
+    p.counters[r] = cnt + 1;
+}
 
-    // A greedy row with no probabilities to report needs only the argmax:
-    // skip the select, sort, softmax and draw.  Same token (same reduction
-    // order as below) and the call count advances as on the full path.
-    if (!p.do_sample[r] && !p.probs_out) {
-        __syncthreads();
-        if (tid == 0) {
-            float bv = wbest_v[0];
-            int bi = wbest_i[0];
-            for (int w = 1; w < NW; ++w)
-                if (wbest_v[w] > bv || (wbest_v[w] == bv && wbest_i[w] < bi)) {
-                    bv = wbest_v[w];
-                    bi = wbest_i[w];
-                }
-            const int64_t tok = bi < 0 ? 0 : (bi >= p.V ? p.V - 1 : bi);
-            p.tokens[r] = tok;
-            if (p.B >= 2) p.tokens[p.half + r] = tok;
-            p.counters[r] = p.counters[r] + 1;
-        }
-        return;
-    }
+// Reductions over 16-lane rows and the wave in DPP moves: a step is one VALU
+// operation where a shuffle is an LDS round trip.
+template <int CTRL>
+__device__ __forceinline__ int dpp_i32(int v) {
+    return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xF, 0xF, false);
+}
+__device__ __forceinline__ int min16_dpp(int v) {
+    v = min(v, dpp_i32<kDppXor1>(v));
+    v = min(v, dpp_i32<kDppXor2>(v));
+    v = min(v, dpp_i32<kDppHalfMirror>(v));
+    return min(v, dpp_i32<kDppRowMirror>(v));
+}
+__device__ __forceinline__ float lane_f32(float v, int lane) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
+}
+__device__ __forceinline__ float wave_max_dpp(float v) {
+    v = max16_dpp(v);
+    return fmaxf(fmaxf(lane_f32(v, 0), lane_f32(v, 16)), fmaxf(lane_f32(v, 32), lane_f32(v, 48)));
+}
+__device__ __forceinline__ int wave_min_dpp(int v) {
+    v = min16_dpp(v);
+    return min(min(__builtin_amdgcn_readlane(v, 0), __builtin_amdgcn_readlane(v, 16)),
+               min(__builtin_amdgcn_readlane(v, 32), __builtin_amdgcn_readlane(v, 48)));
+}
+// inclusive scan of each 16-lane row (row_shr 1, 2, 4, 8), then of the wave
+__device__ __forceinline__ int row_scan_dpp(int v) {
+    v += dpp_i32<0x111>(v);
+    v += dpp_i32<0x112>(v);
+    v += dpp_i32<0x114>(v);
+    return v + dpp_i32<0x118>(v);
+}
+__device__ __forceinline__ int wave_scan_dpp(int v) {
+    v = row_scan_dpp(v);
+    v += __builtin_amdgcn_update_dpp(0, v, kDppRowBcast15, 0xA, 0xF, false);
+    return v + __builtin_amdgcn_update_dpp(0, v, kDppRowBcast31, 0xC, 0xF, false);
+}
 
-    // 2. the k-th largest key (k = top_k, or the whole workspace): radix
-    //    select over 8-bit digits from the top; keys are unique, so exactly k
-    //    keys are >= the result.  A pass whose chosen bucket holds exactly
-    //    the keys still needed ends the search.
-    const int64_t tk = p.top_k[r];
-    const int kk = tk > 0 ? (int)min<int64_t>(tk, p.max_k) : p.max_k;
+struct SampleShared {
+    uint64_t cand[kCand];          // the candidates, bucket by bucket
+    uint64_t sorted[kSampleMaxK];  // the keys of ranks 0, 1, ...
+    unsigned hist[kBuckets];       // counts, then where each bucket ends in cand
+    float wsum[NW], wtop[NW], wlow[NW], wbest_v[NW];
+    int wbest_i[NW];
+    int wcount[NW];
+    int ncand, sel_digit, sel_need, sel_count, pick, last_kept, nsel, full;
+};
+
+// The largest kk keys of the row in sh.sorted, descending, by a radix select
+// over 8-bit digits and a bitonic sort: any keys, any ties.
+__device__ __forceinline__ void select_general(SampleShared& sh, const uint64_t (&key)[kPerThread], int kk) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     uint64_t prefix = 0, mask = 0;
     int need = kk;
+    if (tid == 0) sh.ncand = 0;
     for (int shift = 56; shift >= 0; shift -= 8) {
-        if (tid < 256) hist[tid] = 0u;
+        if (tid < 256) sh.hist[tid] = 0u;
         __syncthreads();
 #pragma unroll
         for (int q = 0; q < kPerThread; ++q)
-            if (key[q] != 0 && (key[q] & mask) == prefix) atomicAdd(&hist[(key[q] >> shift) & 255u], 1u);
+            if (key[q] != 0 && (key[q] & mask) == prefix) atomicAdd(&sh.hist[(key[q] >> shift) & 255u], 1u);
         __syncthreads();
         if (wave == 0) {
             // lane l covers digits 255 - 4l .. 252 - 4l (top down)
             unsigned c4[4], sum = 0;
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                c4[q] = hist[255 - 4 * lane - q];
+                c4[q] = sh.hist[255 - 4 * lane - q];
                 sum += c4[q];
             }
             unsigned incl = sum;
@@ -216,29 +212,28 @@ __global__ void __launch_bounds__(kSampleThreads) sample_cfg_kernel(SampleParams
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 if (above < (unsigned)need && above + c4[q] >= (unsigned)need) {
-                    sel_digit = 255 - 4 * lane - q;
-                    sel_need = need - (int)above;
-                    sel_count = (int)c4[q];
+                    sh.sel_digit = 255 - 4 * lane - q;
+                    sh.sel_need = need - (int)above;
+                    sh.sel_count = (int)c4[q];
                 }
                 above += c4[q];
             }
         }
         __syncthreads();
-        prefix |= (uint64_t)sel_digit << shift;
+        prefix |= (uint64_t)sh.sel_digit << shift;
         mask |= (uint64_t)255u << shift;
-        need = sel_need;
-        if (sel_count == need) break;  // workgroup-uniform
+        need = sh.sel_need;
+        if (sh.sel_count == need) break;  // workgroup-uniform
     }
-
-    // 3. the kk selected keys into LDS, padded with zeros to P (a power of
-    //    two >= 64), then a bitonic sort, descending: partners less than 64
-    //    apart trade through wave shuffles, wider ones through LDS
+    // the kk selected keys, padded with zeros to P (a power of two >= 64),
+    // then a bitonic sort, descending: partners less than 64 apart trade
+    // through wave shuffles, wider ones through LDS
     const int P = max(64, 1 << (32 - __clz(kk - 1)));
 #pragma unroll
     for (int q = 0; q < kPerThread; ++q)
-        if (key[q] != 0 && key[q] >= prefix) cand[atomicAdd(&ncand, 1)] = key[q];
+        if (key[q] != 0 && key[q] >= prefix) sh.cand[atomicAdd(&sh.ncand, 1)] = key[q];
     __syncthreads();
-    uint64_t mine = tid < kk ? cand[tid] : 0;
+    uint64_t mine = tid < kk ? sh.cand[tid] : 0;
     for (int lk = 1; (1 << lk) <= P; ++lk) {
         const int k = 1 << lk;
         for (int lj = lk - 1; lj >= 0; --lj) {
@@ -248,88 +243,250 @@ __global__ void __launch_bounds__(kSampleThreads) sample_cfg_kernel(SampleParams
                 theirs = shfl_xor64(mine, j);
             } else {
                 __syncthreads();
-                if (tid < P) cand[tid] = mine;
+                if (tid < P) sh.cand[tid] = mine;
                 __syncthreads();
-                theirs = tid < P ? cand[tid ^ j] : 0;
+                theirs = tid < P ? sh.cand[tid ^ j] : 0;
             }
             const bool lower = (tid & j) == 0, desc = (tid & k) == 0;
             const uint64_t hi = mine > theirs ? mine : theirs, lo = mine > theirs ? theirs : mine;
             if (tid < P) mine = (lower == desc) ? hi : lo;
         }
     }
-    if (tid == 0) {
-        float bv = wbest_v[0];
-        int bi = wbest_i[0];
-        for (int w = 1; w < NW; ++w)
-            if (wbest_v[w] > bv || (wbest_v[w] == bv && wbest_i[w] < bi)) {
-                bv = wbest_v[w];
-                bi = wbest_i[w];
+    sh.sorted[tid] = mine;
+    __syncthreads();
+}
+
+// One workgroup a row, so latency is all of it: parameters and logits are
+// requested together, reductions stay in DPP moves, and the chain of barriers
+// and LDS round trips is short.  Measured on MI355X in a graph of 16 launches,
+// V = 2051, B = 2, with probs_out: 14.6 us a launch with the radix select and
+// shuffle reductions for every row, 6.0 us now (top_k = 50); 20.8 and 8.6 us
+// at top_k = 1000.
+__global__ void __launch_bounds__(kSampleThreads) sample_cfg_kernel(SampleParams p) {
+    __shared__ SampleShared sh;
+    const int r = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const float* cond = p.logits + (int64_t)r * p.ld;
+    const float* uncond = p.logits + (int64_t)(p.B >= 2 ? p.half + r : r) * p.ld;
+    const float g = p.B >= 2 ? p.guidance[r] : 0.0f;
+    const float temp = p.temperature[r];
+    const int64_t tk = p.top_k[r];
+    const float top_p = p.top_p[r];
+    const bool sample = p.do_sample[r] != 0;
+    const uint64_t cnt = p.counters[r], seed = *p.seed;
+    float* pr = p.probs_out ? p.probs_out + (int64_t)r * p.V : nullptr;
+
+    // 1. combined logits, greedy argmax, the scaled entries' keys (registers)
+    float best_v = -INFINITY, top = -INFINITY, low = INFINITY;
+    int best_i = 0x7FFFFFFF;
+    float sv[kPerThread], cv[kPerThread], uv[kPerThread];
+#pragma unroll
+    for (int q = 0; q < kPerThread; ++q) {  // every load is in flight before the first is used
+        const int v = min(tid + q * kSampleThreads, p.V - 1);
+        cv[q] = cond[v];
+        uv[q] = uncond[v];
+    }
+    sh.hist[tid] = 0u;
+    uint64_t key[kPerThread];
+#pragma unroll
+    for (int q = 0; q < kPerThread; ++q) {
+        const int v = tid + q * kSampleThreads;
+        key[q] = 0;  // absent (below every entry's key)
+        sv[q] = -INFINITY;
+        if (v < p.V) {
+            float c = cv[q];
+            if (p.B >= 2) c = uv[q] + g * (c - uv[q]);
+            if (v >= p.codec) c = -INFINITY;
+            if (p.cfg_out) p.cfg_out[(int64_t)r * p.V + v] = c;
+            if (pr) pr[v] = 0.0f;  // (barriers lie between this and step 3)
+            if (c > best_v || best_i == 0x7FFFFFFF) {  // ascending v: the first maximum wins
+                best_v = c;
+                best_i = v;
             }
-        greedy_s = bi;
+            sv[q] = c / temp;
+            key[q] = entry_key(sv[q], v);
+            // a NaN counts as infinite: neither is left to the fast order
+            top = sv[q] <= top ? top : (sv[q] > top ? sv[q] : INFINITY);
+            if (sv[q] > -INFINITY) low = fminf(low, sv[q]);
+        }
+    }
+    top = wave_max_dpp(top);
+    low = -wave_max_dpp(-low);
+    if (top < INFINITY) {  // no NaNs: the maximum, then its first index
+        const float bv = wave_max_dpp(best_v);
+        best_i = wave_min_dpp(best_v == bv ? best_i : 0x7FFFFFFF);
+        best_v = bv;
+    } else {
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+            const float ov = __shfl_xor(best_v, o, 64);
+            const int oi = __shfl_xor(best_i, o, 64);
+            if (ov > best_v || (ov == best_v && oi < best_i)) {
+                best_v = ov;
+                best_i = oi;
+            }
+        }
+    }
+    if (lane == 0) {
+        sh.wbest_v[wave] = best_v;
+        sh.wbest_i[wave] = best_i;
+        sh.wtop[wave] = top;
+        sh.wlow[wave] = low;
+    }
+    if (tid == 0) {
+        sh.nsel = kSampleWidth;
+        sh.full = 0;
+        sh.pick = 0x7FFFFFFF;
+        sh.last_kept = 0;
+    }
+    __syncthreads();
+    top = lane_f32(max16_dpp(sh.wtop[lane & 15]), 0);
+    low = -lane_f32(max16_dpp(-sh.wlow[lane & 15]), 0);
+    int greedy;
+    if (top < INFINITY) {
+        best_v = sh.wbest_v[lane & 15];
+        best_i = sh.wbest_i[lane & 15];
+        greedy = __builtin_amdgcn_readlane(min16_dpp(best_v == max16_dpp(best_v) ? best_i : 0x7FFFFFFF), 0);
+    } else {
+        float bv = sh.wbest_v[0];
+        greedy = sh.wbest_i[0];
+        for (int w = 1; w < NW; ++w) {
+            const float ov = sh.wbest_v[w];
+            const int oi = sh.wbest_i[w];
+            if (ov > bv || (ov == bv && oi < greedy)) {
+                bv = ov;
+                greedy = oi;
+            }
+        }
     }
 
-    // 4. thread t = rank t: top-k softmax weights, block scan, top-p prefix
-    const int t = tid;
+    // A greedy row with no probabilities to report needs only the argmax:
+    // skip the order, softmax and draw; the call count advances all the same.
+    if (!sample && !p.probs_out) {
+        if (tid == 0) put_token(p, r, greedy, cnt);
+        return;
+    }
+
+    // 2. the entries of ranks 0 .. kk - 1 in order (kk = top_k, or the whole
+    //    workspace).  Fast order: a histogram of the values over kBuckets
+    //    equal steps from the maximum down, the candidates (the buckets that
+    //    hold the first kk entries, whole) grouped by bucket, and each one's
+    //    rank from the few others of its bucket.  Entries more than kExpSpan
+    //    below the maximum weigh 0, as -inf does, and take no rank.  Rows
+    //    with infinities or NaNs, and rows crowded into a bucket, take the
+    //    radix select instead.
+    const int kk = tk > 0 ? (int)min<int64_t>(tk, p.max_k) : p.max_k;
+    low = fmaxf(low, top - kExpSpan);
+    const float range = top - low;
+    bool fast = top < INFINITY && top > -INFINITY;  // (then low and range are finite)
+    int nrank = kk;                                 // ranks in sh.sorted
+    if (fast) {                                     // workgroup-uniform
+        const float scale = range > 1e-30f ? (float)kBuckets / range : 0.0f;
+#pragma unroll
+        for (int q = 0; q < kPerThread; ++q)
+            if (sv[q] >= low) atomicAdd(&sh.hist[value_bucket(sv[q], top, scale)], 1u);
+        __syncthreads();
+        const int c = (int)sh.hist[tid];
+        int incl = wave_scan_dpp(c);
+        if (lane == 63) sh.wcount[wave] = incl;
+        __syncthreads();
+        const int upto = row_scan_dpp(sh.wcount[lane & 15]);  // entries of waves 0 .. lane & 15
+        if (wave) incl += __builtin_amdgcn_readlane(upto, wave - 1);
+        nrank = min(kk, __builtin_amdgcn_readlane(upto, 15));
+        const int start = incl - c;
+        if (start < nrank && incl >= nrank) sh.nsel = incl;  // the last bucket taken
+        if (c > kBucketCap && start < nrank) sh.full = 1;
+        sh.hist[tid] = (unsigned)start;
+        __syncthreads();
+        fast = !sh.full;
+        if (fast) {
+            const int n = sh.nsel;  // < nrank + kBucketCap <= kCand
+#pragma unroll
+            for (int q = 0; q < kPerThread; ++q)
+                if (sv[q] >= low) {
+                    const int b = value_bucket(sv[q], top, scale);
+                    // buckets past the last taken start at n: entries that
+                    // would go there add nothing
+                    if (sh.hist[b] < (unsigned)n) sh.cand[atomicAdd(&sh.hist[b], 1u)] = key[q];
+                }
+            __syncthreads();
+            for (int t = tid; t < n; t += kSampleThreads) {
+                const uint64_t mine = sh.cand[t];
+                const int b = value_bucket(key_value(mine), top, scale);
+                const int lo = b ? (int)sh.hist[b - 1] : 0, hi = (int)sh.hist[b];
+                int rank = lo;
+                for (int j = lo; j < hi; j += 4) {  // four reads in flight
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const uint64_t other = sh.cand[min(j + i, kCand - 1)];
+                        rank += j + i < hi && other > mine;
+                    }
+                }
+                if (rank < nrank) sh.sorted[rank] = mine;
+            }
+            __syncthreads();
+        }
+    }
+    if (!fast) {
+        nrank = kk;
+        select_general(sh, key, kk);
+    }
+
+    // 3. thread t = rank t: top-k softmax weights, scan, top-p prefix, draw.
+    //    The kept set is a prefix of ranks: rank 0, and the ranks whose
+    //    cumulative probability before them is <= top_p.
+    if (nrank <= 64 && wave) return;  // wave 0 holds every rank: no more barriers
+    const float m_s = key_value(sh.sorted[0]);
+    const uint64_t mine = tid < nrank ? sh.sorted[tid] : 0;
     const float sv_t = key_value(mine);
     const int si_t = key_index(mine);
-    __shared__ float m_s;  // rank 0 holds the maximum
-    if (tid == 0) m_s = sv_t;
-    __syncthreads();
-    const float e = (t < kk && sv_t > -INFINITY) ? expf(sv_t - m_s) : 0.0f;
+    const float e = (tid < nrank && sv_t > -INFINITY) ? expf(sv_t - m_s) : 0.0f;
+    uint32_t c[4] = {(uint32_t)cnt, (uint32_t)(cnt >> 32), (uint32_t)r, 0u};
+    philox4x32_10(c, (uint32_t)seed, (uint32_t)(seed >> 32));
+    const float u = (float)(c[0] >> 8) * (1.0f / 16777216.0f);
     float inc = wave_scan_incl(e, lane);
-    if (lane == 63) wsum[wave] = inc;
+    if (nrank <= 64) {
+        const float total = __shfl(inc, 63, 64);
+        const bool kept = e > 0.0f && (tid == 0 || (inc - e) / total <= top_p);
+        const float ke = kept ? e : 0.0f;
+        float kept_total = ke;
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) kept_total += __shfl_xor(kept_total, o, 64);
+        if (pr && kept) pr[si_t] = ke / kept_total;
+        const uint64_t over = __ballot(kept && inc > u * kept_total), any = __ballot(kept);
+        // the first kept rank past the draw; rounding at the top end: the last kept one
+        const int at = over ? __ffsll((unsigned long long)over) - 1
+                            : (any ? 63 - __clzll((long long)any) : 0);
+        if (lane == at) put_token(p, r, sample ? si_t : greedy, cnt);
+        return;
+    }
+    if (lane == 63) sh.wsum[wave] = inc;
     __syncthreads();
     float before_w = 0.0f, total = 0.0f;
     for (int w = 0; w < NW; ++w) {
-        if (w < wave) before_w += wsum[w];
-        total += wsum[w];
+        if (w < wave) before_w += sh.wsum[w];
+        total += sh.wsum[w];
     }
     inc += before_w;
     const float exc = inc - e;
-    // kept: rank 0, or the cumulative probability before this rank <= top_p
-    const bool kept = t < kk && e > 0.0f && (t == 0 || exc / total <= p.top_p[r]);
+    const bool kept = e > 0.0f && (tid == 0 || exc / total <= top_p);
     __syncthreads();  // wsum is reused below
-    const float ke = kept ? e : 0.0f;  // the kept set is a prefix of ranks
+    const float ke = kept ? e : 0.0f;
     float ks = ke;
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) ks += __shfl_xor(ks, o, 64);
-    if (lane == 0) wsum[wave] = ks;
-    if (tid == 0) {
-        pick = 0x7FFFFFFF;
-        last_kept = 0;
-    }
+    if (lane == 0) sh.wsum[wave] = ks;
     __syncthreads();
     float kept_total = 0.0f;
-    for (int w = 0; w < NW; ++w) kept_total += wsum[w];
-
-    if (p.probs_out) {
-        float* pr = p.probs_out + (int64_t)r * p.V;
-        for (int v = tid; v < p.V; v += kSampleThreads) pr[v] = 0.0f;
-        __syncthreads();
-        if (kept) pr[si_t] = ke / kept_total;
-    }
-
-    // 5. the draw: the first kept rank whose cumulative weight exceeds
-    //    u * kept_total (kept ranks are a prefix, so their cumulative weight
-    //    is `inc`)
-    const uint64_t cnt = p.counters[r];
-    uint32_t c[4] = {(uint32_t)cnt, (uint32_t)(cnt >> 32), (uint32_t)r, 0u};
-    const uint64_t keyr = *p.seed;
-    philox4x32_10(c, (uint32_t)keyr, (uint32_t)(keyr >> 32));
-    const float u = (float)(c[0] >> 8) * (1.0f / 16777216.0f);
-    if (kept) {
-        atomicMax(&last_kept, t);
-        if (inc > u * kept_total) atomicMin(&pick, t);
+    for (int w = 0; w < NW; ++w) kept_total += sh.wsum[w];
+    if (pr && kept) pr[si_t] = ke / kept_total;
+    const uint64_t over = __ballot(kept && inc > u * kept_total), any = __ballot(kept);
+    if (lane == 0) {  // one LDS atomic a wave
+        if (any) atomicMax(&sh.last_kept, tid + 63 - __clzll((long long)any));
+        if (over) atomicMin(&sh.pick, tid + __ffsll((unsigned long long)over) - 1);
     }
     __syncthreads();
-    if (tid == (pick == 0x7FFFFFFF ? last_kept : pick)) {  // rounding at the top end: the last kept rank
-        // 6. the token, to the row and its twin; advance the row's call count
-        int64_t tok = p.do_sample[r] ? (int64_t)si_t : (int64_t)greedy_s;
-        tok = tok < 0 ? 0 : (tok >= p.V ? p.V - 1 : tok);
-        p.tokens[r] = tok;
-        if (p.B >= 2) p.tokens[p.half + r] = tok;
-        p.counters[r] = cnt + 1;
-    }
+    if (tid == (sh.pick == 0x7FFFFFFF ? sh.last_kept : sh.pick)) put_token(p, r, sample ? si_t : greedy, cnt);
 }
 
 }  // namespace

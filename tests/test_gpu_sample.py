@@ -177,3 +177,76 @@ def test_graph_replays_advance_and_match_eager():
         assert torch.equal(tokens, eager[i]), i
         _ = torch.randn(256, device=DEV).sum().item()  # eager work between replays
     assert len({tuple(t.tolist()) for t in eager}) > 1
+
+
+def _edge_row(kind, V, gen):
+    x = torch.randn(V, device=DEV, generator=gen) * 3
+    if kind == "ties":
+        x = torch.round(x)                     # a few dozen values: crowded buckets
+    elif kind == "equal":
+        x = torch.zeros_like(x)
+    elif kind == "outlier":
+        x[V // 2] = 90.0                       # weights far below the maximum's
+    elif kind == "lowest":
+        x[::3] = torch.finfo(torch.float32).min  # a mask's lowest value on a third of the row
+    elif kind == "neg_inf":
+        x[V // 4:] = float("-inf")
+    elif kind == "one_left":
+        x[:] = float("-inf")
+        x[V - 3] = -1.5
+    elif kind == "narrow":
+        x = x * 1e-6
+    elif kind == "pos_inf":
+        x[7] = float("inf")
+    return x
+
+
+@pytest.mark.parametrize("V", [1, 65, 1025, 2051, 4096])
+@pytest.mark.parametrize("kind", ["normal", "ties", "equal", "outlier", "lowest", "neg_inf", "one_left", "narrow"])
+def test_rank_order_at_the_edges(V, kind):
+    """The kept set and its probabilities against a stable sort in float64,
+    for rows of both orders (histogram, radix select) and k around one wave,
+    the block and the row.  An fp32 weight exp(s - m) has a relative error of
+    a few 2^-23 plus |s - m| * 2^-24 from the rounded difference; sums of up
+    to 1024 of them add 10 levels of 2^-24: 2e-5 covers |s - m| <= 104."""
+    if kind in ("neg_inf", "one_left") and V < 4:
+        pytest.skip("needs a few entries")
+    ks = sorted({1, 2, 50, 63, 64, 65, 300, 1023, 1024, 0})
+    half = len(ks)
+    gen = torch.Generator(device=DEV).manual_seed(V)
+    row = _edge_row(kind, V, gen)
+    logits = row.expand(2 * half, V).contiguous()
+    prm = _params(half, top_k=ks, guidance=0.0, top_p=2.0)  # uncond + 0 * (cond - uncond): the row itself
+    if kind == "neg_inf" or kind == "one_left":
+        prm["guidance"] = torch.ones(half, device=DEV)  # 0 + (row - 0): two infinities have no difference
+        logits[half:] = 0.0
+    probs = torch.empty(half, V, device=DEV)
+    cfg = torch.empty(half, V, device=DEV)
+    tokens = torch.empty(2 * half, dtype=torch.int64, device=DEV)
+    sample_cfg(logits, tokens, SampleState(half, DEV, seed=5), codec_size=V, max_k=1024, probs_out=probs, cfg_out=cfg,
+               **prm)
+    torch.cuda.synchronize()
+    assert torch.equal(cfg[0], row)
+    s, idx = torch.sort(row.double().cpu(), descending=True, stable=True)
+    for r, k in enumerate(ks):
+        kk = min(k or 1024, 1024, V)
+        w = torch.softmax(s[:kk], 0)
+        want = torch.zeros(V, dtype=torch.float64).scatter_(0, idx[:kk], w)
+        got = probs[r].double().cpu()
+        torch.testing.assert_close(got, want, rtol=2e-5, atol=1e-37, msg=lambda m: f"k={k}: {m}")
+        assert got[tokens[r]] > 0, k
+
+
+@pytest.mark.parametrize("kind", ["pos_inf", "nan"])
+def test_rows_with_infinities_stay_in_range(kind):
+    """A row whose weights are no numbers still gives tokens of the vocabulary."""
+    V = 2051
+    row = _edge_row(kind, V, torch.Generator(device=DEV).manual_seed(2))
+    if kind == "nan":
+        row[100] = float("nan")
+    tokens = torch.full((1,), -1, dtype=torch.int64, device=DEV)
+    prm = _params(1, top_k=50)
+    prm["guidance"] = None
+    sample_cfg(row.view(1, V), tokens, SampleState(1, DEV, seed=5), **prm)
+    torch.cuda.synchronize()
+    assert 0 <= int(tokens[0]) < V
