@@ -45,6 +45,8 @@ EXPORTS = (
     "bz_tiled_bytes",
     "bz_pack_tiled",
     "bz_head_f32",
+    "bz_norm_head_f32",
+    "bz_step_tables",
     "bz_qkv_rope_cache",
     "bz_attn_decode",
     "bz_attn_step",
@@ -136,6 +138,11 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.bz_head_f32.restype = ctypes.c_int
     lib.bz_head_f32.argtypes = [vp, i64, i32, i32, vp, i32, i64, i32, vp, i64, vp, i64, vp]
     lib.bz_qkv_rope_cache.restype = ctypes.c_int
+    lib.bz_norm_head_f32.restype = ctypes.c_int
+    lib.bz_norm_head_f32.argtypes = [vp, i64, i32, i32, vp, f32, vp, i64, vp, i32, i64, i32, vp, i64, vp, i64, vp, i64,
+                                     f32, vp]
+    lib.bz_step_tables.restype = ctypes.c_int
+    lib.bz_step_tables.argtypes = [i32, i32, i32, vp, vp, f32, vp, vp, vp, f32, vp, vp, i32, vp]
     lib.bz_qkv_rope_cache.argtypes = [vp, i64, i32, i32, i32, i32, vp, vp, f32, vp, vp, i32, i64, vp, vp, vp, vp,
                                       i32, i32, vp, vp]
     lib.bz_attn_decode.restype = ctypes.c_int

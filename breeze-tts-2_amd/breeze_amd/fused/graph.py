@@ -15,6 +15,11 @@ in static buffers that the host updates in place before each replay:
                                  pad_lens and the position
                                  (backbone_graph.py:240-252)
 
+Around the layers lie two launches: the mask and the rotary tables
+(bz_step_tables), and the final norm, the head and the guidance combination
+(bz_norm_head_f32).  Both stand in only for modules that compute just that,
+which is checked against the modules at set-up; others run as they are.
+
 The layers are called directly (not through the model's forward), so no
 mask construction or shape logic of the model runs inside the capture.
 """
@@ -24,8 +29,9 @@ from __future__ import annotations
 import torch
 from torch import nn
 
-from ..heads import Fp32Linear
-from .install import static_cache
+from ..heads import NORM_HEAD_MAX_K, NORM_HEAD_MAX_ROWS, Fp32Linear, norm_head_f32
+from .install import static_cache, zero_cache
+from .kernels import rmsnorm, step_tables
 
 __all__ = ["BackboneDecodeGraph"]
 
@@ -55,7 +61,50 @@ class BackboneDecodeGraph:
         vocab = self.lm_head.out_features
         self.logits_buf = torch.zeros(batch_size, vocab, dtype=torch.float32, device=dev)
         self.cfg_logits_buf = torch.zeros(self.half, vocab, dtype=torch.float32, device=dev)
+        self._tables = self._rotary_tables()
+        self._norm = self._plain_norm()
         self.graph = None
+
+    # -- what the two launches around the layers may stand in for -------------------
+
+    def _rotary_tables(self):
+        """(inv_freq, scaling, cos, sin) when rotary_emb gives the default tables
+        of bz_step_tables (same bits at a spread of positions), else None."""
+        rot, dt = self.model.rotary_emb, self.inputs_buf.dtype
+        inv, scale = getattr(rot, "inv_freq", None), getattr(rot, "attention_scaling", 1.0)
+        if (self.device.type != "cuda" or dt not in (torch.bfloat16, torch.float32)
+                or getattr(rot, "rope_type", None) != "default" or not isinstance(inv, torch.Tensor)
+                or not inv.is_floating_point() or inv.dim() != 1 or inv.device != self.device):
+            return None
+        B, D = self.batch_size, 2 * inv.numel()
+        inv, scale = inv.detach().float().contiguous(), float(scale)  # the module widens it on every call
+        mask = torch.empty_like(self.attn_mask)
+        tables = [torch.zeros(B, 1, D, dtype=dt, device=self.device) for _ in range(2)]
+        with torch.no_grad():
+            for p in (0, 1, self.max_seq_len // 3, self.max_seq_len - 1):
+                ids = torch.full_like(self.position_ids, p)
+                step_tables(self.pad_lens, self.cache_position, self.mask_min, mask, ids, inv, scale, *tables)
+                want = rot(self.inputs_buf, ids)
+                if not all(w.dtype == dt and w.shape == t.shape and torch.equal(w, t) for w, t in zip(want, tables)):
+                    return None
+        return inv, scale, *tables
+
+    def _plain_norm(self):
+        """(weight, eps) when model.norm is an RMSNorm x / rms(x) * weight that
+        bz_norm_head_f32 can run with this head, else None."""
+        norm, head, H = self.model.norm, self.lm_head, self.inputs_buf.shape[-1]
+        w, eps = getattr(norm, "weight", None), getattr(norm, "variance_epsilon", None)
+        if (self.device.type != "cuda" or type(head) is not Fp32Linear or w is None or eps is None
+                or self.inputs_buf.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or w.shape != (H,)
+                or not w.is_contiguous() or head.in_features != H or H > NORM_HEAD_MAX_K
+                or self.batch_size > NORM_HEAD_MAX_ROWS or (self.batch_size > 1 and self.batch_size % 2)):
+            return None
+        with torch.no_grad():  # two roundings to bf16 in the module, one here: 2^-7 of the value covers them
+            x = torch.linspace(-3, 3, H, device=self.device).to(torch.bfloat16).view(1, H)
+            want, got = norm(x).float(), rmsnorm(x, w.detach(), float(eps)).float()
+            if want.shape != got.shape or not bool(((want - got).abs() <= 2.0 ** -7 * want.abs()).all()):
+                return None
+        return w.detach(), float(eps)
 
     # -- device-side state ---------------------------------------------------------
 
@@ -67,14 +116,25 @@ class BackboneDecodeGraph:
         self.attn_mask[:, 0, 0, :].masked_fill_(valid, 0.0)
 
     def _decode_step(self) -> None:
-        self._set_attention_mask()
         h = self.inputs_buf
-        pe = self.model.rotary_emb(h, self.position_ids)
+        ints = (self.pad_lens, self.cache_position, self.position_ids)
+        if self._tables is not None and all(t.dtype == torch.long and t.is_contiguous() for t in ints):
+            inv, scale, *pe = self._tables
+            step_tables(self.pad_lens, self.cache_position, self.mask_min, self.attn_mask, self.position_ids, inv, scale,
+                        *pe)
+        else:
+            self._set_attention_mask()
+            pe = self.model.rotary_emb(h, self.position_ids)
         for layer in self.model.layers:
             h = layer(h, attention_mask=self.attn_mask, position_ids=self.position_ids,
                       past_key_values=self.static_cache, use_cache=True, cache_position=self.cache_position,
                       position_embeddings=pe)
             h = h[0] if isinstance(h, tuple) else h
+        if self._norm is not None and isinstance(self.guidance_scale, (int, float)):
+            w, eps = self._norm
+            norm_head_f32(h[:, -1, :], w, eps, self.lm_head.weight, out=self.logits_buf,
+                          normed=self.hidden_buf[:, -1, :], cfg=self.cfg_logits_buf, guidance=self.guidance_scale)
+            return
         h = self.model.norm(h)
         self.hidden_buf.copy_(h)
         self.logits_buf.copy_(self.lm_head(self.hidden_buf[:, -1, :].float()))
@@ -115,12 +175,7 @@ class BackboneDecodeGraph:
 
     @torch.inference_mode()
     def reset(self) -> None:
-        for layer in self.static_cache.layers:
-            if getattr(layer, "is_initialized", False):
-                layer.keys.zero_()
-                layer.values.zero_()
-                if isinstance(getattr(layer, "cumulative_length", None), torch.Tensor):
-                    layer.cumulative_length.zero_()
+        zero_cache(self.static_cache)
 
     @torch.inference_mode()
     def step(self, inputs_embeds: torch.Tensor, position: int, position_ids=None) -> torch.Tensor:

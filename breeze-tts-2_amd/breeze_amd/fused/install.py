@@ -18,7 +18,7 @@ import torch
 
 from .layer import FusedDecoderLayer
 
-__all__ = ["install_fused_backbone", "install_fused_depth", "static_cache"]
+__all__ = ["install_fused_backbone", "install_fused_depth", "static_cache", "zero_cache"]
 
 
 def static_cache(config, max_cache_len: int, batch_size: int):
@@ -30,6 +30,19 @@ def static_cache(config, max_cache_len: int, batch_size: int):
         return StaticCache(config=config, max_cache_len=max_cache_len, batch_size=batch_size)
     except TypeError:
         return StaticCache(config=config, max_cache_len=max_cache_len)
+
+
+def zero_cache(cache) -> None:
+    """Zero a static cache and its fill counters (outside any capture), a few
+    launches for all layers instead of three a layer."""
+    bufs = {}
+    for layer in cache.layers:
+        if getattr(layer, "is_initialized", False):
+            n = getattr(layer, "cumulative_length", None)
+            for t in (layer.keys, layer.values) + ((n,) if isinstance(n, torch.Tensor) else ()):
+                bufs.setdefault((t.device, t.dtype), []).append(t)
+    for group in bufs.values():
+        torch._foreach_zero_(group)
 
 
 def _swap_and_prepare(stack, cache_len: int, batch_size: int, mlp_bits, attn_bits) -> int:

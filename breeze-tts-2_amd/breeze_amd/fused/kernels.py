@@ -25,6 +25,7 @@ from __future__ import annotations
 
 import torch
 
+from .. import _lib
 from ..gemv import (
     EPI_NONE,
     EPI_RESIDUAL,
@@ -273,6 +274,24 @@ def rmsnorm(x, w, eps=1e-6, out=None):
 
 def silu_mul(g, u, out=None):
     return _silu_mul(g, u, out)
+
+
+def step_tables(pad_lens, cache_position, mask_min, mask, position_ids, inv_freq, scaling, cos, sin):
+    """A decode step's additive mask [B, 1, 1, S] and rotary tables [B, 1, D]
+    from its device-side positions, in one launch (bz_step_tables)."""
+    B, S, D = mask.shape[0], mask.shape[-1], cos.shape[-1]
+    dt = {torch.bfloat16: _lib.DT_BF16, torch.float32: _lib.DT_F32}[mask.dtype]
+    for n, t, k, d in (("pad_lens", pad_lens, B, torch.int64), ("cache_position", cache_position, 1, torch.int64),
+                       ("position_ids", position_ids, B, torch.int64), ("inv_freq", inv_freq, D // 2, torch.float32),
+                       ("mask", mask, B * S, mask.dtype), ("cos", cos, B * D, mask.dtype), ("sin", sin, B * D, mask.dtype)):
+        if t.numel() != k or t.dtype != d or not t.is_contiguous() or t.device != mask.device or t.device.type != "cuda":
+            raise ValueError(f"{n} must be a contiguous {d} tensor of {k} entries on {mask.device}")
+    _lib.check(
+        _lib.lib().bz_step_tables(B, S, D, pad_lens.data_ptr(), cache_position.data_ptr(), mask_min, mask.data_ptr(),
+                                  position_ids.data_ptr(), inv_freq.data_ptr(), scaling, cos.data_ptr(), sin.data_ptr(),
+                                  dt, _lib.stream_of(mask)),
+        "bz_step_tables",
+    )
 
 
 def graph_time_us(fn, iters: int = 20, replays: int = 5) -> float:

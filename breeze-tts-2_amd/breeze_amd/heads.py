@@ -26,7 +26,7 @@ from torch import nn
 
 from . import _lib
 
-__all__ = ["head_f32", "Fp32Linear", "Fp32CodebooksHead", "install_fp32_heads"]
+__all__ = ["head_f32", "norm_head_f32", "Fp32Linear", "Fp32CodebooksHead", "install_fp32_heads"]
 
 
 def head_f32(x: torch.Tensor, w: torch.Tensor, *, index: Optional[torch.Tensor] = None, index_offset: int = 0,
@@ -58,6 +58,41 @@ def head_f32(x: torch.Tensor, w: torch.Tensor, *, index: Optional[torch.Tensor] 
                                None if index is None else index.data_ptr(), index_offset, out.data_ptr(),
                                out.stride(0), _lib.stream_of(x)),
         "bz_head_f32",
+    )
+    return out
+
+
+NORM_HEAD_MAX_ROWS = 4
+NORM_HEAD_MAX_K = 4096
+
+
+def norm_head_f32(x: torch.Tensor, gamma: torch.Tensor, eps: float, w: torch.Tensor, *, out: torch.Tensor,
+                  index: Optional[torch.Tensor] = None, index_offset: int = 0, normed: Optional[torch.Tensor] = None,
+                  cfg: Optional[torch.Tensor] = None, guidance: float = 1.0) -> torch.Tensor:
+    """The final RMSNorm of bf16 rows x [M, K] (M <= 4, K <= 4096) and
+    head_f32 of the result in one launch: out[M, N] fp32, the same bits as the
+    two calls.  normed [M, K] bf16 also receives the normed rows, cfg [M / 2
+    (or 1), N] the guidance combination of cond rows [0, M / 2) and uncond rows."""
+    if x.device.type != "cuda" or w.device != x.device:
+        raise RuntimeError("norm_head_f32 runs on the GPU (HIP kernel); the HIP path has no CPU fallback")
+    if w.dtype != torch.float32 or not w.is_contiguous():
+        raise ValueError("w must be a contiguous float32 tensor")
+    C, N, K = (w.shape if w.dim() == 3 else (1, *w.shape))
+    M = x.shape[0]
+    for n, t, shape, dt in (("x", x, (M, K), torch.bfloat16), ("gamma", gamma, (K,), torch.bfloat16),
+                            ("out", out, (M, N), torch.float32), ("normed", normed, (M, K), torch.bfloat16),
+                            ("cfg", cfg, (max(1, M // 2), N), torch.float32)):
+        if t is not None and (t.shape != shape or t.dtype != dt or t.stride(-1) != 1 or t.device != x.device):
+            raise ValueError(f"{n} must be a {dt} {list(shape)} tensor with unit column stride on {x.device}")
+    if index is not None and (index.dtype != torch.int64 or index.device != x.device):
+        raise ValueError("index must be an int64 tensor on the GPU")
+    ptr = lambda t: None if t is None else t.data_ptr()  # noqa: E731
+    ld = lambda t: 0 if t is None else t.stride(0)  # noqa: E731
+    _lib.check(
+        _lib.lib().bz_norm_head_f32(x.data_ptr(), x.stride(0), M, K, gamma.data_ptr(), eps, ptr(normed), ld(normed),
+                                    w.data_ptr(), N, N * K, C, ptr(index), index_offset, out.data_ptr(), out.stride(0),
+                                    ptr(cfg), ld(cfg), guidance, _lib.stream_of(x)),
+        "bz_norm_head_f32",
     )
     return out
 

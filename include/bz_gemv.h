@@ -354,6 +354,38 @@ int bz_head_f32(const float* x, int64_t ldx, int32_t M, int32_t K,
                 const int64_t* index, int64_t index_offset, float* out,
                 int64_t ldo, void* stream);
 
+/* The decoder's final RMSNorm, the fp32 head and the guidance combination of
+ * its logits in one launch, for M <= 4 bf16 rows: xn = bf16(x *
+ * rsqrt(mean(x^2) + eps) * gamma) as bz_rmsnorm gives it, out = xn W^T as
+ * bz_head_f32 gives it.  normed (optional, bf16 [M][ld_normed]) receives xn.
+ * cfg (optional, fp32 [max(1, M / 2)][ld_cfg]; M = 1 or even): row h is
+ * out[H + h] + guidance * (out[h] - out[H + h]) with H = M / 2, or out[0] for
+ * M = 1.  x, gamma and normed need no alignment beyond their type; W as for
+ * bz_head_f32.
+ * Replaces norm, lm_head and the CFG combination at the end of a step
+ * (models/cudagraph/backbone_graph.py:269-285) and norm + codebook head
+ * (models/cudagraph/depth_decoder_graph.py:594-600). */
+int bz_norm_head_f32(const void* x, int64_t ldx, int32_t M, int32_t K,
+                     const void* gamma, float eps, void* normed,
+                     int64_t ld_normed, const float* w, int32_t N,
+                     int64_t mat_stride, int32_t nmat, const int64_t* index,
+                     int64_t index_offset, float* out, int64_t ldo, float* cfg,
+                     int64_t ld_cfg, float guidance, void* stream);
+
+/* What a decode step reads of its position, in one launch: the additive mask
+ * rows mask[b][s] = (pad_lens[b] <= s <= *cache_pos) ? 0 : mask_min, s < S
+ * (contiguous rows), and the default rotary tables cos/sin[b][d] =
+ * cos/sin(fp32(positions[b]) * inv_freq[d % (D / 2)]) * scaling, d < D, B rows
+ * each (contiguous).  mask and tables bf16 (BZ_DT_BF16) or fp32 (BZ_DT_F32)
+ * by `dtype`; positions, pad_lens int64 [B]; inv_freq fp32 [D / 2].
+ * Replaces _set_attention_mask and the rotary embedding of a step
+ * (models/cudagraph/backbone_graph.py:240-252,262-266). */
+int bz_step_tables(int32_t B, int32_t S, int32_t D, const int64_t* pad_lens,
+                   const int64_t* cache_pos, float mask_min, void* mask,
+                   const int64_t* positions, const float* inv_freq,
+                   float scaling, void* cos_out, void* sin_out, int32_t dtype,
+                   void* stream);
+
 #ifdef __cplusplus
 }
 #endif

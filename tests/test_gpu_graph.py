@@ -164,3 +164,27 @@ def test_inductor_compile_then_graph_capture(quant):
     g.replay()
     torch.cuda.synchronize()
     assert torch.equal(out, compiled(x * 2))
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("B,S,D", [(1, 1, 2), (2, 257, 128), (3, 1024, 256), (2, 300, 514)])
+def test_step_tables(B, S, D, dt):
+    """The mask exactly; cos and sin of the same fp32 angle within one rounding
+    of the output type and 4 ulp of the fp32 functions."""
+    from breeze_amd.fused.kernels import step_tables
+
+    dev, low = "cuda", torch.finfo(dt).min
+    pad = torch.tensor([0, 3, S][:B], device=dev)
+    pos = torch.tensor([min(200, S - 1)], device=dev)
+    ids = torch.tensor([[7], [0], [40000]][:B], device=dev)
+    inv = 1.0 / 1e6 ** (torch.arange(0, D, 2, device=dev).float() / D)
+    mask = torch.full((B, 1, 1, S), 5.0, device=dev, dtype=dt)
+    cos, sin = (torch.full((B, 1, D), 5.0, device=dev, dtype=dt) for _ in range(2))
+    step_tables(pad, pos, low, mask, ids, inv, 1.5, cos, sin)
+    s = torch.arange(S, device=dev)
+    valid = (s >= pad.view(B, 1)) & (s <= pos)
+    assert torch.equal(mask.view(B, S), torch.where(valid, 0.0, low).to(dt))
+    a = (ids.view(B, 1).float() * inv).double().repeat(1, 2)
+    tol = 1.5 * (2.0 ** -8 if dt == torch.bfloat16 else 0.0) + 1.5 * 2.0 ** -21
+    for t, f in ((cos, torch.cos), (sin, torch.sin)):
+        assert float((t.view(B, D).double() - 1.5 * f(a)).abs().max()) <= tol

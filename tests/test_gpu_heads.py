@@ -120,3 +120,32 @@ def test_install_fp32_heads():
     assert isinstance(m.lm_head, Hd.Fp32Linear)
     assert isinstance(m.depth_decoder.codebooks_head, Hd.Fp32CodebooksHead)
     assert Hd.install_fp32_heads(m) == 0
+
+
+@pytest.mark.parametrize("M", [1, 2, 3, 4])
+@pytest.mark.parametrize("N,K", [(1, 4), (9, 252), (2051, 1024), (64, 1028), (2052, 2048), (17, 2052), (40, 4096)])
+def test_norm_head_equals_its_parts(M, N, K):
+    """norm_head_f32 against bz_rmsnorm, head_f32 and the guidance formula: the
+    same bits for the first two (edges of its 256-k pieces and of its two
+    instances), one rounding of the combination apart for the last."""
+    from breeze_amd.gemv import rmsnorm
+    from breeze_amd.heads import head_f32, norm_head_f32
+
+    g = torch.Generator(device="cuda").manual_seed(N + K + M)
+    x = torch.randn(M, K + 3, device="cuda", generator=g).to(torch.bfloat16)[:, 3:]
+    gamma = (1 + 0.1 * torch.randn(K, device="cuda", generator=g)).to(torch.bfloat16)
+    w = torch.randn(3, N, K, device="cuda", generator=g)
+    index = torch.tensor([2], device="cuda")
+    normed = torch.zeros(M, K, device="cuda", dtype=torch.bfloat16)
+    out = torch.zeros(M, N, device="cuda")
+    cfg = torch.zeros(max(1, M // 2), N, device="cuda") if M != 3 else None
+    norm_head_f32(x, gamma, 1e-6, w, out=out, index=index, index_offset=-1, normed=normed, cfg=cfg, guidance=1.5)
+    xn = rmsnorm(x, gamma, 1e-6)
+    want = head_f32(xn, w, index=index, index_offset=-1)
+    assert torch.equal(normed, xn)
+    assert torch.equal(out, want)
+    if cfg is not None:
+        h = max(1, M // 2)
+        ref = want if M == 1 else want[h:].double() + 1.5 * (want[:h].double() - want[h:].double())
+        mag = want.abs().max()
+        assert bool(((cfg.double() - ref).abs() <= 2.0 ** -22 * 4 * mag).all())
