@@ -53,6 +53,7 @@ EXPORTS = (
     "bz_attn_workspace",
     "bz_attn_default_split",
     "bz_sample_cfg",
+    "bz_sample_next",
     "bz_stream_read",
     "bz_shared_read",
 )
@@ -137,12 +138,12 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.bz_pack_tiled.argtypes = [i32, vp, vp, i32, i32, i32, i32, vp, i32, i32, vp]
     lib.bz_head_f32.restype = ctypes.c_int
     lib.bz_head_f32.argtypes = [vp, i64, i32, i32, vp, i32, i64, i32, vp, i64, vp, i64, vp]
-    lib.bz_qkv_rope_cache.restype = ctypes.c_int
     lib.bz_norm_head_f32.restype = ctypes.c_int
     lib.bz_norm_head_f32.argtypes = [vp, i64, i32, i32, vp, f32, vp, i64, vp, i32, i64, i32, vp, i64, vp, i64, vp, i64,
                                      f32, vp]
     lib.bz_step_tables.restype = ctypes.c_int
     lib.bz_step_tables.argtypes = [i32, i32, i32, vp, vp, f32, vp, vp, vp, f32, vp, vp, i32, vp]
+    lib.bz_qkv_rope_cache.restype = ctypes.c_int
     lib.bz_qkv_rope_cache.argtypes = [vp, i64, i32, i32, i32, i32, vp, vp, f32, vp, vp, i32, i64, vp, vp, vp, vp,
                                       i32, i32, vp, vp]
     lib.bz_attn_decode.restype = ctypes.c_int
@@ -161,6 +162,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.bz_shared_read.argtypes = [vp, ctypes.c_size_t, vp, ctypes.c_size_t, i32, ctypes.c_uint32, vp, vp]
     lib.bz_sample_cfg.restype = ctypes.c_int
     lib.bz_sample_cfg.argtypes = [vp, i64, i32, i32, i32, i32, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp]
+    lib.bz_sample_next.restype = ctypes.c_int
+    lib.bz_sample_next.argtypes = lib.bz_sample_cfg.argtypes[:-1] + [vp, i64, vp, i64, i64, i64, vp, i64, vp]
 
 
 def lib() -> ctypes.CDLL:

@@ -16,9 +16,12 @@ The depth layers are FusedDecoderLayer (install_fused_depth): their GEMVs and
 attention steps run on libbzgemv.so, the two-position start as two causal
 decode steps.  The codebook head is Fp32CodebooksHead (bz_head_f32), which
 picks the codebook's matrix on the GPU from the cache position.  Bias-free
-embedding projectors run as bf16 GEMVs and the final RMSNorm as bz_rmsnorm;
-the rotary tables of the frame's fixed positions are computed once; the
-embedding lookups are torch ops.
+embedding projectors run as bf16 GEMVs; the rotary tables of the frame's fixed
+positions are computed once.  Between the last layer of a step and the
+projector of the next lie two launches: the final RMSNorm with the codebook
+head (bz_norm_head_f32), and the sampler, which also writes the frame's token
+and gathers its embedding row (bz_sample_next); with more than 4 rows, another
+embedding module or the torch sampler they are separate launches and torch ops.
 
 CFG layout (models/cudagraph/depth_decoder_graph.py:487-558): rows [0, half)
 are the conditional rows and rows [half, 2 half) the unconditional ones; the
@@ -44,9 +47,9 @@ import torch
 from torch import nn
 from torch.nn import functional as F
 
-from ..heads import Fp32CodebooksHead
-from ..sampling import SampleState, sample_cfg
-from .install import static_cache
+from ..heads import NORM_HEAD_MAX_K, NORM_HEAD_MAX_ROWS, Fp32CodebooksHead, norm_head_f32
+from ..sampling import SampleState, sample_next
+from .install import static_cache, zero_cache
 from .kernels import FusedWeight, rms_gemv, rmsnorm
 
 __all__ = ["DepthDecodeGraph", "sampling_probs"]
@@ -162,6 +165,12 @@ class DepthDecodeGraph:
         nw, neps = getattr(dm.norm, "weight", None), getattr(dm.norm, "variance_epsilon", None)
         self._norm_w = None if nw is None or neps is None else nw.detach().to(torch.bfloat16).contiguous()
         self._norm_eps = None if neps is None else float(neps)
+        # the embedding rows the sampler can gather by itself: a plain table
+        emb = dm.embed_tokens
+        ew = emb.weight.detach() if type(emb) is nn.Embedding and emb.max_norm is None else None
+        self._emb_table = ew if (ew is not None and sampler == "hip" and ew.device == dev and ew.is_contiguous()
+                                 and ew.shape[0] >= self.num_codebooks * self.vocab_size
+                                 and ew.shape[1] * ew.element_size() % 16 == 0 and ew.data_ptr() % 16 == 0) else None
         with torch.no_grad():
             z = torch.zeros(1, 2, self.hidden_size, dtype=self.dtype, device=dev)
             self._pe_start = tuple(t.contiguous() for t in dm.rotary_emb(z, self.prefill_cache_pos.unsqueeze(0)))
@@ -187,6 +196,10 @@ class DepthDecodeGraph:
         self.first_cb_token_buf = torch.zeros(batch_size, dtype=torch.long, device=dev)
         self.output_tokens = torch.zeros(batch_size, self.num_decode_codebooks, dtype=torch.long, device=dev)
         self._tok_buf = torch.zeros(batch_size, dtype=torch.long, device=dev)
+        self._emb_buf = (None if self._emb_table is None else
+                         torch.zeros(batch_size, self._emb_table.shape[1], dtype=self._emb_table.dtype, device=dev))
+        self._norm_head = (self._norm_w is not None and dt == torch.bfloat16 and batch_size <= NORM_HEAD_MAX_ROWS
+                           and self.hidden_size <= NORM_HEAD_MAX_K)
         self.prefill_input_ids = torch.zeros(batch_size, 2, dtype=torch.long, device=dev)
         d = self._defaults
         self.temperature_buf = torch.full((self.half, 1), d["temperature"], dtype=torch.float32, device=dev)
@@ -214,12 +227,7 @@ class DepthDecodeGraph:
 
     def reset_cache(self) -> None:
         """Zero the cache and its fill counters (outside any capture)."""
-        for layer in self.static_cache.layers:
-            if getattr(layer, "is_initialized", False):
-                layer.keys.zero_()
-                layer.values.zero_()
-                if isinstance(getattr(layer, "cumulative_length", None), torch.Tensor):
-                    layer.cumulative_length.zero_()
+        zero_cache(self.static_cache)
 
     # -- the loop -------------------------------------------------------------------
 
@@ -229,9 +237,18 @@ class DepthDecodeGraph:
             h = layer(h, attention_mask=mask, position_ids=pos_ids, past_key_values=self.static_cache,
                       use_cache=True, cache_position=cache_pos, position_embeddings=pos_emb)
             h = h[0] if isinstance(h, tuple) else h
-        if self._norm_w is None:
-            return self.depth_model.norm(h)
-        return rmsnorm(h.reshape(-1, h.shape[-1]), self._norm_w, self._norm_eps).reshape(h.shape)
+        return h
+
+    def _logits(self, h, cache_pos):
+        """Final norm and codebook head of the last position: [B, vocab] fp32."""
+        h = h[:, -1, :]
+        head = self.codebooks_head
+        if self._norm_head and h.dtype == torch.bfloat16:
+            out = torch.empty(h.shape[0], head.vocab_size, device=h.device, dtype=torch.float32)
+            return norm_head_f32(h, self._norm_w, self._norm_eps, head.weight_t, out=out, index=cache_pos,
+                                 index_offset=-1)
+        h = self.depth_model.norm(h) if self._norm_w is None else rmsnorm(h, self._norm_w, self._norm_eps)
+        return head(h.unsqueeze(1), cache_position=cache_pos)[:, 0, :]
 
     def reseed(self, seed: int) -> None:
         """New key for the HIP sampler's stream, draw counters back to zero
@@ -240,24 +257,29 @@ class DepthDecodeGraph:
         if self._sample_state is not None:
             self._sample_state.reseed(self._seed)
 
-    def _cfg_sample(self, logits: torch.Tensor, i: int) -> None:
-        """Combined logits of codebook step i -> self._tok_buf (both halves)."""
+    def _cfg_sample(self, logits: torch.Tensor, i: int) -> bool:
+        """Combined logits of codebook step i -> self._tok_buf (both halves)
+        and the frame's tokens; True when the next step's embedding rows are
+        in self._emb_buf too."""
         if self._sample_state is not None:
-            # one launch (bz_sample_cfg): the same filter, its own Philox stream
-            sample_cfg(logits[:, 0, :], self._tok_buf, self._sample_state,
-                       temperature=self.temperature_buf.view(-1), top_k=self.top_k_buf.view(-1),
-                       top_p=self.top_p_buf.view(-1), do_sample=self.do_sample_buf,
-                       guidance=self.guidance_scale.view(-1) if self.batch_size >= 2 else None,
-                       codec_size=self.codec_codebook_size, max_k=self._max_k,
-                       cfg_out=None if self.debug_logits is None else self.debug_logits[i],
-                       probs_out=None if self.debug_probs is None else self.debug_probs[i])
-            return
+            # one launch: the same filter, its own Philox stream
+            kw = dict(temperature=self.temperature_buf.view(-1), top_k=self.top_k_buf.view(-1),
+                      top_p=self.top_p_buf.view(-1), do_sample=self.do_sample_buf,
+                      guidance=self.guidance_scale.view(-1) if self.batch_size >= 2 else None,
+                      codec_size=self.codec_codebook_size, max_k=self._max_k,
+                      cfg_out=None if self.debug_logits is None else self.debug_logits[i],
+                      probs_out=None if self.debug_probs is None else self.debug_probs[i])
+            gather = self._emb_table is not None and i + 1 < self.num_decode_codebooks
+            sample_next(logits, self._tok_buf, self._sample_state, out_tokens=self.output_tokens[:, i],
+                        table=self._emb_table if gather else None, first_row=(i + 1) * self.vocab_size,
+                        emb=self._emb_buf if gather else None, **kw)
+            return gather
         half = self.half
         if self.batch_size >= 2:
-            cond, uncond = logits[:half, 0, :], logits[half: 2 * half, 0, :]
+            cond, uncond = logits[:half], logits[half: 2 * half]
             cfg = uncond + self.guidance_scale * (cond - uncond)
         else:
-            cfg = logits[:half, 0, :].clone()
+            cfg = logits[:half].clone()
         if self.codec_codebook_size < self.vocab_size:
             cfg[:, self.codec_codebook_size: self.vocab_size] = float("-inf")
         if self.debug_logits is not None:
@@ -271,6 +293,9 @@ class DepthDecodeGraph:
         self._tok_buf[:half] = toks
         if self.batch_size >= 2:
             self._tok_buf[half: 2 * half] = toks
+        self._tok_buf.clamp_(0, self.vocab_size - 1)
+        self.output_tokens[:, i] = self._tok_buf
+        return False
 
     def _full_loop(self) -> None:
         """The whole frame on static buffers (graph-safe: no host sync)."""
@@ -284,20 +309,17 @@ class DepthDecodeGraph:
         emb[:, 0] = bh
         h = self._inputs_proj(emb)  # [B, 2, hidden]
         h = self._layers(h, self.prefill_attn, self.prefill_cache_pos, self._pe_start)
-        logits = self.codebooks_head(h[:, 1:, :], cache_position=self.head_prefill_pos)  # [B, 1, vocab] fp32
-        self._cfg_sample(logits, 0)
-        self._tok_buf.clamp_(0, self.vocab_size - 1)
-        self.output_tokens[:, 0] = self._tok_buf
+        gathered = self._cfg_sample(self._logits(h, self.head_prefill_pos), 0)
         top = self.num_codebooks * self.vocab_size - 1
         for i in range(1, self.num_decode_codebooks):
-            tok = (self._tok_buf + self.codebook_offsets[i]).unsqueeze(1).clamp_(0, top)
-            h = self._inputs_proj(dm.embed_tokens(tok))  # [B, 1, hidden]
+            if gathered:
+                emb = self._emb_buf.unsqueeze(1)
+            else:
+                emb = dm.embed_tokens((self._tok_buf + self.codebook_offsets[i]).unsqueeze(1).clamp_(0, top))
+            h = self._inputs_proj(emb)  # [B, 1, hidden]
             cache_pos = self.decode_cache_positions[i - 1]
             h = self._layers(h, self.decode_attn[i - 1], cache_pos, self._pe_decode[i - 1])
-            logits = self.codebooks_head(h, cache_position=cache_pos)
-            self._cfg_sample(logits, i)
-            self._tok_buf.clamp_(0, self.vocab_size - 1)
-            self.output_tokens[:, i] = self._tok_buf
+            gathered = self._cfg_sample(self._logits(h, cache_pos), i)
 
     # -- capture / run ----------------------------------------------------------------
 

@@ -19,7 +19,7 @@ import torch
 
 from . import _lib
 
-__all__ = ["sample_cfg", "SampleState", "MAX_VOCAB", "MAX_TOP_K"]
+__all__ = ["sample_cfg", "sample_next", "SampleState", "MAX_VOCAB", "MAX_TOP_K"]
 
 MAX_VOCAB = 4096
 MAX_TOP_K = 1024
@@ -56,6 +56,15 @@ def sample_cfg(logits: torch.Tensor, tokens: torch.Tensor, state: SampleState, *
     Per-row parameters: temperature / top_p fp32, top_k / do_sample int64,
     guidance fp32 (B >= 2), half entries each.  max_k is the top-k workspace
     (top_k <= 0 means all of it), at most min(V, 1024)."""
+    args = _sample_args(logits, tokens, state, temperature, top_k, top_p, do_sample, guidance, codec_size, max_k,
+                        cfg_out, probs_out)
+    _lib.check(_lib.lib().bz_sample_cfg(*args, _lib.stream_of(logits)), "bz_sample_cfg")
+    return tokens
+
+
+def _sample_args(logits, tokens, state, temperature, top_k, top_p, do_sample, guidance, codec_size, max_k, cfg_out,
+                 probs_out) -> tuple:
+    """The checked arguments of bz_sample_cfg, without the stream."""
     if logits.device.type != "cuda":
         raise RuntimeError("sample_cfg runs on the GPU (HIP kernel); there is no CPU fallback")
     dev = logits.device
@@ -86,11 +95,41 @@ def sample_cfg(logits: torch.Tensor, tokens: torch.Tensor, state: SampleState, *
         if t is not None:
             _dev(n, t, torch.float32, dev, half * V)
     ptr = lambda t: None if t is None else t.data_ptr()  # noqa: E731
+    return (logits.data_ptr(), logits.stride(0), B, V, codec, max_k, ptr(guidance), temperature.data_ptr(),
+            top_k.data_ptr(), top_p.data_ptr(), do_sample.data_ptr(), state.seed.data_ptr(), state.counters.data_ptr(),
+            tokens.data_ptr(), ptr(cfg_out), ptr(probs_out))
+
+
+def sample_next(logits: torch.Tensor, tokens: torch.Tensor, state: SampleState, *, out_tokens: torch.Tensor,
+                table: Optional[torch.Tensor] = None, first_row: int = 0, emb: Optional[torch.Tensor] = None,
+                temperature: torch.Tensor, top_k: torch.Tensor, top_p: torch.Tensor, do_sample: torch.Tensor,
+                guidance: Optional[torch.Tensor] = None, codec_size: Optional[int] = None, max_k: int = MAX_TOP_K,
+                cfg_out: Optional[torch.Tensor] = None, probs_out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """sample_cfg, and what a frame's next step reads of the token in the same
+    launch: every row's token to out_tokens (int64 [B], any stride >= 1) and,
+    with a table [R, C], its row first_row + token (at most R - 1) to emb [B, C]
+    (rows of a multiple of 16 bytes, both contiguous)."""
+    args = _sample_args(logits, tokens, state, temperature, top_k, top_p, do_sample, guidance, codec_size, max_k,
+                        cfg_out, probs_out)
+    B, dev = logits.shape[0], logits.device
+    if out_tokens.device != dev or out_tokens.dtype != torch.int64 or out_tokens.shape != (B,):
+        raise ValueError(f"out_tokens must be an int64 [{B}] tensor on {dev}")
+    if B > 1 and out_tokens.stride(0) < 1:
+        raise ValueError("out_tokens needs a positive stride")
+    row = 0
+    if table is not None:
+        if emb is None or table.dim() != 2 or emb.shape != (B, table.shape[1]) or emb.dtype != table.dtype:
+            raise ValueError("emb must be [B, C] of the table's dtype")
+        if table.device != dev or emb.device != dev or not table.is_contiguous() or not emb.is_contiguous():
+            raise ValueError(f"table and emb must be contiguous tensors on {dev}")
+        if first_row < 0:
+            raise ValueError("first_row must not be negative")
+        row = table.shape[1] * table.element_size()
     _lib.check(
-        _lib.lib().bz_sample_cfg(logits.data_ptr(), logits.stride(0), B, V, codec, max_k, ptr(guidance),
-                                 temperature.data_ptr(), top_k.data_ptr(), top_p.data_ptr(), do_sample.data_ptr(),
-                                 state.seed.data_ptr(), state.counters.data_ptr(), tokens.data_ptr(),
-                                 ptr(cfg_out), ptr(probs_out), _lib.stream_of(logits)),
-        "bz_sample_cfg",
+        _lib.lib().bz_sample_next(*args, out_tokens.data_ptr(), out_tokens.stride(0) if B > 1 else 1,
+                                  None if table is None else table.data_ptr(), 0 if table is None else table.shape[0],
+                                  row, first_row, None if table is None else emb.data_ptr(), row,
+                                  _lib.stream_of(logits)),
+        "bz_sample_next",
     )
     return tokens

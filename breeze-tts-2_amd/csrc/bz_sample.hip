@@ -26,7 +26,11 @@
 //      kept rank whose cumulative weight exceeds u times the kept total;
 //   5. the token (sampled, or the argmax when do_sample is 0) to the row and
 //      its unconditional twin; the row's call count is advanced, so graph
-//      replays draw fresh numbers.
+//      replays draw fresh numbers;
+//   6. bz_sample_next only: the token also to a column of the frame's tokens,
+//      and its row of the embedding table to the next step's input (that
+//      replaced a clamp, a copy, an offset add, a clamp and an index-select
+//      launch of about 2.5 us each).
 // A greedy row that reports no probabilities stops after step 1.
 //
 // The random stream is this library's own, not torch's: the sampled tokens
@@ -78,6 +82,12 @@ struct SampleParams {
     int64_t* tokens;
     float* cfg_out;
     float* probs_out;
+    int64_t* out_tokens;  // optional: [B] with stride out_ld
+    int64_t out_ld;
+    const uint8_t* table;  // optional: embedding rows of row_bytes
+    int64_t table_rows, row_bytes, first_row;
+    uint8_t* emb;          // [B] rows, emb_ld bytes apart
+    int64_t emb_ld;
 };
 
 // Sort key of a row entry: the temperature-scaled value mapped to an
@@ -124,13 +134,38 @@ __device__ __forceinline__ int value_bucket(float s, float top, float scale) {
     return min((int)((top - s) * scale), kBuckets - 1);
 }
 
-// The row's token, in one wave: to the row and its twin; the row's call
-// count advances.
-__device__ __forceinline__ void put_token(const SampleParams& p, int r, int tok, uint64_t cnt) {
+// The row's token, by one whole wave: to the row and its twin, and what the
+// next step reads of it; the row's call count advances.
+__device__ __forceinline__ void put_token(const SampleParams& p, int r, int tok, uint64_t cnt, int lane) {
     tok = tok < 0 ? 0 : (tok >= p.V ? p.V - 1 : tok);
-    p.tokens[r] = tok;
-    if (p.B >= 2) p.tokens[p.half + r] = tok;
-    p.counters[r] = cnt + 1;
+    const bool twin = p.B >= 2;
+    if (lane == 0) {
+        p.tokens[r] = tok;
+        if (twin) p.tokens[p.half + r] = tok;
+        p.counters[r] = cnt + 1;
+        if (p.out_tokens) {
+            p.out_tokens[r * p.out_ld] = tok;
+            if (twin) p.out_tokens[(p.half + r) * p.out_ld] = tok;
+        }
+    }
+    if (!p.table) return;
+    const int64_t row = min<int64_t>(max<int64_t>(p.first_row + tok, 0), p.table_rows - 1);
+    const uint8_t* src = p.table + row * p.row_bytes;
+    uint8_t* d0 = p.emb + r * p.emb_ld;
+    uint8_t* d1 = p.emb + (p.half + r) * p.emb_ld;
+    for (int64_t o0 = lane * 16; o0 < p.row_bytes; o0 += 4096) {  // four loads in flight: 4 KiB a turn
+        u32x4 v[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = ldg16(src + min<int64_t>(o0 + 1024 * i, p.row_bytes - 16));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int64_t o = o0 + 1024 * i;
+            if (o < p.row_bytes) {
+                *reinterpret_cast<u32x4*>(d0 + o) = v[i];
+                if (twin) *reinterpret_cast<u32x4*>(d1 + o) = v[i];
+            }
+        }
+    }
 }
 
 // Reductions over 16-lane rows and the wave in DPP moves: a step is one VALU
@@ -260,7 +295,7 @@ __device__ __forceinline__ void select_general(SampleShared& sh, const uint64_t 
 // requested together, reductions stay in DPP moves, and the chain of barriers
 // and LDS round trips is short.  Measured on MI355X in a graph of 16 launches,
 // V = 2051, B = 2, with probs_out: 14.6 us a launch with the radix select and
-// shuffle reductions for every row, 6.0 us now (top_k = 50); 20.8 and 8.6 us
+// shuffle reductions for every row, 6.0 us now (top_k = 50); 20.8 and 7.9 us
 // at top_k = 1000.
 __global__ void __launch_bounds__(kSampleThreads) sample_cfg_kernel(SampleParams p) {
     __shared__ SampleShared sh;
@@ -363,7 +398,7 @@ __global__ void __launch_bounds__(kSampleThreads) sample_cfg_kernel(SampleParams
     // A greedy row with no probabilities to report needs only the argmax:
     // skip the order, softmax and draw; the call count advances all the same.
     if (!sample && !p.probs_out) {
-        if (tid == 0) put_token(p, r, greedy, cnt);
+        if (wave == 0) put_token(p, r, greedy, cnt, lane);
         return;
     }
 
@@ -457,7 +492,7 @@ __global__ void __launch_bounds__(kSampleThreads) sample_cfg_kernel(SampleParams
         // the first kept rank past the draw; rounding at the top end: the last kept one
         const int at = over ? __ffsll((unsigned long long)over) - 1
                             : (any ? 63 - __clzll((long long)any) : 0);
-        if (lane == at) put_token(p, r, sample ? si_t : greedy, cnt);
+        put_token(p, r, sample ? __builtin_amdgcn_readlane(si_t, at) : greedy, cnt, lane);
         return;
     }
     if (lane == 63) sh.wsum[wave] = inc;
@@ -486,7 +521,10 @@ __global__ void __launch_bounds__(kSampleThreads) sample_cfg_kernel(SampleParams
         if (over) atomicMin(&sh.pick, tid + __ffsll((unsigned long long)over) - 1);
     }
     __syncthreads();
-    if (tid == (sh.pick == 0x7FFFFFFF ? sh.last_kept : sh.pick)) put_token(p, r, sample ? si_t : greedy, cnt);
+    if (wave == 0) {
+        const int at = sh.pick == 0x7FFFFFFF ? sh.last_kept : sh.pick;
+        put_token(p, r, sample ? key_index(sh.sorted[at]) : greedy, cnt, lane);
+    }
 }
 
 }  // namespace
@@ -494,16 +532,16 @@ __global__ void __launch_bounds__(kSampleThreads) sample_cfg_kernel(SampleParams
 
 using namespace bz;
 
-extern "C" int bz_sample_cfg(const float* logits, int64_t ld_logits, int32_t B, int32_t V, int32_t codec_size,
-                             int32_t max_k, const float* guidance, const float* temperature, const int64_t* top_k,
-                             const float* top_p, const int64_t* do_sample, const uint64_t* seed, uint64_t* counters,
-                             int64_t* tokens, float* cfg_out, float* probs_out, void* stream) {
+static int fill_params(SampleParams& p, const float* logits, int64_t ld_logits, int32_t B, int32_t V, int32_t codec_size,
+                       int32_t max_k, const float* guidance, const float* temperature, const int64_t* top_k,
+                       const float* top_p, const int64_t* do_sample, const uint64_t* seed, uint64_t* counters,
+                       int64_t* tokens, float* cfg_out, float* probs_out) {
     if (!logits || !temperature || !top_k || !top_p || !do_sample || !seed || !counters || !tokens)
         return BZ_ERR_INVALID_ARG;
     if (B < 1 || (B > 1 && B % 2) || V < 1 || V > kSampleWidth || ld_logits < V) return BZ_ERR_INVALID_ARG;
     if (codec_size < 1 || codec_size > V || max_k < 1 || max_k > kSampleMaxK || max_k > V) return BZ_ERR_INVALID_ARG;
     if (B >= 2 && !guidance) return BZ_ERR_INVALID_ARG;
-    SampleParams p;
+    p = SampleParams{};
     p.logits = logits;
     p.ld = ld_logits;
     p.B = B;
@@ -521,6 +559,47 @@ extern "C" int bz_sample_cfg(const float* logits, int64_t ld_logits, int32_t B, 
     p.tokens = tokens;
     p.cfg_out = cfg_out;
     p.probs_out = probs_out;
+    return BZ_OK;
+}
+
+static int launch(const SampleParams& p, void* stream) {
     hipLaunchKernelGGL(sample_cfg_kernel, dim3(p.half), dim3(kSampleThreads), 0, static_cast<hipStream_t>(stream), p);
     return hipGetLastError() == hipSuccess ? BZ_OK : BZ_ERR_LAUNCH;
+}
+
+extern "C" int bz_sample_cfg(const float* logits, int64_t ld_logits, int32_t B, int32_t V, int32_t codec_size,
+                             int32_t max_k, const float* guidance, const float* temperature, const int64_t* top_k,
+                             const float* top_p, const int64_t* do_sample, const uint64_t* seed, uint64_t* counters,
+                             int64_t* tokens, float* cfg_out, float* probs_out, void* stream) {
+    SampleParams p;
+    const int rc = fill_params(p, logits, ld_logits, B, V, codec_size, max_k, guidance, temperature, top_k, top_p,
+                               do_sample, seed, counters, tokens, cfg_out, probs_out);
+    return rc == BZ_OK ? launch(p, stream) : rc;
+}
+
+extern "C" int bz_sample_next(const float* logits, int64_t ld_logits, int32_t B, int32_t V, int32_t codec_size,
+                              int32_t max_k, const float* guidance, const float* temperature, const int64_t* top_k,
+                              const float* top_p, const int64_t* do_sample, const uint64_t* seed, uint64_t* counters,
+                              int64_t* tokens, float* cfg_out, float* probs_out, int64_t* out_tokens, int64_t out_ld,
+                              const void* table, int64_t table_rows, int64_t row_bytes, int64_t first_row, void* emb,
+                              int64_t emb_ld, void* stream) {
+    SampleParams p;
+    const int rc = fill_params(p, logits, ld_logits, B, V, codec_size, max_k, guidance, temperature, top_k, top_p,
+                               do_sample, seed, counters, tokens, cfg_out, probs_out);
+    if (rc != BZ_OK) return rc;
+    if (out_tokens && out_ld < 1) return BZ_ERR_INVALID_ARG;
+    if (table) {
+        if (!emb || table_rows < 1 || row_bytes < 16 || first_row < 0) return BZ_ERR_INVALID_ARG;
+        if (row_bytes % 16 || emb_ld % 16 || emb_ld < row_bytes) return BZ_ERR_SHAPE;
+        if ((reinterpret_cast<uintptr_t>(table) | reinterpret_cast<uintptr_t>(emb)) & 15) return BZ_ERR_ALIGNMENT;
+    }
+    p.out_tokens = out_tokens;
+    p.out_ld = out_ld;
+    p.table = static_cast<const uint8_t*>(table);
+    p.table_rows = table_rows;
+    p.row_bytes = row_bytes;
+    p.first_row = first_row;
+    p.emb = static_cast<uint8_t*>(emb);
+    p.emb_ld = emb_ld;
+    return launch(p, stream);
 }

@@ -33,6 +33,22 @@ int bz_sample_cfg(const float* logits, int64_t ld_logits, int32_t B, int32_t V,
                   uint64_t* counters, int64_t* tokens, float* cfg_out,
                   float* probs_out, void* stream);
 
+/* bz_sample_cfg, and what the next step of a frame reads of the token, in the
+ * same launch: the token of row b (twins included) to out_tokens[b * out_ld]
+ * (out_tokens NULL: not), and row min(first_row + token, table_rows - 1) of
+ * `table` (rows of row_bytes, contiguous; NULL: not) to emb + b * emb_ld.
+ * row_bytes and emb_ld are multiples of 16, table and emb 16-byte aligned.
+ * Replaces the token clamp, codebook offset and embedding lookup between two
+ * steps (models/cudagraph/depth_decoder_graph.py:615-638). */
+int bz_sample_next(const float* logits, int64_t ld_logits, int32_t B, int32_t V,
+                   int32_t codec_size, int32_t max_k, const float* guidance,
+                   const float* temperature, const int64_t* top_k,
+                   const float* top_p, const int64_t* do_sample, const uint64_t* seed,
+                   uint64_t* counters, int64_t* tokens, float* cfg_out,
+                   float* probs_out, int64_t* out_tokens, int64_t out_ld,
+                   const void* table, int64_t table_rows, int64_t row_bytes,
+                   int64_t first_row, void* emb, int64_t emb_ld, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -250,3 +250,32 @@ def test_rows_with_infinities_stay_in_range(kind):
     sample_cfg(row.view(1, V), tokens, SampleState(1, DEV, seed=5), **prm)
     torch.cuda.synchronize()
     assert 0 <= int(tokens[0]) < V
+
+
+@pytest.mark.parametrize("B", [1, 2, 6])
+@pytest.mark.parametrize("width", [8, 512, 2048, 2056, 5000])
+def test_next_step_inputs(B, width):
+    """sample_next: the tokens of sample_cfg, in the frame's column too, and
+    their embedding rows (one 16-byte piece, the 4 KiB turn, past it), the
+    table's last row where first_row + token leaves it."""
+    from breeze_amd.sampling import sample_next
+
+    V, half = 300, max(1, B // 2)
+    gen = torch.Generator(device=DEV).manual_seed(B + width)
+    logits = torch.randn(B, V, device=DEV, generator=gen)
+    table = torch.randn(2 * V, width, device=DEV, generator=gen).to(torch.bfloat16)
+    for do_sample in (0, 1):
+        for first in (0, V, 2 * V - 5):
+            prm = _params(half, top_k=20, do_sample=do_sample)
+            if B == 1:
+                prm["guidance"] = None
+            want = torch.zeros(B, dtype=torch.int64, device=DEV)
+            sample_cfg(logits, want, SampleState(half, DEV, seed=9), **prm)
+            frame = torch.full((B, 3), -1, dtype=torch.int64, device=DEV)
+            got, emb = torch.zeros_like(want), torch.zeros(B, width, dtype=torch.bfloat16, device=DEV)
+            sample_next(logits, got, SampleState(half, DEV, seed=9), out_tokens=frame[:, 1], table=table,
+                        first_row=first, emb=emb, **prm)
+            torch.cuda.synchronize()
+            assert torch.equal(got, want) and torch.equal(frame[:, 1], want)
+            assert bool((frame[:, [0, 2]] == -1).all())
+            assert torch.equal(emb, table[(want + first).clamp(max=2 * V - 1)])
