@@ -9,6 +9,7 @@ mirror the reference's separate rope/cache and attention kernels.
 
 from __future__ import annotations
 
+import functools
 from typing import Optional
 
 import torch
@@ -22,6 +23,8 @@ _DT = {torch.bfloat16: DT_BF16, torch.float32: DT_F32}
 
 
 def _gpu(name: str, t: torch.Tensor, dev: torch.device) -> None:
+    if t.get_device() == dev.index:  # (-1 on the CPU)
+        return
     if t.device.type != "cuda":
         raise RuntimeError(f"{name} must be a GPU tensor (got {t.device}); the HIP path has no CPU fallback")
     if t.device != dev:
@@ -38,7 +41,7 @@ def _dtype_code(name: str, t: torch.Tensor) -> int:
 def _rows(t: torch.Tensor, B: int, name: str) -> tuple[torch.Tensor, int]:
     """(B or 1, ...) -> a [rows, n] view with unit column stride and its row
     stride (0 when one row serves every batch row)."""
-    t2 = t.reshape(t.shape[0], -1)
+    t2 = t if t.dim() == 2 else t.reshape(t.shape[0], -1)
     if t2.stride(1) != 1:
         t2 = t2.contiguous()
     if t2.shape[0] == B:
@@ -48,10 +51,12 @@ def _rows(t: torch.Tensor, B: int, name: str) -> tuple[torch.Tensor, int]:
     raise ValueError(f"{name} has {t2.shape[0]} rows for a batch of {B}")
 
 
+@functools.lru_cache(maxsize=256)
 def default_split(S: int) -> int:
     return int(_lib.lib().bz_attn_default_split(S))
 
 
+@functools.lru_cache(maxsize=1024)
 def attn_workspace_bytes(B: int, HQ: int, HKV: int, D: int, split: int) -> int:
     return int(_lib.lib().bz_attn_workspace(B, HQ, HKV, D, split))
 
@@ -215,8 +220,8 @@ def attention_step(qkv, cos, sin, cache_position, keys, values, mask, q_norm_w=N
         raise ValueError("cos and sin must share shape, layout and dtype, with D columns")
     qn = kn = None
     if q_norm_w is not None:
-        qn = q_norm_w.to(torch.bfloat16).contiguous()
-        kn = k_norm_w.to(torch.bfloat16).contiguous()
+        qn, kn = (w if w.dtype == torch.bfloat16 and w.is_contiguous() else w.to(torch.bfloat16).contiguous()
+                  for w in (q_norm_w, k_norm_w))
     if seq_len is not None:
         _gpu("seq_len", seq_len, dev)
         if seq_len.dtype != torch.int64 or seq_len.numel() != 1:
@@ -225,7 +230,8 @@ def attention_step(qkv, cos, sin, cache_position, keys, values, mask, q_norm_w=N
             raise ValueError("seq_len must not alias cache_position")
     m2, mcode, ld_mask = _mask_rows(mask, B, S)
     split = default_split(S) if split is None else split
-    ws = _attn_workspace(B, HQ, HKV, D, split, dev, _lib.stream_of(qkv))
+    stream = _lib.stream_of(qkv)
+    ws = _attn_workspace(B, HQ, HKV, D, split, dev, stream)
     out = _out_buffer(out, B, HQ, D, dev)
     _lib.check(
         _lib.lib().bz_attn_step(
@@ -233,7 +239,7 @@ def attention_step(qkv, cos, sin, cache_position, keys, values, mask, q_norm_w=N
             None if kn is None else kn.data_ptr(), eps, cos2.data_ptr(), sin2.data_ptr(), _dtype_code("cos", cos2),
             ld_cs, cache_position.data_ptr(), keys.data_ptr(), values.data_ptr(), S, _dtype_code("keys", keys),
             None if seq_len is None else seq_len.data_ptr(), m2.data_ptr(), mcode, ld_mask, D ** -0.5, split,
-            None if ws is None else ws.data_ptr(), out.data_ptr(), out.stride(0), _lib.stream_of(qkv)),
+            None if ws is None else ws.data_ptr(), out.data_ptr(), out.stride(0), stream),
         "bz_attn_step",
     )
     return out

@@ -39,7 +39,7 @@ import torch
 from torch import nn
 
 from ._swap import swap_linears
-from .gemv import (W_FP8, W_FP8_TILED, dequant_matmul, gemv_traceable, pack_tiled, quantize_fp8_device,
+from .gemv import (W_FP8, W_FP8_TILED, dequant_matmul, gemv, gemv_traceable, pack_tiled, quantize_fp8_device,
                    tiled_bytes)
 
 # Max representable magnitude of float8_e4m3fn.
@@ -138,21 +138,27 @@ class Fp8Linear(nn.Module):
         return self._padded, k16
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
+        # (views and casts that change nothing are skipped, as in Int4Linear)
         shape = x.shape
-        flat = x.reshape(-1, shape[-1]).to(torch.bfloat16)
-        N, K = self.out_features, self.in_features
-        if layout_of(self.weight_fp8, N, K) == LAYOUT_TILED:
-            w = self.weight_fp8.view(torch.uint8)
-            if flat.shape[0] > PREFILL_ROWS and not torch.compiler.is_compiling():
+        flat = x if x.dim() == 2 else x.reshape(-1, shape[-1])
+        if flat.dtype != torch.bfloat16:
+            flat = flat.to(torch.bfloat16)
+        w, N, K = self.weight_fp8, self.out_features, self.in_features
+        if layout_of(w, N, K) == LAYOUT_TILED:
+            if torch.compiler.is_compiling():
+                out = gemv_traceable(flat, w.view(torch.uint8), W_FP8_TILED, N)
+            elif flat.shape[0] > PREFILL_ROWS:
                 out = dequant_matmul(flat, w, W_FP8_TILED, N, K)
             else:
-                out = gemv_traceable(flat, w, W_FP8_TILED, N)
-            return out.to(x.dtype).reshape(*shape[:-1], N)
-        codes, k = self._gemv_codes()
-        if k != K:
-            flat = torch.nn.functional.pad(flat, (0, k - K))
-        out = gemv_traceable(flat, codes, W_FP8, N, sc0=self.weight_scale)
-        return out.to(x.dtype).reshape(*shape[:-1], N)
+                out = gemv(flat, w, W_FP8_TILED, N)
+        else:
+            codes, k = self._gemv_codes()
+            if k != K:
+                flat = torch.nn.functional.pad(flat, (0, k - K))
+            out = gemv_traceable(flat, codes, W_FP8, N, sc0=self.weight_scale)
+        if x.dtype != torch.bfloat16:
+            out = out.to(x.dtype)
+        return out if x.dim() == 2 else out.reshape(*shape[:-1], N)
 
     def extra_repr(self) -> str:
         return f"in_features={self.in_features}, out_features={self.out_features}, fp8=True"

@@ -15,6 +15,7 @@ graphs (no allocation, sync or tuning inside the library call).
 from __future__ import annotations
 
 import ctypes
+import functools
 from typing import Optional
 
 import torch
@@ -64,6 +65,7 @@ __all__ = [
 TILED_FORMATS = (W_INT4_TILED, W_INT4_TILED_PAIRED, W_FP8_TILED, W_FP8_TILED_PAIRED)
 
 _DT = {torch.bfloat16: DT_BF16, torch.float32: DT_F32}
+_NO_CFG = (0, 0, 0, 0, 0)
 
 
 def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
@@ -71,6 +73,8 @@ def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
 
 
 def _require_gpu(name: str, t: torch.Tensor, device: torch.device) -> None:
+    if t.get_device() == device.index:  # (-1 on the CPU)
+        return
     if t.device.type != "cuda":
         raise RuntimeError(f"{name} must be a GPU tensor (got {t.device}); the HIP path has no CPU fallback")
     if t.device != device:
@@ -129,7 +133,8 @@ def gemv(
     x = _rows_aligned(x)
     if gamma is not None:
         _require_gpu("gamma", gamma, dev)
-        gamma = gamma.to(torch.bfloat16).contiguous()
+        if gamma.dtype != torch.bfloat16 or not gamma.is_contiguous():
+            gamma = gamma.to(torch.bfloat16).contiguous()
         if gamma.numel() != K:
             raise ValueError(f"gamma has {gamma.numel()} elements, K = {K}")
     res_dt = DT_BF16
@@ -161,43 +166,35 @@ def gemv(
     _check_weight(w, wfmt, n, K, group, sc0, sc1)
     if M == 0:  # no rows: the empty result, nothing launched (the library rejects M = 0)
         return out
-    d = _lib.GemvDesc()
-    d.abi_version = _lib.ABI_VERSION
-    d.M, d.N, d.K = M, n, K
-    d.group = group
-    d.wfmt = wfmt
-    d.epilogue = epilogue
-    d.out_dtype = _DT[out.dtype]
-    d.residual_dtype = res_dt
-    cfg = (tuple(cfg) + (0, 0, 0, 0, 0))[:5]
-    if cfg == (0, 0, 0, 0, 0):
-        found = _tuning.lookup(dev, n, K, wfmt, epilogue, gamma is not None, M)
+    if cfg == _NO_CFG or not any(cfg):
+        cfg = _tuning.lookup(dev, n, K, wfmt, epilogue, gamma is not None, M) or _NO_CFG
         # an entry forcing a matrix-core path (2, 3, 4) is tuned for int4
         # group 128 and cannot run a smaller group: the built-in rule decides
-        if found and not (wfmt in (W_INT4_ZP, W_INT4_MIN) and group < 128 and found[3] in (2, 3, 4)):
-            cfg = (tuple(found) + (0, 0, 0, 0, 0))[:5]
-    d.cfg_depth, d.cfg_waves, d.cfg_tiles, d.cfg_path, d.cfg_slices = cfg
-    d.eps = eps
-    d.x, d.ldx = x.data_ptr(), x.stride(0)
-    d.w = w.data_ptr()
-    d.sc0 = _ptr(sc0)
-    d.sc1 = _ptr(sc1)
-    d.gamma = _ptr(gamma)
-    if epilogue == EPI_RESIDUAL:
-        d.residual, d.ldr = residual.data_ptr(), residual.stride(0)
-    d.out, d.ldo = out.data_ptr(), out.stride(0)
-    if out2 is not None:
-        d.out2, d.ldo2, d.n_out2 = out2.data_ptr(), out2.stride(0), out2.shape[1]
+        if wfmt in (W_INT4_ZP, W_INT4_MIN) and group < 128 and cfg[3] in (2, 3, 4):
+            cfg = _NO_CFG
+    if len(cfg) != 5:
+        cfg = (tuple(cfg) + _NO_CFG)[:5]
+    ptr = lambda t: 0 if t is None else t.data_ptr()  # noqa: E731
+    has_res = epilogue == EPI_RESIDUAL
+    d = _lib.gemv_desc(
+        _lib.ABI_VERSION, M, n, K, group, wfmt, epilogue, _DT[out.dtype], res_dt, *cfg, eps, x.data_ptr(), x.stride(0),
+        w.data_ptr(), ptr(sc0), ptr(sc1), ptr(gamma), residual.data_ptr() if has_res else 0,
+        residual.stride(0) if has_res else 0, out.data_ptr(), out.stride(0), 0, 0, ptr(out2),
+        0 if out2 is None else out2.stride(0), 0 if out2 is None else out2.shape[1], 0)
     stream = _lib.stream_of(x)
+    lib = _lib.lib()
     if M >= _TILE_MIN_ROWS or cfg[3] in (_PATH_TILE, _PATH_PANEL):
-        need = _lib.lib().bz_gemv_workspace(ctypes.byref(d))
+        need = lib.bz_gemv_workspace(ctypes.byref(d))
         if need:
             ws = _workspace(dev, stream, need)
             d.workspace, d.workspace_bytes = ws.data_ptr(), ws.numel() * 4
-    _lib.check(_lib.lib().bz_gemv(ctypes.byref(d), stream), "bz_gemv")
+    rc = lib.bz_gemv(ctypes.byref(d), stream)
+    if rc != _lib.OK:
+        _lib.check(rc, "bz_gemv")
     return out
 
 
+@functools.lru_cache(maxsize=1024)
 def _weight_spec(wfmt: int, n: int, k: int, group: int):
     """(bytes of w, (dtype, numel) of sc0 or None, of sc1 or None) a GEMV of
     this format and shape reads; None when the format is unknown."""

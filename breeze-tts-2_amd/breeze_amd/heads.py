@@ -41,7 +41,14 @@ def head_f32(x: torch.Tensor, w: torch.Tensor, *, index: Optional[torch.Tensor] 
         raise ValueError("w must be a contiguous float32 tensor")
     stack = w.dim() == 3
     C, N, K = (w.shape if stack else (1, *w.shape))
-    x = x.float()
+    if x.dtype == torch.bfloat16 and x.dim() == 2 and x.shape == (x.shape[0], K) and out is None \
+            and 0 < x.shape[0] <= NORM_HEAD_MAX_ROWS and K <= NORM_HEAD_MAX_K and x.stride(1) == 1 \
+            and x.stride(0) >= K and w.device == x.device:
+        # the fused form without a norm widens bf16 rows itself: no cast launch
+        return norm_head_f32(x, None, 0.0, w, out=torch.empty(x.shape[0], N, device=x.device, dtype=torch.float32),
+                             index=index, index_offset=index_offset)
+    if x.dtype != torch.float32:
+        x = x.float()
     if x.dim() != 2 or x.shape[1] != K:
         raise ValueError(f"x must be [M, {K}], got {tuple(x.shape)}")
     if x.stride(1) != 1 or x.stride(0) % 4 or x.data_ptr() % 16:
@@ -66,12 +73,12 @@ NORM_HEAD_MAX_ROWS = 4
 NORM_HEAD_MAX_K = 4096
 
 
-def norm_head_f32(x: torch.Tensor, gamma: torch.Tensor, eps: float, w: torch.Tensor, *, out: torch.Tensor,
+def norm_head_f32(x: torch.Tensor, gamma: Optional[torch.Tensor], eps: float, w: torch.Tensor, *, out: torch.Tensor,
                   index: Optional[torch.Tensor] = None, index_offset: int = 0, normed: Optional[torch.Tensor] = None,
                   cfg: Optional[torch.Tensor] = None, guidance: float = 1.0) -> torch.Tensor:
     """The final RMSNorm of bf16 rows x [M, K] (M <= 4, K <= 4096) and
     head_f32 of the result in one launch: out[M, N] fp32, the same bits as the
-    two calls.  normed [M, K] bf16 also receives the normed rows, cfg [M / 2
+    two calls.  Without a gamma the rows are the head's input as they are.  normed [M, K] bf16 also receives the normed rows, cfg [M / 2
     (or 1), N] the guidance combination of cond rows [0, M / 2) and uncond rows."""
     if x.device.type != "cuda" or w.device != x.device:
         raise RuntimeError("norm_head_f32 runs on the GPU (HIP kernel); the HIP path has no CPU fallback")
@@ -89,7 +96,7 @@ def norm_head_f32(x: torch.Tensor, gamma: torch.Tensor, eps: float, w: torch.Ten
     ptr = lambda t: None if t is None else t.data_ptr()  # noqa: E731
     ld = lambda t: 0 if t is None else t.stride(0)  # noqa: E731
     _lib.check(
-        _lib.lib().bz_norm_head_f32(x.data_ptr(), x.stride(0), M, K, gamma.data_ptr(), eps, ptr(normed), ld(normed),
+        _lib.lib().bz_norm_head_f32(x.data_ptr(), x.stride(0), M, K, ptr(gamma), eps, ptr(normed), ld(normed),
                                     w.data_ptr(), N, N * K, C, ptr(index), index_offset, out.data_ptr(), out.stride(0),
                                     ptr(cfg), ld(cfg), guidance, _lib.stream_of(x)),
         "bz_norm_head_f32",
@@ -114,6 +121,8 @@ class Fp32Linear(nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         shape = x.shape
+        if x.dim() == 2:
+            return head_f32(x, self.weight)
         y = head_f32(x.reshape(-1, shape[-1]), self.weight)
         return y.reshape(*shape[:-1], self.out_features)
 

@@ -147,24 +147,25 @@ class Int4Linear(nn.Module):
         self.register_buffer("scales_zeros", scales_zeros)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
+        # (views and casts that change nothing are skipped: each is a torch call
+        # as long as the launch's own host work)
         shape = x.shape
-        flat = x.reshape(-1, shape[-1])
-        if layout_of(self.weight_int4, self.out_features, self.in_features) == LAYOUT_TILED:
-            wfmt, sc0 = W_INT4_TILED, None
-            if flat.shape[0] > PREFILL_ROWS and not torch.compiler.is_compiling():
-                out = dequant_matmul(flat, self.weight_int4, W_INT4_TILED, self.out_features, self.in_features)
-                return out.to(x.dtype).reshape(*shape[:-1], self.out_features)
+        flat = x if x.dim() == 2 else x.reshape(-1, shape[-1])
+        w, n = self.weight_int4, self.out_features
+        sc0 = None
+        if layout_of(w, n, self.in_features) == LAYOUT_TILED:
+            wfmt = W_INT4_TILED
         else:
             wfmt, sc0 = W_INT4_ZP, self.scales_zeros
-        out = gemv_traceable(
-            flat.to(torch.bfloat16),
-            self.weight_int4,
-            wfmt,
-            self.out_features,
-            sc0=sc0,
-            group=self.group_size,
-        )
-        return out.to(x.dtype).reshape(*shape[:-1], self.out_features)
+        if wfmt == W_INT4_TILED and flat.shape[0] > PREFILL_ROWS and not torch.compiler.is_compiling():
+            out = dequant_matmul(flat, w, W_INT4_TILED, n, self.in_features)
+        else:
+            if flat.dtype != torch.bfloat16:
+                flat = flat.to(torch.bfloat16)
+            out = gemv_traceable(flat, w, wfmt, n, sc0=sc0, group=self.group_size)
+        if x.dtype != torch.bfloat16:
+            out = out.to(x.dtype)
+        return out if x.dim() == 2 else out.reshape(*shape[:-1], n)
 
     def extra_repr(self) -> str:
         return (

@@ -41,7 +41,7 @@ class SampleState:
 
 
 def _dev(name, t, dtype, dev, numel=None):
-    if t.device != dev or t.dtype != dtype or not t.is_contiguous():
+    if t.dtype != dtype or t.get_device() != dev.index or not t.is_contiguous():
         raise ValueError(f"{name} must be a contiguous {dtype} tensor on {dev}")
     if numel is not None and t.numel() != numel:
         raise ValueError(f"{name} has {t.numel()} entries, expected {numel}")

@@ -68,5 +68,10 @@ def _table(arch: str) -> dict:
 def lookup(device: torch.device, N: int, K: int, wfmt: int, epilogue: int, norm: bool, M: int) -> Optional[tuple]:
     """The table's launch shape for this GEMV, or None for the built-in rule."""
     arch = arch_of(device)
-    cfg = _table(arch).get(table_key(arch, N, K, wfmt, epilogue, norm, M))
-    return tuple(cfg) if cfg is not None else None
+    table, key = _table(arch), (N, K, wfmt, epilogue, norm, m_bucket(M))
+    # the entry under its fields, beside the file's string keys: one string
+    # per shape and bucket instead of one per call
+    if key not in table:
+        cfg = table.get(table_key(arch, N, K, wfmt, epilogue, norm, M))
+        table[key] = tuple(cfg) if cfg is not None else None
+    return table[key]

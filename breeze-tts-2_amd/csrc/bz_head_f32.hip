@@ -52,7 +52,7 @@ __device__ __forceinline__ float head_row_sum(float v) {
 // The fused form's inputs and outputs beside the head's.
 struct HeadNorm {
     const uint16_t* x;      // bf16 rows, NULL: fp32 x without a norm
-    const uint16_t* gamma;
+    const uint16_t* gamma;  // NULL: the bf16 rows as they are
     float eps;
     uint16_t* normed;       // optional: the normed rows, bf16
     int64_t ldn;
@@ -96,7 +96,7 @@ __global__ void __launch_bounds__(kHeadThreads) head_f32_kernel(const float* x, 
             const int k = min(tid + i * kHeadThreads, K - 1);
 #pragma unroll
             for (int m = 0; m < M; ++m) xb[i][m] = hn.x[m * ldx + k];
-            gb[i] = hn.gamma[k];
+            gb[i] = hn.gamma ? hn.gamma[k] : (uint16_t)0;
         }
         __builtin_amdgcn_sched_barrier(0);
     } else {
@@ -139,12 +139,14 @@ __global__ void __launch_bounds__(kHeadThreads) head_f32_kernel(const float* x, 
         __syncthreads();
 #pragma unroll
         for (int m = 0; m < M; ++m) {
+            const bool plain = !hn.gamma;  // uniform
             const float inv = rsqrtf(((part[m][0] + part[m][1]) + (part[m][2] + part[m][3])) / (float)K + hn.eps);
 #pragma unroll
             for (int i = 0; i < XN; ++i) {
                 const int k = tid + i * kHeadThreads;
                 if (k < K) {
-                    const uint16_t o = f32_to_bf16(bf16_to_f32(xb[i][m]) * inv * bf16_to_f32(gb[i]));
+                    const uint16_t o =
+                        plain ? xb[i][m] : f32_to_bf16(bf16_to_f32(xb[i][m]) * inv * bf16_to_f32(gb[i]));
                     xs[m * K + k] = bf16_to_f32(o);
                     if (hn.normed && blockIdx.x == 0) hn.normed[m * hn.ldn + k] = o;
                 }
@@ -291,7 +293,7 @@ extern "C" int bz_norm_head_f32(const void* x, int64_t ldx, int32_t M, int32_t K
                                 float* cfg, int64_t ld_cfg, float guidance, void* stream) {
     const int rc = check_head(M, K, w, N, mat_stride, nmat, x, ldx, out, ldo);
     if (rc != BZ_OK) return rc;
-    if (!gamma || (cfg && M > 1 && M % 2)) return BZ_ERR_INVALID_ARG;
+    if (cfg && M > 1 && M % 2) return BZ_ERR_INVALID_ARG;
     if (M > kHeadMaxRows || (normed && ld_normed < K) || (cfg && ld_cfg < N)) return BZ_ERR_SHAPE;
     const HeadNorm hn{static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(gamma), eps,
                       static_cast<uint16_t*>(normed), ld_normed, cfg, ld_cfg, guidance};

@@ -357,7 +357,7 @@ int bz_head_f32(const float* x, int64_t ldx, int32_t M, int32_t K,
 /* The decoder's final RMSNorm, the fp32 head and the guidance combination of
  * its logits in one launch, for M <= 4 bf16 rows: xn = bf16(x *
  * rsqrt(mean(x^2) + eps) * gamma) as bz_rmsnorm gives it, out = xn W^T as
- * bz_head_f32 gives it.  normed (optional, bf16 [M][ld_normed]) receives xn.
+ * bz_head_f32 gives it; gamma NULL: xn = x.  normed (optional, bf16 [M][ld_normed]) receives xn.
  * cfg (optional, fp32 [max(1, M / 2)][ld_cfg]; M = 1 or even): row h is
  * out[H + h] + guidance * (out[h] - out[H + h]) with H = M / 2, or out[0] for
  * M = 1.  x, gamma and normed need no alignment beyond their type; W as for

@@ -144,6 +144,8 @@ def test_norm_head_equals_its_parts(M, N, K):
     want = head_f32(xn, w, index=index, index_offset=-1)
     assert torch.equal(normed, xn)
     assert torch.equal(out, want)
+    assert torch.equal(head_f32(x, w, index=index, index_offset=-1),  # bf16 rows, widened by the kernel
+                       head_f32(x.float().clone(memory_format=torch.contiguous_format), w, index=index, index_offset=-1))
     if cfg is not None:
         h = max(1, M // 2)
         ref = want if M == 1 else want[h:].double() + 1.5 * (want[:h].double() - want[h:].double())
