@@ -165,12 +165,6 @@ class DepthDecodeGraph:
         nw, neps = getattr(dm.norm, "weight", None), getattr(dm.norm, "variance_epsilon", None)
         self._norm_w = None if nw is None or neps is None else nw.detach().to(torch.bfloat16).contiguous()
         self._norm_eps = None if neps is None else float(neps)
-        # the embedding rows the sampler can gather by itself: a plain table
-        emb = dm.embed_tokens
-        ew = emb.weight.detach() if type(emb) is nn.Embedding and emb.max_norm is None else None
-        self._emb_table = ew if (ew is not None and sampler == "hip" and ew.device == dev and ew.is_contiguous()
-                                 and ew.shape[0] >= self.num_codebooks * self.vocab_size
-                                 and ew.shape[1] * ew.element_size() % 16 == 0 and ew.data_ptr() % 16 == 0) else None
         with torch.no_grad():
             z = torch.zeros(1, 2, self.hidden_size, dtype=self.dtype, device=dev)
             self._pe_start = tuple(t.contiguous() for t in dm.rotary_emb(z, self.prefill_cache_pos.unsqueeze(0)))
@@ -196,8 +190,8 @@ class DepthDecodeGraph:
         self.first_cb_token_buf = torch.zeros(batch_size, dtype=torch.long, device=dev)
         self.output_tokens = torch.zeros(batch_size, self.num_decode_codebooks, dtype=torch.long, device=dev)
         self._tok_buf = torch.zeros(batch_size, dtype=torch.long, device=dev)
-        self._emb_buf = (None if self._emb_table is None else
-                         torch.zeros(batch_size, self._emb_table.shape[1], dtype=self._emb_table.dtype, device=dev))
+        table = self._embedding_rows()
+        self._emb_buf = None if table is None else torch.zeros(batch_size, table.shape[1], dtype=table.dtype, device=dev)
         self._norm_head = (self._norm_w is not None and dt == torch.bfloat16 and batch_size <= NORM_HEAD_MAX_ROWS
                            and self.hidden_size <= NORM_HEAD_MAX_K)
         self.prefill_input_ids = torch.zeros(batch_size, 2, dtype=torch.long, device=dev)
@@ -239,6 +233,17 @@ class DepthDecodeGraph:
             h = h[0] if isinstance(h, tuple) else h
         return h
 
+    def _embedding_rows(self):
+        """The embedding table where the sampler can gather its rows by itself
+        (a plain nn.Embedding over every codebook's tokens), else None."""
+        emb = self.depth_model.embed_tokens
+        if self.sampler != "hip" or type(emb) is not nn.Embedding or emb.max_norm is not None:
+            return None
+        w = emb.weight.detach()
+        ok = (w.device == self.device and w.is_contiguous() and w.shape[0] >= self.num_codebooks * self.vocab_size
+              and w.shape[1] * w.element_size() % 16 == 0 and w.data_ptr() % 16 == 0)
+        return w if ok else None
+
     def _logits(self, h, cache_pos):
         """Final norm and codebook head of the last position: [B, vocab] fp32."""
         h = h[:, -1, :]
@@ -269,9 +274,11 @@ class DepthDecodeGraph:
                       codec_size=self.codec_codebook_size, max_k=self._max_k,
                       cfg_out=None if self.debug_logits is None else self.debug_logits[i],
                       probs_out=None if self.debug_probs is None else self.debug_probs[i])
-            gather = self._emb_table is not None and i + 1 < self.num_decode_codebooks
+            table = self._embedding_rows() if i + 1 < self.num_decode_codebooks else None
+            gather = table is not None and self._emb_buf is not None and self._emb_buf.shape[1] == table.shape[1] \
+                and self._emb_buf.dtype == table.dtype
             sample_next(logits, self._tok_buf, self._sample_state, out_tokens=self.output_tokens[:, i],
-                        table=self._emb_table if gather else None, first_row=(i + 1) * self.vocab_size,
+                        table=table if gather else None, first_row=(i + 1) * self.vocab_size,
                         emb=self._emb_buf if gather else None, **kw)
             return gather
         half = self.half

@@ -90,7 +90,7 @@ class BackboneDecodeGraph:
         return inv, scale, *tables
 
     def _plain_norm(self):
-        """(weight, eps) when model.norm is an RMSNorm x / rms(x) * weight that
+        """eps when model.norm is an RMSNorm x / rms(x) * weight that
         bz_norm_head_f32 can run with this head, else None."""
         norm, head, H = self.model.norm, self.lm_head, self.inputs_buf.shape[-1]
         w, eps = getattr(norm, "weight", None), getattr(norm, "variance_epsilon", None)
@@ -104,7 +104,7 @@ class BackboneDecodeGraph:
             want, got = norm(x).float(), rmsnorm(x, w.detach(), float(eps)).float()
             if want.shape != got.shape or not bool(((want - got).abs() <= 2.0 ** -7 * want.abs()).all()):
                 return None
-        return w.detach(), float(eps)
+        return float(eps)
 
     # -- device-side state ---------------------------------------------------------
 
@@ -131,8 +131,7 @@ class BackboneDecodeGraph:
                       position_embeddings=pe)
             h = h[0] if isinstance(h, tuple) else h
         if self._norm is not None and isinstance(self.guidance_scale, (int, float)):
-            w, eps = self._norm
-            norm_head_f32(h[:, -1, :], w, eps, self.lm_head.weight, out=self.logits_buf,
+            norm_head_f32(h[:, -1, :], self.model.norm.weight, self._norm, self.lm_head.weight, out=self.logits_buf,
                           normed=self.hidden_buf[:, -1, :], cfg=self.cfg_logits_buf, guidance=self.guidance_scale)
             return
         h = self.model.norm(h)
