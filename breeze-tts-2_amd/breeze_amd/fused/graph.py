@@ -30,8 +30,9 @@ import torch
 from torch import nn
 
 from ..heads import NORM_HEAD_MAX_K, NORM_HEAD_MAX_ROWS, Fp32Linear, norm_head_f32
+from .checks import is_rmsnorm
 from .install import static_cache, zero_cache
-from .kernels import rmsnorm, step_tables
+from .kernels import step_tables
 
 __all__ = ["BackboneDecodeGraph"]
 
@@ -99,12 +100,7 @@ class BackboneDecodeGraph:
                 or not w.is_contiguous() or head.in_features != H or H > NORM_HEAD_MAX_K
                 or self.batch_size > NORM_HEAD_MAX_ROWS or (self.batch_size > 1 and self.batch_size % 2)):
             return None
-        with torch.no_grad():  # two roundings to bf16 in the module, one here: 2^-7 of the value covers them
-            x = torch.linspace(-3, 3, H, device=self.device).to(torch.bfloat16).view(1, H)
-            want, got = norm(x).float(), rmsnorm(x, w.detach(), float(eps)).float()
-            if want.shape != got.shape or not bool(((want - got).abs() <= 2.0 ** -7 * want.abs()).all()):
-                return None
-        return float(eps)
+        return float(eps) if is_rmsnorm(norm, w, float(eps)) else None
 
     # -- device-side state ---------------------------------------------------------
 

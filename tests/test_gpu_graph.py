@@ -188,3 +188,78 @@ def test_step_tables(B, S, D, dt):
     tol = 1.5 * (2.0 ** -8 if dt == torch.bfloat16 else 0.0) + 1.5 * 2.0 ** -21
     for t, f in ((cos, torch.cos), (sin, torch.sin)):
         assert float((t.view(B, D).double() - 1.5 * f(a)).abs().max()) <= tol
+
+
+class _MeanNorm(nn.Module):
+    """A norm with RMSNorm's attributes that subtracts the mean (as transformers' CohereLayerNorm)."""
+
+    def __init__(self, weight, eps):
+        super().__init__()
+        self.weight, self.variance_epsilon = weight, eps
+
+    def forward(self, x):
+        f = x.float()
+        f = f - f.mean(-1, keepdim=True)
+        f = f * torch.rsqrt(f.square().mean(-1, keepdim=True) + self.variance_epsilon)
+        return (self.weight.float() * f).to(x.dtype)
+
+
+def _mean_norm(m):
+    m.norm = _MeanNorm(m.norm.weight, m.norm.variance_epsilon)
+
+
+def _linear_rope(m):
+    """Positions divided by 3: not the default rotary type."""
+    m.rotary_emb.rope_type = "linear"
+    m.rotary_emb.inv_freq = m.rotary_emb.inv_freq / 3
+
+
+def _graph(B, change=None, scale=1.7, S=48):
+    cfg, ref, head = _model()
+    if change is not None:
+        change(ref)
+    gpu = copy.deepcopy(ref).to("cuda", torch.bfloat16)
+    # (a module's own cast would round the frequencies)
+    gpu.rotary_emb.inv_freq = ref.rotary_emb.inv_freq.float().cuda()
+    install_fused_backbone(types.SimpleNamespace(backbone_model=gpu), batch_size=B, max_seq_len=S)
+    g = BackboneDecodeGraph(gpu, copy.deepcopy(head).cuda(), batch_size=B, max_seq_len=S, guidance_scale=scale)
+    return cfg, ref, head, g
+
+
+def _inputs(B, n, seed=3):
+    gen = torch.Generator().manual_seed(seed)
+    return [torch.randn(B, 1, 512, generator=gen).to(torch.bfloat16).float() for _ in range(n)]
+
+
+@pytest.mark.parametrize("B,change", [(1, None), (4, None), (6, None), (2, _mean_norm), (2, _linear_rope), (6, _linear_rope)],
+                         ids=["1", "4", "6", "mean", "rope", "rope6"])
+def test_backbone_stand_ins_and_fallbacks_match_cpu_model(B, change):
+    """The launches around the layers and what takes their place: more rows
+    than the fused head takes, a norm that is no RMSNorm, other rotary tables.
+    CFG logits against the CPU float32 model."""
+    S, scale = 48, 1.7
+    cfg, ref, head, g = _graph(B, change, scale, S)
+    pads = torch.arange(B) % 3
+    g.pad_lens.copy_(pads)
+    xs = _inputs(B, 8)
+    g.set_step(xs[0].cuda(), 0)
+    g.capture(num_warmup=1)
+    g.reset()
+    c_ref = static_cache(cfg, S, B)
+    kv, half = torch.arange(S), max(1, B // 2)
+    for t, x in enumerate(xs):
+        out = g.step(x.to("cuda", torch.bfloat16), t).float().cpu().numpy()
+        pid = torch.full((B, 1), t)
+        valid = (kv >= pads.unsqueeze(1)) & (kv <= t)
+        mask = torch.where(valid, 0.0, torch.finfo(torch.float32).min).view(B, 1, 1, S)
+        with torch.no_grad():
+            h, pe = x, ref.rotary_emb(x, pid)
+            for layer in ref.layers:
+                h = layer(h, attention_mask=mask, position_ids=pid, past_key_values=c_ref, use_cache=True,
+                          position_embeddings=pe)
+                h = h[0] if isinstance(h, tuple) else h
+            h = ref.norm(h)[:, -1, :]
+        logits = O.linear_f32_ref(h.numpy(), head.weight.detach().numpy())
+        want = logits if B == 1 else logits[half:] + scale * (logits[:half] - logits[half:])
+        if t >= 2:  # a padded row attends to nothing before position 2
+            assert O.rel_err(out, want) <= TOL, t
