@@ -4,7 +4,16 @@ from __future__ import annotations
 
 import torch
 
-__all__ = ["is_rmsnorm"]
+__all__ = ["is_rmsnorm", "plain_call"]
+
+
+def plain_call(mod) -> bool:
+    """Whether calling the module runs its class's forward and nothing else: no
+    forward hook, on it or on every module, and no forward of its own (as
+    tools that wrap a module in place leave it)."""
+    every = torch.nn.modules.module
+    return not (mod._forward_hooks or mod._forward_pre_hooks or every._global_forward_hooks
+                or every._global_forward_pre_hooks or "forward" in vars(mod))
 
 
 @torch.no_grad()

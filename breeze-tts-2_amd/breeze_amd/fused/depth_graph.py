@@ -21,7 +21,8 @@ positions are computed once.  Between the last layer of a step and the
 projector of the next lie two launches: the final RMSNorm with the codebook
 head (bz_norm_head_f32), and the sampler, which also writes the frame's token
 and gathers its embedding row (bz_sample_next); with more than 4 rows, another
-embedding module or the torch sampler they are separate launches and torch ops.
+embedding module or the torch sampler they are separate launches and torch ops,
+and an embedding or head with forward hooks is called as the module it is.
 
 CFG layout (models/cudagraph/depth_decoder_graph.py:487-558): rows [0, half)
 are the conditional rows and rows [half, 2 half) the unconditional ones; the
@@ -49,6 +50,7 @@ from torch.nn import functional as F
 
 from ..heads import NORM_HEAD_MAX_K, NORM_HEAD_MAX_ROWS, Fp32CodebooksHead, norm_head_f32
 from ..sampling import SampleState, sample_next
+from .checks import plain_call
 from .install import static_cache, zero_cache
 from .kernels import FusedWeight, rms_gemv, rmsnorm
 
@@ -235,9 +237,10 @@ class DepthDecodeGraph:
 
     def _embedding_rows(self):
         """The embedding table where the sampler can gather its rows by itself
-        (a plain nn.Embedding over every codebook's tokens), else None."""
+        (a plain nn.Embedding over every codebook's tokens, without forward
+        hooks), else None."""
         emb = self.depth_model.embed_tokens
-        if self.sampler != "hip" or type(emb) is not nn.Embedding or emb.max_norm is not None:
+        if self.sampler != "hip" or type(emb) is not nn.Embedding or emb.max_norm is not None or not plain_call(emb):
             return None
         w = emb.weight.detach()
         ok = (w.device == self.device and w.is_contiguous() and w.shape[0] >= self.num_codebooks * self.vocab_size
@@ -248,7 +251,7 @@ class DepthDecodeGraph:
         """Final norm and codebook head of the last position: [B, vocab] fp32."""
         h = h[:, -1, :]
         head = self.codebooks_head
-        if self._norm_head and h.dtype == torch.bfloat16:
+        if self._norm_head and h.dtype == torch.bfloat16 and type(head) is Fp32CodebooksHead and plain_call(head):
             out = torch.empty(h.shape[0], head.vocab_size, device=h.device, dtype=torch.float32)
             return norm_head_f32(h, self._norm_w, self._norm_eps, head.weight_t, out=out, index=cache_pos,
                                  index_offset=-1)

@@ -18,7 +18,8 @@ in static buffers that the host updates in place before each replay:
 Around the layers lie two launches: the mask and the rotary tables
 (bz_step_tables), and the final norm, the head and the guidance combination
 (bz_norm_head_f32).  Both stand in only for modules that compute just that,
-which is checked against the modules at set-up; others run as they are.
+which is checked against the modules at set-up; others, and modules with
+forward hooks, run as they are.
 
 The layers are called directly (not through the model's forward), so no
 mask construction or shape logic of the model runs inside the capture.
@@ -30,7 +31,7 @@ import torch
 from torch import nn
 
 from ..heads import NORM_HEAD_MAX_K, NORM_HEAD_MAX_ROWS, Fp32Linear, norm_head_f32
-from .checks import is_rmsnorm
+from .checks import is_rmsnorm, plain_call
 from .install import static_cache, zero_cache
 from .kernels import step_tables
 
@@ -114,7 +115,8 @@ class BackboneDecodeGraph:
     def _decode_step(self) -> None:
         h = self.inputs_buf
         ints = (self.pad_lens, self.cache_position, self.position_ids)
-        if self._tables is not None and all(t.dtype == torch.long and t.is_contiguous() for t in ints):
+        if self._tables is not None and plain_call(self.model.rotary_emb) \
+                and all(t.dtype == torch.long and t.is_contiguous() for t in ints):
             inv, scale, *pe = self._tables
             step_tables(self.pad_lens, self.cache_position, self.mask_min, self.attn_mask, self.position_ids, inv, scale,
                         *pe)
@@ -126,7 +128,8 @@ class BackboneDecodeGraph:
                       past_key_values=self.static_cache, use_cache=True, cache_position=self.cache_position,
                       position_embeddings=pe)
             h = h[0] if isinstance(h, tuple) else h
-        if self._norm is not None and isinstance(self.guidance_scale, (int, float)):
+        if self._norm is not None and plain_call(self.model.norm) and plain_call(self.lm_head) \
+                and isinstance(self.guidance_scale, (int, float)):
             norm_head_f32(h[:, -1, :], self.model.norm.weight, self._norm, self.lm_head.weight, out=self.logits_buf,
                           normed=self.hidden_buf[:, -1, :], cfg=self.cfg_logits_buf, guidance=self.guidance_scale)
             return

@@ -235,3 +235,50 @@ def test_smaller_batch_is_padded_and_larger_recaptures():
     assert torch.equal(toks, g.debug_logits.cpu().argmax(-1).T)
     with pytest.raises(ValueError):
         g.run(bh6[:3].cuda(), first6[:3].cuda())
+
+
+def test_more_rows_than_the_fused_head_takes():
+    """Six rows: the final norm and the codebook head as separate launches."""
+    cfg, dd = _depth_decoder()
+    B, gs = 6, 2.5
+    g = _gpu_graph(cfg, dd, B, do_sample=False, guidance_scale=gs)
+    g.capture(num_warmup=1)
+    for seed in (1, 2):
+        bh, first = _inputs(B, seed)
+        toks = g.run(bh.cuda(), first.cuda()).cpu()
+        logits = g.debug_logits.cpu()
+        assert torch.equal(toks, logits.argmax(-1).T)
+        ref = _cpu_frame_logits(cfg, dd, bh, first, toks, gs)
+        for i in range(C - 1):
+            assert _rel(logits[i], ref[i]) <= TOL_FRAME, (seed, i)
+
+
+def test_forward_hooks_run():
+    """A hook on the embedding or on the codebook head fires at every step and
+    what it returns counts: halved rows give the frame of a halved table, and
+    doubled logits the doubled frame (powers of two: the same bits)."""
+    cfg, dd = _depth_decoder()
+    bh, first = (t.cuda() for t in _inputs(2, 60))
+    calls = []
+
+    def hook(factor):
+        def run(mod, args, out):
+            calls.append(1)
+            return out * factor
+        return run
+
+    half = copy.deepcopy(dd)
+    with torch.no_grad():
+        half.model.embed_tokens.weight.mul_(0.5)
+    want = _gpu_graph(cfg, half, 2, do_sample=False)
+    tokens = want.run(bh, first)
+    g = _gpu_graph(cfg, dd, 2, do_sample=False)
+    h = g.depth_model.embed_tokens.register_forward_hook(hook(0.5))
+    assert torch.equal(g.run(bh, first), tokens) and torch.equal(g.debug_logits, want.debug_logits)
+    assert len(calls) == C - 1
+    h.remove()
+    calls.clear()
+    tokens, logits = g.run(bh, first), g.debug_logits.clone()
+    g.codebooks_head.register_forward_hook(hook(2.0))
+    assert torch.equal(g.run(bh, first), tokens) and torch.equal(g.debug_logits, 2 * logits)
+    assert len(calls) == C - 1

@@ -263,3 +263,30 @@ def test_backbone_stand_ins_and_fallbacks_match_cpu_model(B, change):
         want = logits if B == 1 else logits[half:] + scale * (logits[:half] - logits[half:])
         if t >= 2:  # a padded row attends to nothing before position 2
             assert O.rel_err(out, want) <= TOL, t
+
+
+@pytest.mark.parametrize("what", ["norm", "rotary_emb", "lm_head"])
+def test_backbone_step_runs_forward_hooks(what):
+    """A module with a forward hook is called, and what the hook returns counts."""
+    _, _, _, g = _graph(2)
+    x = _inputs(2, 1)[0].to("cuda", torch.bfloat16)
+    g.step(x, 5)
+    plain = (g.hidden_buf.clone(), g.logits_buf.clone())
+    mod, seen = g.lm_head if what == "lm_head" else getattr(g.model, what), []
+
+    def hook(m, args, out):
+        seen.append(tuple(t * 0.5 for t in out) if isinstance(out, tuple) else out * 0.5)
+        return seen[-1]
+
+    handle = mod.register_forward_hook(hook)
+    g.step(x, 5)
+    assert len(seen) == 1
+    if what == "norm":
+        assert torch.equal(g.hidden_buf, seen[0])
+    elif what == "lm_head":
+        assert torch.equal(g.logits_buf, seen[0])
+    else:
+        assert not torch.equal(g.logits_buf, plain[1])
+    handle.remove()
+    g.step(x, 5)
+    assert torch.equal(g.hidden_buf, plain[0]) and torch.equal(g.logits_buf, plain[1])

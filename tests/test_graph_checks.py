@@ -6,7 +6,7 @@ import pytest
 import torch
 from torch import nn
 
-from breeze_amd.fused.checks import is_rmsnorm
+from breeze_amd.fused.checks import is_rmsnorm, plain_call
 
 
 class _Norm(nn.Module):
@@ -47,3 +47,16 @@ def test_is_rmsnorm_of_the_model():
 
     norm = Qwen3RMSNorm(2048, 1e-6).to(torch.bfloat16)
     assert is_rmsnorm(norm, norm.weight, norm.variance_epsilon)
+
+
+def test_plain_call():
+    mod = nn.Embedding(4, 4)
+    assert plain_call(mod)
+    for register in (mod.register_forward_hook, mod.register_forward_pre_hook,
+                     nn.modules.module.register_module_forward_hook, nn.modules.module.register_module_forward_pre_hook):
+        handle = register(lambda *a: None)
+        assert not plain_call(mod)
+        handle.remove()
+        assert plain_call(mod)
+    mod.forward = lambda ids: None
+    assert not plain_call(mod)
