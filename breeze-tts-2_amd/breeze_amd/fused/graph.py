@@ -18,8 +18,8 @@ in static buffers that the host updates in place before each replay:
 Around the layers lie two launches: the mask and the rotary tables
 (bz_step_tables), and the final norm, the head and the guidance combination
 (bz_norm_head_f32).  Both stand in only for modules that compute just that,
-which is checked against the modules at set-up; others, and modules with
-forward hooks, run as they are.
+which is checked against the modules at set-up and before a capture; others,
+and modules with forward hooks, run as they are.
 
 The layers are called directly (not through the model's forward), so no
 mask construction or shape logic of the model runs inside the capture.
@@ -63,45 +63,63 @@ class BackboneDecodeGraph:
         vocab = self.lm_head.out_features
         self.logits_buf = torch.zeros(batch_size, vocab, dtype=torch.float32, device=dev)
         self.cfg_logits_buf = torch.zeros(self.half, vocab, dtype=torch.float32, device=dev)
-        self._tables = self._rotary_tables()
-        self._norm = self._plain_norm()
+        self._rotary_class = self._norm_class = self._tables = None
+        self._find_stand_ins()
         self.graph = None
 
     # -- what the two launches around the layers may stand in for -------------------
+    #
+    # That a class of modules computes what its launch does is found by running
+    # it (at set-up and before every capture); everything the launch reads of
+    # the module is read when the step runs.
 
-    def _rotary_tables(self):
-        """(inv_freq, scaling, cos, sin) when rotary_emb gives the default tables
-        of bz_step_tables (same bits at a spread of positions), else None."""
-        rot, dt = self.model.rotary_emb, self.inputs_buf.dtype
+    def _rotary(self):
+        """(inv_freq, scaling) of a rotary embedding of the default type, else None."""
+        rot = self.model.rotary_emb
         inv, scale = getattr(rot, "inv_freq", None), getattr(rot, "attention_scaling", 1.0)
-        if (self.device.type != "cuda" or dt not in (torch.bfloat16, torch.float32)
-                or getattr(rot, "rope_type", None) != "default" or not isinstance(inv, torch.Tensor)
-                or not inv.is_floating_point() or inv.dim() != 1 or inv.device != self.device):
+        if (self.device.type != "cuda" or self.inputs_buf.dtype not in (torch.bfloat16, torch.float32)
+                or not plain_call(rot) or getattr(rot, "rope_type", None) != "default"
+                or not isinstance(inv, torch.Tensor) or not inv.is_floating_point() or inv.dim() != 1
+                or inv.device != self.device):
             return None
-        B, D = self.batch_size, 2 * inv.numel()
-        inv, scale = inv.detach().float().contiguous(), float(scale)  # the module widens it on every call
-        mask = torch.empty_like(self.attn_mask)
-        tables = [torch.zeros(B, 1, D, dtype=dt, device=self.device) for _ in range(2)]
-        with torch.no_grad():
-            for p in (0, 1, self.max_seq_len // 3, self.max_seq_len - 1):
-                ids = torch.full_like(self.position_ids, p)
-                step_tables(self.pad_lens, self.cache_position, self.mask_min, mask, ids, inv, scale, *tables)
-                want = rot(self.inputs_buf, ids)
-                if not all(w.dtype == dt and w.shape == t.shape and torch.equal(w, t) for w, t in zip(want, tables)):
-                    return None
-        return inv, scale, *tables
+        return inv.detach().float().contiguous(), float(scale)  # the module widens it on every call
 
-    def _plain_norm(self):
-        """eps when model.norm is an RMSNorm x / rms(x) * weight that
+    def _norm(self):
+        """(weight, eps) of a norm with an RMSNorm's parameters that
         bz_norm_head_f32 can run with this head, else None."""
         norm, head, H = self.model.norm, self.lm_head, self.inputs_buf.shape[-1]
         w, eps = getattr(norm, "weight", None), getattr(norm, "variance_epsilon", None)
         if (self.device.type != "cuda" or type(head) is not Fp32Linear or w is None or eps is None
-                or self.inputs_buf.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or w.shape != (H,)
-                or not w.is_contiguous() or head.in_features != H or H > NORM_HEAD_MAX_K
-                or self.batch_size > NORM_HEAD_MAX_ROWS or (self.batch_size > 1 and self.batch_size % 2)):
+                or not plain_call(norm) or not plain_call(head) or self.inputs_buf.dtype != torch.bfloat16
+                or w.dtype != torch.bfloat16 or w.shape != (H,) or not w.is_contiguous() or w.device != self.device
+                or head.in_features != H or H > NORM_HEAD_MAX_K or self.batch_size > NORM_HEAD_MAX_ROWS
+                or (self.batch_size > 1 and self.batch_size % 2)):
             return None
-        return float(eps) if is_rmsnorm(norm, w, float(eps)) else None
+        return w.detach(), float(eps)
+
+    def _find_stand_ins(self) -> None:
+        """Which classes of rotary embedding and norm the launches stand in for:
+        one whose tables have the same bits at a spread of positions, and one
+        that is an RMSNorm."""
+        self._rotary_class = self._norm_class = None
+        facts = self._rotary()
+        if facts is not None:
+            B, D, dt = self.batch_size, 2 * facts[0].numel(), self.inputs_buf.dtype
+            if self._tables is None or self._tables[0].shape[-1] != D:
+                self._tables = [torch.zeros(B, 1, D, dtype=dt, device=self.device) for _ in range(2)]
+            mask, same = torch.empty_like(self.attn_mask), True
+            with torch.no_grad():
+                for p in (0, 1, self.max_seq_len // 3, self.max_seq_len - 1):
+                    ids = torch.full((B, 1), p, dtype=torch.long, device=self.device)
+                    step_tables(torch.zeros_like(ids[:, 0]), ids[:1, 0], self.mask_min, mask, ids, *facts, *self._tables)
+                    want = self.model.rotary_emb(self.inputs_buf, ids)
+                    same = same and all(w.dtype == dt and w.shape == t.shape and torch.equal(w, t)
+                                        for w, t in zip(want, self._tables))
+            if same:
+                self._rotary_class = type(self.model.rotary_emb)
+        facts = self._norm()
+        if facts is not None and is_rmsnorm(self.model.norm, *facts):
+            self._norm_class = type(self.model.norm)
 
     # -- device-side state ---------------------------------------------------------
 
@@ -115,10 +133,11 @@ class BackboneDecodeGraph:
     def _decode_step(self) -> None:
         h = self.inputs_buf
         ints = (self.pad_lens, self.cache_position, self.position_ids)
-        if self._tables is not None and plain_call(self.model.rotary_emb) \
+        rotary = self._rotary() if type(self.model.rotary_emb) is self._rotary_class else None
+        if rotary is not None and 2 * rotary[0].numel() == self._tables[0].shape[-1] \
                 and all(t.dtype == torch.long and t.is_contiguous() for t in ints):
-            inv, scale, *pe = self._tables
-            step_tables(self.pad_lens, self.cache_position, self.mask_min, self.attn_mask, self.position_ids, inv, scale,
+            pe = self._tables
+            step_tables(self.pad_lens, self.cache_position, self.mask_min, self.attn_mask, self.position_ids, *rotary,
                         *pe)
         else:
             self._set_attention_mask()
@@ -128,9 +147,9 @@ class BackboneDecodeGraph:
                       past_key_values=self.static_cache, use_cache=True, cache_position=self.cache_position,
                       position_embeddings=pe)
             h = h[0] if isinstance(h, tuple) else h
-        if self._norm is not None and plain_call(self.model.norm) and plain_call(self.lm_head) \
-                and isinstance(self.guidance_scale, (int, float)):
-            norm_head_f32(h[:, -1, :], self.model.norm.weight, self._norm, self.lm_head.weight, out=self.logits_buf,
+        norm = self._norm() if type(self.model.norm) is self._norm_class else None
+        if norm is not None and h.dtype == torch.bfloat16 and isinstance(self.guidance_scale, (int, float)):
+            norm_head_f32(h[:, -1, :], *norm, self.lm_head.weight, out=self.logits_buf,
                           normed=self.hidden_buf[:, -1, :], cfg=self.cfg_logits_buf, guidance=self.guidance_scale)
             return
         h = self.model.norm(h)
@@ -159,6 +178,8 @@ class BackboneDecodeGraph:
         """Warm up (loads the library, sizes the allocator) and capture one step
         on a side stream, as backbone_graph.py:287-320.  The warm-up writes into
         the cache at the staged position; reset() clears it."""
+        self._find_stand_ins()
+        self._captured = (self._rotary(), self._norm())  # replays read these, replaced in their modules or not
         for _ in range(num_warmup):
             self._decode_step()
         torch.cuda.synchronize(self.device)

@@ -290,3 +290,48 @@ def test_backbone_step_runs_forward_hooks(what):
     handle.remove()
     g.step(x, 5)
     assert torch.equal(g.hidden_buf, plain[0]) and torch.equal(g.logits_buf, plain[1])
+
+
+def _new_inv_freq(m):
+    m.rotary_emb.inv_freq = m.rotary_emb.inv_freq * 0.5
+
+
+def _new_scaling(m):
+    m.rotary_emb.attention_scaling = 0.75
+
+
+def _new_eps(m):
+    m.norm.variance_epsilon = 0.5
+
+
+def _new_norm(m):
+    m.norm = _MeanNorm(m.norm.weight, 1e-6)
+
+
+def _fp32_norm(m):
+    m.norm.weight = nn.Parameter(m.norm.weight.detach().float() * 1.5, requires_grad=False)
+
+
+@pytest.mark.parametrize("captured", [False, True])
+@pytest.mark.parametrize("change", [_new_inv_freq, _new_scaling, _new_eps, _new_norm, _fp32_norm])
+def test_backbone_step_follows_its_modules(change, captured):
+    """A module changed after the graph was built counts in the next eager
+    step and in the next capture, as in a graph built after the change."""
+    x = _inputs(2, 1)[0].to("cuda", torch.bfloat16)
+    got = []
+    for late in (True, False):
+        _, _, _, g = _graph(2, None)
+        if not late:  # the same change before the graph is built
+            change(g.model)
+            g = BackboneDecodeGraph(g.model, g.lm_head, batch_size=2, max_seq_len=48, guidance_scale=1.7)
+        else:
+            change(g.model)
+        g.set_step(x, 5)
+        if captured:
+            g.capture(num_warmup=1)
+            g.reset()
+        got.append((g.step(x, 5).clone(), g.hidden_buf.clone()))
+    assert torch.isfinite(got[0][0]).all()
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+    _, _, _, g = _graph(2)
+    assert not torch.equal(g.step(x, 5), got[0][0])
