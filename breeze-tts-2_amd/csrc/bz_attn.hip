@@ -501,6 +501,9 @@ __device__ __forceinline__ void all_rows(float v, float (&o)[4]) {
     o[3] = __uint_as_float(hi[1]);
 }
 
+// attended positions up to which attn_bf16 runs unsplit (figures at nsp below)
+__host__ __device__ constexpr int attn_unsplit(int DL) { return DL == 4 ? 224 : 256; }
+
 template <int DL, int GM, bool FUSED, int NWV>
 __global__ void __launch_bounds__(64 * NWV) attn_bf16(const void* hrows, const void* hcos, const void* hsin,
                                                       const int64_t* hpos, void* hkc, void* hvc, int hld_qkv,
@@ -605,14 +608,16 @@ __global__ void __launch_bounds__(64 * NWV) attn_bf16(const void* hrows, const v
     // Splits in use (decided from the device position, so a captured graph
     // follows it): none while two blocks per wave cover the positions, else
     // as many as have a block for every wave, and no more workgroups than
-    // CUs; the others leave before any barrier.  Measured on MI355X, unsplit
+    // CUs (more are not launched); of those launched, the ones that the
+    // position leaves without a range leave before any barrier.  Measured on MI355X, unsplit
     // against 8 splits: D = 128 (16 / 8 heads, B = 2) 7.54 / 7.09 us at 331
     // positions (6.56 / 7.02 at 256 when both could be forced); D = 256 (16 / 4
     // heads, B = 1) 8.69 / 8.78 at 160, 10.63 / 10.22 at 256.  64 (row, kv head)
-    // pairs at 2001 positions: 4 splits 16.5 us, 5 21.8, 8 19.5, 16 25.8.
-    constexpr int kUnsplit = DL == 4 ? 224 : 256;
-    const int nsp =
-        kv_len <= kUnsplit ? 1 : min(a.split_cap, (nblk + NWV - 1) / NWV);
+    // pairs at 2001 positions: 4 splits 16.5 us, 5 21.8, 8 19.5, 16 25.8.  Above
+    // 128 pairs one split is left; against the kernel named
+    // above at 16 splits (16 / 8 heads of 128, 1902 of 2048 positions): 96 pairs
+    // 28.2 -> 22.0 us, 136 37.7 -> 29.7, 200 43.1 -> 30.5, 256 54.6 -> 38.4.
+    const int nsp = kv_len <= attn_unsplit(DL) ? 1 : min(a.split_cap, (nblk + NWV - 1) / NWV);
     KvRows<DL> cur;
     int s0 = (sp * NWV + wave) * kBlk;
     uint32_t live = kv_bytes;
@@ -1089,6 +1094,15 @@ static void launch_attn(const AttnParams& a, bool f32c, dim3 grid, hipStream_t s
         // what the first loads need in one preloaded word (grid.y <= 65535)
         const uint32_t shape =
             (uint32_t)a.G | (uint32_t)a.HKV << 5 | (a.cs_f32 ? 1u << 21 : 0u) | (a.ld_cs == 0 ? 1u << 22 : 0u);
+        // no more splits than the longest context of this cache uses: a
+        // workgroup without one still loads its prologue's rows before it knows
+        // (MI355X, S = 1024, 41 positions, 16 / 8 heads of 128, 8 splits asked for:
+        // 200 (row, kv head) pairs 7.89 -> 6.05 us, 512 16.6 -> 10.3, 96 5.42 -> 5.39;
+        // 200 pairs over S = 2048, 16 splits 9.65 -> 4.99)
+        if (a.S <= attn_unsplit(DL))
+            grid.z = 1;
+        else
+            grid.z = std::min(a.split_cap, ((a.S + kBlk - 1) / kBlk + NWV - 1) / NWV);
         hipLaunchKernelGGL((attn_bf16<DL, GM, FUSED, NWV>), grid, dim3(64 * NWV), 0, st, rows, a.cosp, a.sinp, a.pos,
                            a.kc, a.vc, ld, shape, a);
     } else {

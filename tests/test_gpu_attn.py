@@ -317,3 +317,26 @@ def test_attention_step_split_rule(HQ, HKV, D, B, pos):
     assert O.rel_err(outs[0], outs[3]) <= TIGHT and O.rel_err(outs[2], outs[3]) <= TIGHT
     q_ref = A.qkv_rope_cache(qkv, HQ, HKV, D, cos, sin, pos, keys, values)
     assert O.rel_err(outs[0], A.attn_decode(q_ref, keys, values, madd, pos)) <= TIGHT
+
+
+@pytest.mark.parametrize("HQ,HKV,D,B,S,pos,split", [
+    (16, 8, 128, 25, 300, 40, 8), (16, 8, 128, 33, 512, 500, 8), (16, 8, 128, 12, 512, 511, 8), (8, 8, 64, 1, 256, 255, 4),
+    (8, 8, 64, 1, 257, 256, 4), (16, 4, 256, 1, 224, 223, 4), (16, 4, 256, 1, 225, 224, 4), (16, 4, 256, 3, 640, 639, 16),
+    (48, 3, 256, 2, 1000, 999, 16)])
+def test_attention_step_launched_splits(HQ, HKV, D, B, S, pos, split):
+    """The splits that the launch brings cover the last position of the cache
+    and of every range: caches around the unsplit bound, (row, kv head) pairs
+    that leave one or two splits, more splits asked for than the cache has
+    blocks for; twice through one workspace, against the oracle."""
+    qkv, keys, values = _case(B, HQ, HKV, D, S, 60 + S, fill=pos)
+    cos, sin = (O.round_bf16(t) for t in _rope_tables(B, D, 61))
+    madd = np.zeros((B, S), dtype=np.float32)
+    kc, vc = _bf16(keys), _bf16(values)
+    args = (_bf16(qkv), _bf16(cos), _bf16(sin), torch.tensor([pos], device=DEV), kc, vc, _bf16(madd).view(B, 1, 1, S),
+            None, None, 1e-6)
+    out = torch.full((B, HQ * D), float("nan"), device=DEV, dtype=torch.bfloat16)
+    first = T.attention_step(*args, out=out, split=split).clone()
+    again = T.attention_step(*args, out=torch.full_like(out, float("nan")), split=split)
+    assert torch.isfinite(first).all() and torch.equal(first, again)
+    q_ref = A.qkv_rope_cache(qkv, HQ, HKV, D, cos, sin, pos, keys, values)
+    assert O.rel_err(f32(first), A.attn_decode(q_ref, keys, values, madd, pos)) <= TIGHT
