@@ -44,13 +44,12 @@ HIP_FLAGS = [
 
 # Kernels of the decode paths that must not use scratch (private memory): a
 # spilled or dynamically indexed register array costs a memory round trip per
-# access.  Patterns over the mangled names; the attention kernel's bf16-cache
-# instances with D <= 256 (attn_kernel<DL = 1, 2, 4, GM, F32C = false, ...>)
-# are covered, its fp32-cache and D = 512 instances are allowed scratch.
+# access.  Patterns over the mangled names, each of which has to match a
+# kernel.  Attention over bf16 caches with D <= 256 (attn_bf16) is covered;
+# attn_kernel (fp32 caches, D = 512) is allowed scratch.
 NO_SCRATCH = (r"gemv_persist", r"gemv_mfma", r"gemv_i8mma", r"gemv_tile", r"gemv_stream", r"gemv_wide", r"gemv_panel",
               r"gemm_tiled", r"gemv_rows", r"gemv_slab",
-              r"head_f32", r"qkv_rope_cache",
-              r"attn_kernelILi[124]ELi\d+ELb0E", r"attn_bf16")
+              r"head_f32", r"sample_cfg", r"step_tables", r"qkv_rope_cache", r"attn_bf16")
 
 
 def kernel_resources(remarks: str) -> list[tuple[str, int, int]]:
@@ -70,6 +69,17 @@ def kernel_resources(remarks: str) -> list[tuple[str, int, int]]:
             out.append((name, vgpr, int(body.split(":")[1].split()[0])))
             name = None
     return out
+
+
+def check_scratch(kernels: list[tuple[str, int, int]]) -> None:
+    """RuntimeError for a decode kernel that uses scratch memory, and for a
+    pattern that matches no kernel (a renamed or removed one)."""
+    spilled = [name for name, _, sc in kernels if sc and any(re.search(t, name) for t in NO_SCRATCH)]
+    if spilled:
+        raise RuntimeError("decode kernels using scratch memory:\n  " + "\n  ".join(spilled))
+    unused = [t for t in NO_SCRATCH if not any(re.search(t, name) for name, _, _ in kernels)]
+    if unused:
+        raise RuntimeError("no compiled kernel matches: " + ", ".join(unused))
 
 
 def _hipcc() -> str:
@@ -109,9 +119,7 @@ def build(verbose: bool = False) -> Path:
     kernels = sorted({k for _, ks in done for k in ks})
     (obj_dir / "kernel_resources.txt").write_text(
         "".join(f"{vg:4d} vgpr {sc:6d} scratch  {name}\n" for name, vg, sc in kernels))
-    spilled = [name for name, _, sc in kernels if sc and any(re.search(t, name) for t in NO_SCRATCH)]
-    if spilled:
-        raise RuntimeError("decode kernels using scratch memory:\n  " + "\n  ".join(spilled))
+    check_scratch(kernels)
     tmp = LIB_PATH.with_suffix(".so.tmp")
     cmd = [hipcc, f"--offload-arch={ARCH}", "-shared", "-fPIC", *map(str, objs), "-o", str(tmp)]
     if verbose:

@@ -229,7 +229,8 @@ struct AttnParams {
 template <int DL, bool F32C>
 struct KvBlock {
     static constexpr int T = 2 * DL;                                    // MFMA k-steps per key row
-    static constexpr int VW = F32C ? DL : (DL >= 2 ? DL / 2 : 1);  // value words per row
+    static_assert(F32C || DL == 8, "bf16 caches of D <= 256 run on attn_bf16");
+    static constexpr int VW = F32C ? DL : DL / 2;  // value words per row
     u32x4 kh[T], kl[T];
     uint32_t v[kBlk][VW];
     uint32_t mraw;  // raw mask entry at this lane's key position
@@ -268,26 +269,14 @@ __device__ __forceinline__ void load_vraw(const void* vc, int64_t off, uint32_t 
             for (int i = 0; i < DL; ++i) w[i] = p[i];
         }
     } else {
-        const uint16_t* p = reinterpret_cast<const uint16_t*>(vc) + off;
-        if constexpr (DL == 8) {
-            const u32x4 t = *reinterpret_cast<const u32x4*>(p);
-            for (int i = 0; i < 4; ++i) w[i] = t[i];
-        } else if constexpr (DL == 4) {
-            const uint2 t = *reinterpret_cast<const uint2*>(p);
-            w[0] = t.x;
-            w[1] = t.y;
-        } else if constexpr (DL == 2) {
-            w[0] = *reinterpret_cast<const uint32_t*>(p);
-        } else {
-            w[0] = p[0];
-        }
+        const u32x4 t = *reinterpret_cast<const u32x4*>(reinterpret_cast<const uint16_t*>(vc) + off);
+        for (int i = 0; i < 4; ++i) w[i] = t[i];
     }
 }
 
 template <int DL, bool F32C>
 __device__ __forceinline__ float vword(const uint32_t (&w)[KvBlock<DL, F32C>::VW], int e) {
     if constexpr (F32C) return __uint_as_float(w[e]);
-    if constexpr (DL == 1) return bf16_lo(w[0]);
     return (e & 1) ? bf16_hi(w[e >> 1]) : bf16_lo(w[e >> 1]);
 }
 
@@ -808,8 +797,9 @@ __global__ void __launch_bounds__(64 * NWV) attn_bf16(const void* hrows, const v
 
 // DL = D / 64 columns per lane; GM = 4 or 16 heads of register state (G <=
 // GM); F32C: fp32 cache; FUSED: q (and the new k, v) computed from qkv.
-template <int DL, int GM, bool F32C, bool FUSED, int NWV>
-__global__ void __launch_bounds__(64 * NWV) attn_kernel(const void* hrows, const void* hcos, const void* hsin,
+constexpr int kAttnWaves = 4;
+template <int DL, int GM, bool F32C, bool FUSED>
+__global__ void __launch_bounds__(64 * kAttnWaves) attn_kernel(const void* hrows, const void* hcos, const void* hsin,
                                                         const int64_t* hpos, void* hkc, void* hvc, int hld_qkv, int hG,
                                                         AttnParams a) {
     // the fields of the first loads, preloaded into SGPRs at wave launch
@@ -826,8 +816,7 @@ __global__ void __launch_bounds__(64 * NWV) attn_kernel(const void* hrows, const
     a.vc = hvc;
     a.ld_qkv = hld_qkv;
     a.G = hG;
-    constexpr int kAttnWaves = NWV;
-    constexpr int kAttnThreads = 64 * NWV;
+    constexpr int kAttnThreads = 64 * kAttnWaves;
     constexpr int D = 64 * DL;
     constexpr int T = D / 32;
     using Blk = KvBlock<DL, F32C>;
@@ -1079,15 +1068,15 @@ __global__ void __launch_bounds__(64 * NWV) attn_kernel(const void* hrows, const
                                             &st_acc[0][0][0], &last);
 }
 
-// Waves per workgroup: attn_bf16 eight (four where 16 heads of 256 columns
-// fill the LDS), attn_kernel four.
+// Waves per workgroup of attn_bf16: eight, or four where 16 heads of 256 columns
+// fill the LDS.
 template <int DL, int GM, bool FUSED>
 static void launch_attn(const AttnParams& a, bool f32c, dim3 grid, hipStream_t st) {
     const void* rows = FUSED ? static_cast<const void*>(a.qkv) : static_cast<const void*>(a.q);
     const int ld = (int)a.ld_qkv;  // bz_attn_step: checked to fit 32 bits
     if (f32c) {
-        hipLaunchKernelGGL((attn_kernel<DL, GM, true, FUSED, 4>), grid, dim3(64 * 4), 0, st, rows, a.cosp, a.sinp, a.pos,
-                           a.kc, a.vc, ld, a.G, a);
+        hipLaunchKernelGGL((attn_kernel<DL, GM, true, FUSED>), grid, dim3(64 * kAttnWaves), 0, st, rows, a.cosp, a.sinp,
+                           a.pos, a.kc, a.vc, ld, a.G, a);
     } else if constexpr (DL <= 4) {
         constexpr int NWV = GM == 16 && DL == 4 ? 4 : 8;
         // G, HKV, whether cos / sin are fp32 and whether one row serves all:
@@ -1106,8 +1095,8 @@ static void launch_attn(const AttnParams& a, bool f32c, dim3 grid, hipStream_t s
         hipLaunchKernelGGL((attn_bf16<DL, GM, FUSED, NWV>), grid, dim3(64 * NWV), 0, st, rows, a.cosp, a.sinp, a.pos,
                            a.kc, a.vc, ld, shape, a);
     } else {
-        hipLaunchKernelGGL((attn_kernel<DL, GM, false, FUSED, 4>), grid, dim3(64 * 4), 0, st, rows, a.cosp, a.sinp, a.pos,
-                           a.kc, a.vc, ld, a.G, a);
+        hipLaunchKernelGGL((attn_kernel<DL, GM, false, FUSED>), grid, dim3(64 * kAttnWaves), 0, st, rows, a.cosp, a.sinp,
+                           a.pos, a.kc, a.vc, ld, a.G, a);
     }
 }
 

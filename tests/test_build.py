@@ -6,6 +6,8 @@ from __future__ import annotations
 
 import re
 
+import pytest
+
 from breeze_amd import build as B
 
 _TAG = " [-Rpass-analysis=kernel-resource-usage]"
@@ -40,19 +42,42 @@ def _checked(name: str) -> bool:
     return any(re.search(t, name) for t in B.NO_SCRATCH)
 
 
+# one instance of every covered kernel, as compiled
+COVERED = (
+    "_ZN2bz12gemv_persistILi0ELi1ELi1ELi16ELb0EEEvPKtPKhPKvS2_iiiiiiNS_10GemvParamsE",
+    "_ZN2bz9gemv_mfmaILi0ELi1ELi1ELi16ELb0EEEvPKtPKhPKvS2_iiiiiiNS_10GemvParamsE",
+    "_ZN2bz10gemv_i8mmaILi0ELi1ELi1ELi2ELb0EEEvPKtPKhPKvS2_iiiiiiNS_10GemvParamsEi",
+    "_ZN2bz9gemv_tileILi0ELi1ELi1ELi2EEEvPKtPKhPKviiiiiiiiNS_10TileParamsE",
+    "_ZN2bz11gemv_streamILi4ELi1ELi10EEEvPKhPKtS4_iiiiiiiNS_12StreamParamsE",
+    "_ZN2bz9gemv_wideILi4ELi1ELi2ELi0EEEvPKhPKtS4_iiiiiiiiNS_12StreamParamsE",
+    "_ZN2bz10gemv_panelILi4ELi1ELi1ELi10EEEvPKhPKtiiiiiiiiNS_11PanelParamsE",
+    "_ZN2bz9gemv_rowsILi1ELi1ELi2ELb0EEEvPKtPKhS2_iiiiiiNS_10GemvParamsE",
+    "_ZN2bz9gemv_slabILi10EEEvPKhPKtiiiiiiNS_12StreamParamsE",
+    "_ZN2bz10gemm_tiledILi4ELi2ELi1EEEvNS_10GemmParamsE",
+    "_ZN2bz15head_f32_kernelILi1ELi1ELi0ELb0EEEvPKfliS2_liPKlliPflNS_8HeadNormE",
+    "_ZN2bz12_GLOBAL__N_117sample_cfg_kernelENS0_12SampleParamsE",
+    "_ZN2bz18step_tables_kernelIfEEviiPKlS2_fPT_S2_PKffS4_S4_",
+    "_ZN2bz21qkv_rope_cache_kernelEPKtliiiS1_S1_fPKvS3_blPKlPfPvS7_ibPl",
+    "_ZN2bz9attn_bf16ILi1ELi16ELb0ELi8EEEvPKvS2_S2_PKlPvS5_ijNS_10AttnParamsE",
+)
+
+
 def test_patterns_cover_the_decode_kernels():
-    for name in (
-        "_ZN2bz12gemv_persistILi0ELi1ELi2ELi2ELb1EEEvNS_10GemvParamsE",
-        "_ZN2bz9gemv_mfmaILi2ELi2ELi1ELi4ELb0EEEvNS_10GemvParamsE",
-        "_ZN2bz10gemv_i8mmaILi0ELi4ELi1ELi4ELb0EEEvNS_10GemvParamsEi",
-        "_ZN2bz9gemv_tileILi0ELi2ELi1ELi4EEEvNS_10TileParamsE",
-        "_ZN2bz11attn_kernelILi4ELi4ELb0ELb1EEEvNS_10AttnParamsE",
-        "_ZN2bz11attn_kernelILi1ELi16ELb0ELb0EEEvNS_10AttnParamsE",
-    ):
+    for name in COVERED:
         assert _checked(name), name
     # fp32 caches and D = 512 are allowed scratch
     for name in (
-        "_ZN2bz11attn_kernelILi4ELi16ELb1ELb0EEEvNS_10AttnParamsE",
-        "_ZN2bz11attn_kernelILi8ELi4ELb0ELb1EEEvNS_10AttnParamsE",
+        "_ZN2bz11attn_kernelILi4ELi16ELb1ELb0EEEvPKvS2_S2_PKlPvS5_iiNS_10AttnParamsE",
+        "_ZN2bz11attn_kernelILi8ELi4ELb0ELb1EEEvPKvS2_S2_PKlPvS5_iiNS_10AttnParamsE",
     ):
         assert not _checked(name), name
+
+
+def test_scratch_and_patterns_without_a_kernel_fail_the_build():
+    kernels = [(name, 64, 0) for name in COVERED]
+    B.check_scratch(kernels)
+    for i, name in enumerate(COVERED):
+        with pytest.raises(RuntimeError, match="no compiled kernel"):
+            B.check_scratch(kernels[:i] + kernels[i + 1:])
+        with pytest.raises(RuntimeError, match="scratch"):
+            B.check_scratch(kernels[:i] + [(name, 64, 16)] + kernels[i + 1:])
