@@ -237,19 +237,32 @@ def test_rank_order_at_the_edges(V, kind):
         assert got[tokens[r]] > 0, k
 
 
+@pytest.mark.parametrize("probs", [False, True])
+@pytest.mark.parametrize("do_sample", [0, 1])
+@pytest.mark.parametrize("top_k", [50, 300])
 @pytest.mark.parametrize("kind", ["pos_inf", "nan"])
-def test_rows_with_infinities_stay_in_range(kind):
-    """A row whose weights are no numbers still gives tokens of the vocabulary."""
-    V = 2051
+def test_rows_with_infinities(kind, top_k, do_sample, probs):
+    """Rows whose weights are no numbers (the shuffle argmax and the radix
+    select; within one wave's ranks and past them).  No rank has a positive
+    weight then, so a sampled row takes rank 0: the infinity, or the NaN, which
+    sorts above it.  A greedy row takes the infinity, or the largest number.
+    Every probability is 0."""
+    V, at = 2051, {"pos_inf": 7, "nan": 100}[kind]
     row = _edge_row(kind, V, torch.Generator(device=DEV).manual_seed(2))
+    row[1500] = 60.0
     if kind == "nan":
-        row[100] = float("nan")
+        row[at] = float("nan")
     tokens = torch.full((1,), -1, dtype=torch.int64, device=DEV)
-    prm = _params(1, top_k=50)
+    out = torch.full((1, V), 9.0, device=DEV) if probs else None
+    prm = _params(1, top_k=top_k, do_sample=do_sample)
     prm["guidance"] = None
-    sample_cfg(row.view(1, V), tokens, SampleState(1, DEV, seed=5), **prm)
+    state = SampleState(1, DEV, seed=5)
+    sample_cfg(row.view(1, V), tokens, state, probs_out=out, **prm)
     torch.cuda.synchronize()
-    assert 0 <= int(tokens[0]) < V
+    assert int(tokens[0]) == (1500 if kind == "nan" and not do_sample else at)
+    assert int(state.counters[0]) == 1
+    if probs:
+        assert int(torch.count_nonzero(out)) == 0
 
 
 @pytest.mark.parametrize("B", [1, 2, 6])
