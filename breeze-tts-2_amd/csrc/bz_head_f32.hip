@@ -36,7 +36,10 @@ constexpr int kHeadThreads = 256;
 constexpr int kHeadWaves = kHeadThreads / 64;
 constexpr int kHeadRowsPerWave = 2;
 constexpr int kHeadMaxRows = 4;                  // x rows per launch
-constexpr int kHeadMaxK = 4096;                  // LDS: kHeadMaxRows * K floats <= 64 KB
+constexpr int kHeadMaxK = 4096;
+// the x rows in dynamic LDS, within the 64 KB that a launch may ask for without
+// raising the kernel's limit (the fused form has 64 bytes of static sums beside)
+static_assert(kHeadMaxRows * kHeadMaxK * sizeof(float) <= 65536, "dynamic LDS of the largest head");
 
 __device__ __forceinline__ float head_row_sum(float v) {
     v += dpp_f32<kDppXor1>(v);
@@ -63,11 +66,15 @@ struct HeadNorm {
 
 // S = 256-k loads per row issued together (min(8, K / 256), so no load is
 // issued past a row for K a multiple of 256 S; the last chunk of other K
-// clamps its indices into the row).  XN > 0: the fused form, K <= 256 XN.
-// EXACT: K = 256 S, the usual widths: one chunk, no guards (each was a branch
-// that waited for the LDS reads before it) and no spare x loads.  Measured on
-// MI355X (graph replays, 1, 2 and 4 rows): N2051 K1024 4.35, 5.06, 6.88 ->
-// 3.67, 4.33, 5.35 us; N2052 K2048 5.67, 6.56, 8.76 -> 5.29, 6.13, 7.59.
+// clamps its indices into the row).  XN > 0: the fused form, K <= 256 XN; a
+// thread loads XN elements of each row and of gamma whatever K is (N2052 K2560,
+// 1, 2 and 4 bf16 rows: XN = 16 7.03, 8.87, 12.30 us, XN = 10 6.59, 8.32, 11.26;
+// a cast launch and the fp32 form 8.39, 9.51, 12.18).
+// EXACT: K = 256 S in one chunk, no guards (each was a branch that waited for
+// the LDS reads before it) and no spare x loads: K = 1024 and 2048, the two
+// heads' widths; other multiples of 256 run guarded.  Measured on MI355X (graph
+// replays, 1, 2 and 4 rows): N2051 K1024 4.35, 5.06, 6.88 -> 3.67, 4.33, 5.35
+// us; N2052 K2048 5.67, 6.56, 8.76 -> 5.29, 6.13, 7.59.
 template <int M, int S, int XN, bool EXACT>
 __global__ void __launch_bounds__(kHeadThreads) head_f32_kernel(const float* x, int64_t ldx, int argK, const float* w,
                                                                int64_t mat_stride, int nmat, const int64_t* index,
@@ -233,6 +240,8 @@ static void launch_head_m(const HeadCall& c, hipStream_t st) {
         launch_head_s<M, 8, X8, true>(c, st);
     else if (c.K == 1024)
         launch_head_s<M, 4, X4, true>(c, st);
+    else if (NORM && c.K > 2048 && c.K <= 2560)
+        launch_head_s<M, 8, NORM ? 10 : 0, false>(c, st);
     else if (NORM ? c.K > 2048 : c.K >= 2048)
         launch_head_s<M, 8, NORM ? 16 : 0, false>(c, st);
     else if (NORM && c.K > 1024)

@@ -123,7 +123,7 @@ def test_install_fp32_heads():
 
 
 @pytest.mark.parametrize("M", [1, 2, 3, 4])
-@pytest.mark.parametrize("N,K", [(1, 4), (9, 252), (2051, 1024), (64, 1028), (2052, 2048), (17, 2052), (40, 4096)])
+@pytest.mark.parametrize("N,K", [(1, 4), (9, 252), (2051, 1024), (64, 1028), (2052, 2048), (17, 2052), (33, 2560), (33, 2564), (40, 4096)])
 def test_norm_head_equals_its_parts(M, N, K):
     """norm_head_f32 against bz_rmsnorm, head_f32 and the guidance formula: the
     same bits for the first two (edges of its 256-k pieces and of its two
