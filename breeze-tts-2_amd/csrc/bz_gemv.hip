@@ -651,10 +651,11 @@ static int gemv_panel_rows(const bz_gemv_desc* d, hipStream_t st) {
 // the better of the dot2 and matrix-core kernels: N4096 K2048 M = 2 6.94 ->
 // 4.96, N2048 K2048 5.36 -> 3.80, N12288 K2048 SiLU-gate 13.1 -> 10.8, N1024
 // K8192 8.36 -> 5.39, N8192 K2560 M = 3 11.5 -> 10.5.  Plain products (no norm,
-// no epilogue) stay on those kernels all the same, for their order of sums: the
-// depth decoder's embedding projector is one, and a last-bit difference there
-// changes the tokens of a frame whose logits nearly tie; it runs once a
-// codebook (N1024 K2048 M = 2 3.9 us, 2.9 here).
+// no epilogue) stay on those kernels although this one is faster there too
+// (N1024 K2048 M = 2 3.9 us, 2.9 here), for their order of sums: the depth
+// decoder's embedding projector is a plain product, a last-bit difference there
+// changes the tokens of a frame whose logits nearly tie, and nothing in the
+// descriptor tells it from another plain product.
 static bool rows_plan(const bz_gemv_desc* d, const DescInfo& di, int rows, RowsLaunch& l) {
     if (d->wfmt != BZ_W_BF16 || d->cfg_path || d->cfg_waves || d->cfg_tiles || d->cfg_depth) return false;
     if (!d->gamma && d->epilogue == BZ_EPI_NONE) return false;
