@@ -28,6 +28,7 @@ W_INT4_TILED, W_INT4_TILED_PAIRED, W_FP8_TILED, W_FP8_TILED_PAIRED = 4, 5, 6, 7
 EPI_NONE, EPI_SILU_GATE, EPI_RESIDUAL = 0, 1, 2
 DT_BF16, DT_F32 = 0, 1
 MASK_BOOL = 2  # include/bz_attn.h
+STEP_INV_BF16 = 256  # added to bz_step_tables' dtype
 
 EXPORTS = (
     "bz_abi_version",

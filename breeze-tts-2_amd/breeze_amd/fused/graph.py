@@ -82,7 +82,10 @@ class BackboneDecodeGraph:
                 or not isinstance(inv, torch.Tensor) or not inv.is_floating_point() or inv.dim() != 1
                 or inv.device != self.device):
             return None
-        return inv.detach().float().contiguous(), float(scale)  # the module widens it on every call
+        inv = inv.detach()  # the module widens it to fp32 on every call, and so does the kernel
+        if inv.dtype not in (torch.float32, torch.bfloat16):
+            inv = inv.float()
+        return inv.contiguous(), float(scale)
 
     def _norm(self):
         """(weight, eps) of a norm with an RMSNorm's parameters that

@@ -278,18 +278,22 @@ def silu_mul(g, u, out=None):
 
 def step_tables(pad_lens, cache_position, mask_min, mask, position_ids, inv_freq, scaling, cos, sin):
     """A decode step's additive mask [B, 1, 1, S] and rotary tables [B, 1, D]
-    from its device-side positions, in one launch (bz_step_tables)."""
+    from its device-side positions, in one launch (bz_step_tables); inv_freq
+    fp32 or bf16."""
     B, S, D = mask.shape[0], mask.shape[-1], cos.shape[-1]
     dt = {torch.bfloat16: _lib.DT_BF16, torch.float32: _lib.DT_F32}[mask.dtype]
+    if inv_freq.dtype not in (torch.float32, torch.bfloat16):
+        raise ValueError("inv_freq must be float32 or bfloat16")
     for n, t, k, d in (("pad_lens", pad_lens, B, torch.int64), ("cache_position", cache_position, 1, torch.int64),
-                       ("position_ids", position_ids, B, torch.int64), ("inv_freq", inv_freq, D // 2, torch.float32),
+                       ("position_ids", position_ids, B, torch.int64), ("inv_freq", inv_freq, D // 2, inv_freq.dtype),
                        ("mask", mask, B * S, mask.dtype), ("cos", cos, B * D, mask.dtype), ("sin", sin, B * D, mask.dtype)):
         if t.numel() != k or t.dtype != d or not t.is_contiguous() or t.device != mask.device or t.device.type != "cuda":
             raise ValueError(f"{n} must be a contiguous {d} tensor of {k} entries on {mask.device}")
     _lib.check(
         _lib.lib().bz_step_tables(B, S, D, pad_lens.data_ptr(), cache_position.data_ptr(), mask_min, mask.data_ptr(),
                                   position_ids.data_ptr(), inv_freq.data_ptr(), scaling, cos.data_ptr(), sin.data_ptr(),
-                                  dt, _lib.stream_of(mask)),
+                                  dt + (_lib.STEP_INV_BF16 if inv_freq.dtype == torch.bfloat16 else 0),
+                                  _lib.stream_of(mask)),
         "bz_step_tables",
     )
 

@@ -203,7 +203,7 @@ __global__ void silu_mul_kernel(const uint16_t* g, int64_t ldg, const uint16_t* 
 template <typename T>
 __global__ void __launch_bounds__(256) step_tables_kernel(int S, int D, const int64_t* pad_lens, const int64_t* cache_pos,
                                                           float mask_min, T* mask, const int64_t* positions,
-                                                          const float* inv_freq, float scaling, T* cos_out,
+                                                          const void* inv_freq, int inv_bf16, float scaling, T* cos_out,
                                                           T* sin_out) {
     const int b = blockIdx.y, mblk = (S + 255) / 256;
     auto cast = [](float v) -> T {
@@ -219,7 +219,9 @@ __global__ void __launch_bounds__(256) step_tables_kernel(int S, int D, const in
     }
     const int d = ((int)blockIdx.x - mblk) * 256 + threadIdx.x;
     if (d >= D) return;
-    const float a = (float)positions[b] * inv_freq[d % (D / 2)];
+    const int f = d % (D / 2);
+    const float inv = inv_bf16 ? bf16_to_f32(static_cast<const uint16_t*>(inv_freq)[f]) : static_cast<const float*>(inv_freq)[f];
+    const float a = (float)positions[b] * inv;
     cos_out[(int64_t)b * D + d] = cast(cosf(a) * scaling);
     sin_out[(int64_t)b * D + d] = cast(sinf(a) * scaling);
 }
@@ -266,8 +268,10 @@ extern "C" int bz_rmsnorm(const void* x, int64_t ldx, const void* gamma, float e
 }
 
 extern "C" int bz_step_tables(int32_t B, int32_t S, int32_t D, const int64_t* pad_lens, const int64_t* cache_pos,
-                              float mask_min, void* mask, const int64_t* positions, const float* inv_freq, float scaling,
+                              float mask_min, void* mask, const int64_t* positions, const void* inv_freq, float scaling,
                               void* cos_out, void* sin_out, int32_t dtype, void* stream) {
+    const int inv_bf16 = (dtype & BZ_STEP_INV_BF16) != 0;
+    dtype &= ~BZ_STEP_INV_BF16;
     if (!pad_lens || !cache_pos || !mask || !positions || !inv_freq || !cos_out || !sin_out) return BZ_ERR_INVALID_ARG;
     if (B < 1 || B > 65535 || S < 1 || D < 2 || D % 2 || (dtype != BZ_DT_BF16 && dtype != BZ_DT_F32))
         return BZ_ERR_INVALID_ARG;
@@ -275,12 +279,12 @@ extern "C" int bz_step_tables(int32_t B, int32_t S, int32_t D, const int64_t* pa
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (dtype == BZ_DT_BF16)
         hipLaunchKernelGGL(step_tables_kernel<uint16_t>, grid, dim3(256), 0, st, S, D, pad_lens, cache_pos, mask_min,
-                           static_cast<uint16_t*>(mask), positions, inv_freq, scaling, static_cast<uint16_t*>(cos_out),
-                           static_cast<uint16_t*>(sin_out));
+                           static_cast<uint16_t*>(mask), positions, inv_freq, inv_bf16, scaling,
+                           static_cast<uint16_t*>(cos_out), static_cast<uint16_t*>(sin_out));
     else
         hipLaunchKernelGGL(step_tables_kernel<float>, grid, dim3(256), 0, st, S, D, pad_lens, cache_pos, mask_min,
-                           static_cast<float*>(mask), positions, inv_freq, scaling, static_cast<float*>(cos_out),
-                           static_cast<float*>(sin_out));
+                           static_cast<float*>(mask), positions, inv_freq, inv_bf16, scaling,
+                           static_cast<float*>(cos_out), static_cast<float*>(sin_out));
     return launched();
 }
 

@@ -377,12 +377,14 @@ int bz_norm_head_f32(const void* x, int64_t ldx, int32_t M, int32_t K,
  * (contiguous rows), and the default rotary tables cos/sin[b][d] =
  * cos/sin(fp32(positions[b]) * inv_freq[d % (D / 2)]) * scaling, d < D, B rows
  * each (contiguous).  mask and tables bf16 (BZ_DT_BF16) or fp32 (BZ_DT_F32)
- * by `dtype`; positions, pad_lens int64 [B]; inv_freq fp32 [D / 2].
+ * by `dtype`; positions, pad_lens int64 [B]; inv_freq fp32 [D / 2], or bf16
+ * with BZ_STEP_INV_BF16 added to `dtype`.
  * Replaces _set_attention_mask and the rotary embedding of a step
  * (models/cudagraph/backbone_graph.py:240-252,262-266). */
+#define BZ_STEP_INV_BF16 256
 int bz_step_tables(int32_t B, int32_t S, int32_t D, const int64_t* pad_lens,
                    const int64_t* cache_pos, float mask_min, void* mask,
-                   const int64_t* positions, const float* inv_freq,
+                   const int64_t* positions, const void* inv_freq,
                    float scaling, void* cos_out, void* sin_out, int32_t dtype,
                    void* stream);
 

@@ -56,7 +56,7 @@ COVERED = (
     "_ZN2bz10gemm_tiledILi4ELi2ELi1EEEvNS_10GemmParamsE",
     "_ZN2bz15head_f32_kernelILi1ELi1ELi0ELb0EEEvPKfliS2_liPKlliPflNS_8HeadNormE",
     "_ZN2bz12_GLOBAL__N_117sample_cfg_kernelENS0_12SampleParamsE",
-    "_ZN2bz18step_tables_kernelIfEEviiPKlS2_fPT_S2_PKffS4_S4_",
+    "_ZN2bz18step_tables_kernelIfEEviiPKlS2_fPT_S2_PKvifS4_S4_",
     "_ZN2bz21qkv_rope_cache_kernelEPKtliiiS1_S1_fPKvS3_blPKlPfPvS7_ibPl",
     "_ZN2bz9attn_bf16ILi1ELi16ELb0ELi8EEEvPKvS2_S2_PKlPvS5_ijNS_10AttnParamsE",
 )

@@ -181,6 +181,11 @@ def test_step_tables(B, S, D, dt):
     mask = torch.full((B, 1, 1, S), 5.0, device=dev, dtype=dt)
     cos, sin = (torch.full((B, 1, D), 5.0, device=dev, dtype=dt) for _ in range(2))
     step_tables(pad, pos, low, mask, ids, inv, 1.5, cos, sin)
+    rounded = inv.to(torch.bfloat16)  # frequencies as a model cast to bf16 holds them
+    same = [torch.zeros_like(t) for t in (mask, cos, sin, cos, sin)]
+    step_tables(pad, pos, low, same[0], ids, rounded, 1.5, *same[1:3])
+    step_tables(pad, pos, low, same[0], ids, rounded.float(), 1.5, *same[3:])
+    assert torch.equal(same[1], same[3]) and torch.equal(same[2], same[4])
     s = torch.arange(S, device=dev)
     valid = (s >= pad.view(B, 1)) & (s <= pos)
     assert torch.equal(mask.view(B, S), torch.where(valid, 0.0, low).to(dt))
