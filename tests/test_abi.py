@@ -487,3 +487,42 @@ def test_shared_read_validation(L):
     assert lib.bz_shared_read(fake + 8, 4096, fake, 1024, 4, 0, fake, None) == L.ERR_ALIGNMENT
     assert lib.bz_shared_read(fake, 4096, fake + 8, 1024, 4, 0, fake, None) == L.ERR_ALIGNMENT
     assert lib.bz_shared_read(fake, 4096, fake, 1024, 65537, 0, fake, None) == L.ERR_UNSUPPORTED
+
+
+FAKE = 1 << 20  # never dereferenced: the calls below fail validation
+
+
+@pytest.mark.parametrize("kw", [
+    *({n: None} for n in ("pad", "pos", "mask", "ids", "inv", "cos", "sin")), {"B": 0}, {"B": 65536}, {"S": 0}, {"D": 0},
+    {"D": 3}, {"dtype": 2}, {"dtype": -1}, {"dtype": 256 + 2}, {"dtype": 512}])
+def test_step_tables_validation(L, kw):
+    a = dict(B=2, S=16, D=8, pad=FAKE, pos=FAKE, mask=FAKE, ids=FAKE, inv=FAKE, cos=FAKE, sin=FAKE, dtype=0)
+    a.update(kw)
+    assert L.lib().bz_step_tables(a["B"], a["S"], a["D"], a["pad"], a["pos"], -1.0, a["mask"], a["ids"], a["inv"], 1.0,
+                                  a["cos"], a["sin"], a["dtype"], None) == L.ERR_INVALID_ARG
+
+
+@pytest.mark.parametrize("kw,status", [
+    *(({n: None}, "INVALID_ARG") for n in ("x", "w", "out")), ({"M": 0}, "INVALID_ARG"), ({"N": 0}, "INVALID_ARG"),
+    ({"nmat": 0}, "INVALID_ARG"), ({"M": 3, "cfg": FAKE, "ldc": 64}, "INVALID_ARG"), ({"M": 5}, "SHAPE"), ({"K": 130}, "SHAPE"),
+    ({"K": 4100, "ldx": 4100}, "SHAPE"), ({"ldx": 124}, "SHAPE"), ({"ldo": 60}, "SHAPE"), ({"stride": 64 * 128 - 4, "nmat": 2}, "SHAPE"),
+    ({"normed": FAKE, "ldn": 120}, "SHAPE"), ({"cfg": FAKE, "ldc": 60}, "SHAPE"), ({"w": FAKE + 8}, "ALIGNMENT")])
+def test_norm_head_validation(L, kw, status):
+    a = dict(x=FAKE, ldx=128, M=2, K=128, normed=None, ldn=0, w=FAKE, N=64, stride=64 * 128, nmat=1, out=FAKE, ldo=64, cfg=None,
+             ldc=0)
+    a.update(kw)
+    assert L.lib().bz_norm_head_f32(a["x"], a["ldx"], a["M"], a["K"], FAKE, 1e-6, a["normed"], a["ldn"], a["w"], a["N"],
+                                    a["stride"], a["nmat"], None, 0, a["out"], a["ldo"], a["cfg"], a["ldc"], 1.0,
+                                    None) == getattr(L, "ERR_" + status)
+
+
+@pytest.mark.parametrize("kw,status", [
+    ({"out_ld": 0}, "INVALID_ARG"), ({"emb": None}, "INVALID_ARG"), ({"rows": 0}, "INVALID_ARG"), ({"row": 8}, "INVALID_ARG"),
+    ({"first": -1}, "INVALID_ARG"), ({"row": 40, "ld": 48}, "SHAPE"), ({"ld": 40}, "SHAPE"), ({"ld": 16}, "SHAPE"),
+    ({"table": FAKE + 8}, "ALIGNMENT"), ({"emb": FAKE + 8}, "ALIGNMENT")])
+def test_sample_next_validation(L, kw, status):
+    a = dict(out_ld=1, table=FAKE, rows=10, row=32, first=0, emb=FAKE, ld=32)
+    a.update(kw)
+    args = list(_sample_args(L))[:-1]
+    assert L.lib().bz_sample_next(*args, FAKE, a["out_ld"], a["table"], a["rows"], a["row"], a["first"], a["emb"], a["ld"],
+                                  None) == getattr(L, "ERR_" + status)
