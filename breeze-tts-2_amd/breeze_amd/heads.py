@@ -78,8 +78,9 @@ def norm_head_f32(x: torch.Tensor, gamma: Optional[torch.Tensor], eps: float, w:
                   cfg: Optional[torch.Tensor] = None, guidance: float = 1.0) -> torch.Tensor:
     """The final RMSNorm of bf16 rows x [M, K] (M <= 4, K <= 4096) and
     head_f32 of the result in one launch: out[M, N] fp32, the same bits as the
-    two calls.  Without a gamma the rows are the head's input as they are.  normed [M, K] bf16 also receives the normed rows, cfg [M / 2
-    (or 1), N] the guidance combination of cond rows [0, M / 2) and uncond rows."""
+    two calls.  Without a gamma the rows are the head's input as they are.
+    normed [M, K] bf16 also receives the normed rows, cfg [M / 2 (or 1), N] the
+    guidance combination of cond rows [0, M / 2) and uncond rows."""
     if x.device.type != "cuda" or w.device != x.device:
         raise RuntimeError("norm_head_f32 runs on the GPU (HIP kernel); the HIP path has no CPU fallback")
     if w.dtype != torch.float32 or not w.is_contiguous():

@@ -645,11 +645,12 @@ static int gemv_panel_rows(const bz_gemv_desc* d, hipStream_t st) {
 // spans).  Four weight rows per wave, or two where four give less than one
 // workgroup per CU or a second, mostly empty round (257..383 workgroups).
 // Measured on MI355X at M = 2, four against two rows: N4096 K2048 4.96 / 5.27
-// us, N2048 K2048 4.12 / 3.80, N2560 K4096 (320 workgroups) 6.65 / 6.07,
+// us, N2048 K2048 4.12 / 3.80 (3.65 since the residual is loaded without a
+// branch on its type), N2560 K4096 (320 workgroups) 6.65 / 6.07,
 // N6144 K2560 (384) 7.95 / 8.12, N1024 K8192 (4 waves per row) 5.39 / 5.40.
 // The kernel was the faster one at every shape and M = 1..4 timed, against
 // the better of the dot2 and matrix-core kernels: N4096 K2048 M = 2 6.94 ->
-// 4.96, N2048 K2048 5.36 -> 3.80, N12288 K2048 SiLU-gate 13.1 -> 10.8, N1024
+// 5.01, N2048 K2048 5.36 -> 3.65, N12288 K2048 SiLU-gate 13.1 -> 10.8, N1024
 // K8192 8.36 -> 5.39, N8192 K2560 M = 3 11.5 -> 10.5.  Plain products (no norm,
 // no epilogue) stay on those kernels although this one is faster there too
 // (N1024 K2048 M = 2 3.9 us, 2.9 here), for their order of sums: the depth
